@@ -265,6 +265,21 @@ VAFA_API int vafa_absorb_fwd_fold(const void *q_proj, const void *W_K, const voi
                                   int32_t dtype, float scale, void *workspace,
                                   int64_t workspace_bytes, void *stream);
 
+/* The whole packed_target_attn forward (ta/interface.py:429-435, then
+ * ta/interface.py:141-220) in one call: q_proj = q_raw [T_q,D_Q] W_Q
+ * [D_Q,H,D_H] (written for the backward, as by vafa_absorb_project_fwd), then
+ * vafa_absorb_fwd_fold on it; the shapes of both apply, results are the same
+ * bits.  T_q may exceed the plan's query tokens (then only q_proj covers the
+ * rest). */
+VAFA_API int64_t vafa_absorb_fwd_full_workspace(const vafa_plan_info *info, int64_t D_Q,
+                                                int64_t D_KV, int64_t D_H);
+VAFA_API int vafa_absorb_fwd_full(const void *q_raw, const void *X, const void *W_Q,
+                                  const void *W_K, const void *W_V, void *q_proj, void *O,
+                                  float *lse, int64_t T_q, const int32_t *plan_dev,
+                                  const vafa_plan_info *info, int64_t D_Q, int64_t D_KV,
+                                  int64_t D_H, int32_t dtype, float scale, void *workspace,
+                                  int64_t workspace_bytes, void *stream);
+
 /* The head projection of packed_target_attn, which the reference runs as a
  * torch einsum (ta/interface.py:434-435, 'thd,khd->thk'):
  * u[t,h,f] = sum_d q_proj[t, h*D_H + d] * W_K[f,h,d] with q_proj [T_q, H*D_H],

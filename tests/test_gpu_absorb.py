@@ -147,6 +147,24 @@ def test_absorb_wide_dh_split(device, H, D_H, d_kv, dtype):
         assert_close(n, a, r)
 
 
+# The dU pass over key chunks of at least 256 keys (fp32 partials summed in
+# order): ranges at the chunk's edges, tiles of one token and of several per
+# sample, whole and split tiles in one launch, D_KV = 512 (two workgroups per
+# tile), a padded D_KV.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32],
+                         ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("H,d_kv", [(8, 256), (8, 512), (5, 100), (64, 32)])
+def test_absorb_du_split(device, H, d_kv, dtype):
+    q_lens, k_lens = [1, 9, 4, 0, 17, 2], [256, 257, 511, 300, 1025, 3]
+    plan = _lib.plan_absorb(cu_from_lens(q_lens).numpy(), cu_from_lens(k_lens).numpy(), H,
+                            d_kv, 32)
+    assert plan.info.n_dqc > 0, "the case must split a key range"
+    print(f"[absorb du split {dtype}] H={H} d_kv={d_kv}", flush=True)
+    got, ref = run_case(q_lens, k_lens, dtype, device, d_q=64, d_kv=d_kv, H=H, D_H=32)
+    for n, a, r in zip(NAMES, got, ref):
+        assert_close(n, a, r)
+
+
 def test_absorb_bf16_config4_dims(device):
     """C4 dims (D_in=256, N(0,1) inputs, Xavier weights) on a small sample."""
     from varlenabsorbflashattn_amd import workloads as W

@@ -517,3 +517,52 @@ def test_varlen_bwd_rejects_fused_items_at_wider_head_dim(D):
         assert rc != 0 and "fused key-major items" in _lib.last_error()
         with pytest.raises(ValueError, match="build the plan with this head_dim"):
             _lib.check(rc)
+
+
+@pytest.mark.parametrize("q_lens,k_lens,H", [
+    ([3, 9, 0, 20], [256, 257, 900, 1000], 8),   # at and just past the smallest chunk
+    ([1], [1], 8), ([40], [6000], 64), ([5, 2], [700, 12], 3),
+    ([5, 2], [7000, 12], 65),                    # wave-per-row kernels: whole ranges
+])
+def test_absorb_du_split_sections(q_lens, k_lens, H):
+    """The dU pass's items (dq) cover every token tile's key range once, in
+    equal chunks of at least 128 keys (but the last), with partial rows that tile
+    [0, n_fpart_rows); without a split both sections are empty."""
+    cq, ck = _cu(q_lens), _cu(k_lens)
+    p = _lib.plan_absorb(cq, ck, H, 256, 32)
+    dq, dqc = p.section("dq").tolist(), p.section("dqc").tolist()
+    split = H <= 64 and any(q > 0 and k > 256 for q, k in zip(q_lens, k_lens))
+    assert bool(dq) == bool(dqc) == split
+    assert p.info.max_dqc_rows == max([r[1] - r[0] for r in dqc], default=0)
+    rows = np.zeros(p.info.n_fpart_rows, dtype=np.int64)
+    comb = {(r[0], r[1]): r for r in dqc}
+    tiles = {}
+    for t0, t1, k0, k1, pb, seg, j, ns in dq:
+        tiles.setdefault((t0, t1), []).append((j, k0, k1, pb, ns))
+    if split:
+        assert set(tiles) == {(r[0], r[1]) for r in p.section("qt").tolist()}
+    for (t0, t1), its in tiles.items():
+        its.sort()
+        seg = int(np.searchsorted(cq, t0, side="right")) - 1
+        assert its[0][1] == ck[seg] and its[-1][2] == ck[seg + 1]
+        assert all(a[2] == b[1] and a[2] - a[1] >= 128 for a, b in zip(its, its[1:]))
+        assert [i[0] for i in its] == list(range(its[0][4]))
+        if its[0][4] == 1:
+            assert its[0][3] == -1 and (t0, t1) not in comb
+            continue
+        _, _, pbase, ns, *_ = comb[(t0, t1)]
+        R = t1 - t0
+        assert ns == its[0][4] and [i[3] for i in its] == [pbase + j * R for j in range(ns)]
+        rows[pbase:pbase + ns * R] += 1
+    assert (rows == 1).all()
+
+
+def test_absorb_small_launch_chunks():
+    """Small launches: forward chunks down to 128 keys, at most 16 of them below
+    1024 keys; dX tiles of 128 keys up to 192k keys in all, 256 beyond."""
+    for lk, ns in ((128, 1), (129, 2), (2000, 16), (2048, 16), (2049, 11), (20000, 20)):
+        p = _lib.plan_absorb(_cu([4]), _cu([lk]), 8, 256, 32)
+        assert p.info.max_split == ns, lk
+    for n, bk in ((192, 128), (193, 256)):
+        p = _lib.plan_absorb(_cu([1] * n), _cu([1024] * n), 8, 256, 32)
+        assert p.info.k_tile == bk

@@ -88,6 +88,9 @@ _SIGS = {
                                   _I32, C.c_float, _P, _I64, _P]),
     "vafa_absorb_fwd_fold": (C.c_int, [_P, _P, _P, _P, _P, _P, _P, _PINFO, _I64, _I64, _I32,
                                        C.c_float, _P, _I64, _P]),
+    "vafa_absorb_fwd_full_workspace": (C.c_int64, [_PINFO, _I64, _I64, _I64]),
+    "vafa_absorb_fwd_full": (C.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _PINFO, _I64,
+                                       _I64, _I64, _I32, C.c_float, _P, _I64, _P]),
 }
 
 EXPORTED = tuple(_SIGS)
@@ -216,17 +219,29 @@ class HostPlan:
         return self.items[off:off + n * ITEM_INTS].reshape(n, ITEM_INTS)
 
 
+def _plan(fn, guess: int, *args) -> HostPlan:
+    """Runs a planner into a buffer of ``guess`` items, and again into one of
+    the reported size when the plan is longer (pages of an over-long guess are
+    never touched)."""
+    info = PlanInfo()
+    n = min(guess, 1 << 20) * ITEM_INTS
+    while True:
+        items = np.empty(n, dtype=np.int32)
+        rc = fn(*args, _i32p(items), n, C.byref(info))
+        if rc != VAFA_ERR_CAPACITY:
+            check(rc)
+            return HostPlan(info, items[:info.plan_ints])
+        n = info.plan_ints
+
+
 def plan_varlen(cu_q: np.ndarray, cu_k: np.ndarray, H: int, D: int) -> HostPlan:
     a = np.ascontiguousarray(cu_q, dtype=np.int64)
     b = np.ascontiguousarray(cu_k, dtype=np.int64)
     if a.shape != b.shape:
         raise AssertionError(f"segment count mismatch: q has {a.size - 1}, k has {b.size - 1}")
-    info = PlanInfo()
-    check(lib().vafa_plan_varlen(_i64p(a), _i64p(b), a.size, H, D, None, 0, C.byref(info)))
-    items = np.empty(info.plan_ints, dtype=np.int32)
-    check(lib().vafa_plan_varlen(_i64p(a), _i64p(b), a.size, H, D, _i32p(items), items.size,
-                                 C.byref(info)))
-    return HostPlan(info, items)
+    # forward, dQ and dK/dV items of 128 tokens, a few splits of short queries
+    guess = 64 + 12 * a.size + int(max(a[-1], 0) + max(b[-1], 0)) // 32 if a.size else 64
+    return _plan(lib().vafa_plan_varlen, guess, _i64p(a), _i64p(b), a.size, H, D)
 
 
 def plan_absorb(cu_q: np.ndarray, cu_k: np.ndarray, H: int, F: int, DH: int) -> HostPlan:
@@ -234,12 +249,9 @@ def plan_absorb(cu_q: np.ndarray, cu_k: np.ndarray, H: int, F: int, DH: int) -> 
     b = np.ascontiguousarray(cu_k, dtype=np.int64)
     if a.shape != b.shape:
         raise AssertionError("segment count mismatch q vs k")
-    info = PlanInfo()
-    check(lib().vafa_plan_absorb(_i64p(a), _i64p(b), a.size, H, F, DH, None, 0, C.byref(info)))
-    items = np.empty(info.plan_ints, dtype=np.int32)
-    check(lib().vafa_plan_absorb(_i64p(a), _i64p(b), a.size, H, F, DH, _i32p(items),
-                                 items.size, C.byref(info)))
-    return HostPlan(info, items)
+    # token tiles of two passes, key tiles of 128
+    guess = 64 + 12 * a.size + int(max(a[-1], 0)) + int(max(b[-1], 0)) // 64 if a.size else 64
+    return _plan(lib().vafa_plan_absorb, guess, _i64p(a), _i64p(b), a.size, H, F, DH)
 
 
 # ---- device plans (cached by cu_seqlens content) ------------------------------

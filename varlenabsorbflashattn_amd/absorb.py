@@ -329,9 +329,10 @@ class _FoldedTargetAttn(torch.autograd.Function):
     """packed_target_attn with the u projection folded into the attention
     forward (ta/interface.py:429-435 followed by ta/interface.py:141-321).
 
-    Forward: q_proj = q_raw W_Q (row-GEMM kernel, rounded to the input dtype),
-    then vafa_absorb_fwd_fold, whose workgroups form u = q_proj_h W_K,h^T for
-    their own rows on the matrix cores -- u is never written to memory.
+    Forward (vafa_absorb_fwd_full): q_proj = q_raw W_Q (row-GEMM kernel,
+    rounded to the input dtype), then the attention, whose workgroups form
+    u = q_proj_h W_K,h^T for their own rows on the matrix cores -- u is never
+    written to memory.
     Backward: u is formed once from the saved q_proj (vafa_absorb_project_u,
     the same products), then the inner backward gives du / dX / dW_V and the
     projection backward dq_raw / dW_Q / dW_K, as the unfused path."""
@@ -349,17 +350,13 @@ class _FoldedTargetAttn(torch.autograd.Function):
         L = _lib.lib()
         st = _lib.stream_ptr(X.device)
         q_proj = torch.empty((T_q, H * D_H), dtype=q_raw.dtype, device=q_raw.device)
-        pws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 0), X.device)
-        _lib.check(L.vafa_absorb_project_fwd(
-            q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), None,
-            T_q, H, d_q, d_kv, D_H, dcode, pws.data_ptr(), pws.numel(), st))
         O = torch.empty((T_q, H, D_H), dtype=q_raw.dtype, device=X.device)
         LSE = torch.empty((T_q, H), dtype=torch.float32, device=X.device)
-        ws = _workspace(L.vafa_absorb_fwd_fold_workspace(plan.info, d_kv, D_H), X.device)
-        _lib.check(L.vafa_absorb_fwd_fold(
-            q_proj.data_ptr(), W_K.data_ptr(), X.data_ptr(), W_V.data_ptr(), O.data_ptr(),
-            LSE.data_ptr(), plan.items.data_ptr(), plan.info, d_kv, D_H, dcode, float(scale),
-            ws.data_ptr() if ws.numel() else None, ws.numel(), st))
+        ws = _workspace(L.vafa_absorb_fwd_full_workspace(plan.info, d_q, d_kv, D_H), X.device)
+        _lib.check(L.vafa_absorb_fwd_full(
+            q_raw.data_ptr(), X.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), W_V.data_ptr(),
+            q_proj.data_ptr(), O.data_ptr(), LSE.data_ptr(), T_q, plan.items.data_ptr(),
+            plan.info, d_q, d_kv, D_H, dcode, float(scale), ws.data_ptr(), ws.numel(), st))
         ctx.save_for_backward(q_raw, W_Q, W_K, q_proj, X, W_V, O, LSE)
         ctx.plan = plan
         ctx.scale = scale

@@ -4,8 +4,9 @@
 // With rows r = (token, head) pairs, P = exp2(c * u_r.X_j - LSE_r) rebuilt
 // from the forward's log2-domain LSE, dP = dAX_r . X_j and dS = P (dP - delta):
 //   * query side, absorb_du_kernel: one workgroup (4 waves x 16 rows) per
-//     token tile with the sample's whole key range; raw X streams through a
-//     3-deep LDS-DMA ring like the forward's.  Per 32-key tile, on 16x16x32
+//     token tile with the sample's whole key range (or one chunk of it, whose
+//     fp32 partials absorb_du_combine_kernel sums, where the plan splits); raw
+//     X streams through a 3-deep LDS-DMA ring like the forward's.  Per 32-key tile, on 16x16x32
 //     products (16 rows per wave keep both fp32 accumulators in registers):
 //       S^T = X U^T, dP^T = X dAX^T   (X rows as A, U^T / dAX^T in registers)
 //       du^T += X^T dS^T, aX^T += X^T P^T   (X^T from ds_read_b64_tr_b16)
@@ -45,8 +46,8 @@ template <typename T, int FP>
 __global__ __launch_bounds__(64 * kDuWaves, FP > kMaxF ? 1 : 2) void absorb_du_kernel(
     const T *__restrict__ u, const T *__restrict__ X, const T *__restrict__ dax,
     const float *__restrict__ lse, const float *__restrict__ delta, T *__restrict__ du,
-    float *__restrict__ ax, const int32_t *__restrict__ items, int n_items, int H, int F,
-    float c, float scale) {
+    float *__restrict__ ax, float *__restrict__ part_du, float *__restrict__ part_ax,
+    const int32_t *__restrict__ items, int n_items, int H, int F, float c, float scale) {
   using M16 = Mfma16<T>;
   using v8 = typename Mfma<T>::v8;
   using S = AbsSmem<FP>;
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(64 * kDuWaves, FP > kMaxF ? 1 : 2) void absorb_du_k
     if (item >= n_items) return;  // padding of the last group of 16
   }
   const PlanItem it = load_item(items, item);
-  const int t0 = it.v[0], t1 = it.v[1], k0 = it.v[2], k1 = it.v[3];
+  const int t0 = it.v[0], t1 = it.v[1], k0 = it.v[2], k1 = it.v[3], pbase = it.v[4];
   if (t1 <= t0) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -204,6 +205,17 @@ __global__ __launch_bounds__(64 * kDuWaves, FP > kMaxF ? 1 : 2) void absorb_du_k
 
   if (!row_ok) return;
   typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
+  if (pbase >= 0) {  // one key chunk of a split tile: fp32 partial rows
+    const int64_t po = ((int64_t)pbase * H + row) * F;
+#pragma unroll
+    for (int ft = 0; ft < NF; ++ft) {
+      const int f = (ft0 + ft) * 16 + lq * 4;
+      if (f >= F) continue;
+      *reinterpret_cast<f32x4 *>(part_du + po + f) = adu[ft] * scale;
+      *reinterpret_cast<f32x4 *>(part_ax + po + f) = aax[ft];
+    }
+    return;
+  }
   const int64_t ro = ((int64_t)t0 * H + row) * F;
 #pragma unroll
   for (int ft = 0; ft < NF; ++ft) {
@@ -648,8 +660,8 @@ void launch_du_fp(const AbsorbArgs &a, hipStream_t st) {
   const int64_t grid = DuSlices<FP>::NS == 2 ? (a.n_qseg + 7) / 8 * 16 : a.n_qseg;
   hipLaunchKernelGGL((absorb_du_kernel<T, FP>), dim3((unsigned)grid), dim3(64 * kDuWaves), smem,
                      st, (const T *)a.u, (const T *)a.X, (const T *)a.dax, a.lse_in, a.delta,
-                     (T *)a.du, a.ax, a.qseg_items, (int)a.n_qseg, a.H, a.F, a.scale * kLog2e,
-                     a.scale);
+                     (T *)a.du, a.ax, a.part_du, a.part_ax, a.qseg_items, (int)a.n_qseg, a.H, a.F,
+                     a.scale * kLog2e, a.scale);
 }
 
 template <typename T, int FP>
@@ -689,6 +701,7 @@ void launch_mfma_absorb_du(const AbsorbArgs &a, hipStream_t st) {
     case 512: launch_du_fp<T, 512>(a, st); break;
     default: break;
   }
+  launch_du_combine<T>(a, st);
 }
 
 template <typename T>

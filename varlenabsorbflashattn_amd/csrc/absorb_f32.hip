@@ -7,7 +7,7 @@
 //     of one sample (head-major; with H not dividing 64 the last rows idle)
 //     and streams the sample's X rows once through a 3-deep ring of 16-key
 //     LDS tiles filled by buffer_load ... lds;
-//   * dX (ta/kernels.py:528-900): a workgroup owns up to 512 keys of one
+//   * dX (ta/kernels.py:528-900): a workgroup owns up to 256 keys of one
 //     sample, 16 per wave per pass, and streams the sample's (token, head)
 //     rows of u and dAX through LDS in blocks of 32, summing over heads in
 //     registers (deterministic).
@@ -302,7 +302,8 @@ __global__ __launch_bounds__(256, FP > 256 ? 1 : 2) void absorb_fwd_f32_kernel(
 
 // ---------------------------------------------------------------------------
 // Backward, query side (ta/kernels.py:354-498): per token tile with the
-// sample's whole key range, P rebuilt from the saved LSE:
+// sample's whole key range (or one chunk of it, to fp32 partial rows), P
+// rebuilt from the saved LSE:
 //   du = scale * sum_j dS_j X_j,  aX = sum_j P_j X_j (fp32, for dW_V),
 //   dS = P (dP - delta), dP = dAX . X_j, dAX = dO W_V^T (workspace).
 // ---------------------------------------------------------------------------
@@ -310,8 +311,8 @@ template <int FP>
 __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
     const float *__restrict__ u, const float *__restrict__ X, const float *__restrict__ lse,
     const float *__restrict__ delta, const float *__restrict__ dax, float *__restrict__ du,
-    float *__restrict__ ax_ws, const int32_t *__restrict__ items, int n_items, int H, int F,
-    float c, float scale) {
+    float *__restrict__ ax_ws, float *__restrict__ part_du, float *__restrict__ part_ax,
+    const int32_t *__restrict__ items, int n_items, int H, int F, float c, float scale) {
   using S = F32Smem<FP>;
   // FP = 512: two workgroups of one XCD share a token tile (blocks b and
   // b + 8 of each 16), each forming S and dP over every feature and
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
     if (item >= n_items) return;  // padding of the last group of 16
   }
   const PlanItem it = load_item(items, item);
-  const int t0 = it.v[0], t1 = it.v[1], k0 = it.v[2], k1 = it.v[3];
+  const int t0 = it.v[0], t1 = it.v[1], k0 = it.v[2], k1 = it.v[3], pbase = it.v[4];
   if (t1 <= t0) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
   for (int b = 0; b < kNBuf - 1; ++b) issue(k0 + b * kKT, b);
 
   float uf[Q], df[Q];
-  const int64_t grow = (int64_t)(t0 + g.tl) * H + g.hh;  // global (token, head) row
+  int64_t grow = (int64_t)(t0 + g.tl) * H + g.hh;  // global (token, head) row
   {
     const int64_t nb = (int64_t)ntok * H * F * 4;
     const int off = g.row_ok ? (g.tl * H + g.hh) * F * 4 : 0x7fff0000;
@@ -410,7 +411,13 @@ __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
   }
   wait_vmcnt<0>();
   if (!g.wave_active || !g.row_ok) return;
-  // lane: row grow, features 64a + 16*lq + 4r + b (b = 0..3 consecutive)
+  // lane: row grow, features 64a + 16*lq + 4r + b (b = 0..3 consecutive); a
+  // key chunk of a split tile goes to its partial rows
+  if (pbase >= 0) {
+    du = part_du;
+    ax_ws = part_ax;
+    grow = (int64_t)(pbase + g.tl) * H + g.hh;
+  }
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
 
 // ---------------------------------------------------------------------------
 // Backward, key side (ta/kernels.py:528-900): item {k0, k1, t0, t1, ...}
-// covers up to 512 keys of one sample and all of its (token, head) rows
+// covers up to 256 keys of one sample and all of its (token, head) rows
 // R = t*H + h in [t0*H, t1*H):
 //   dX_j = sum_R (scale * dS_Rj u_R + P_Rj dAX_R),
 // summed over rows and heads in registers in a fixed order.  Each pass gives
@@ -573,8 +580,9 @@ void launch_bwd_fp(const AbsorbArgs &a, hipStream_t st) {
     const int64_t grid = FP > 256 ? (a.n_qseg + 7) / 8 * 16 : a.n_qseg;
     hipLaunchKernelGGL(absorb_du_f32_kernel<FP>, dim3((unsigned)grid), dim3(256), smem, st,
                        (const float *)a.u, (const float *)a.X, a.lse_in, a.delta,
-                       (const float *)a.dax, (float *)a.du, a.ax, a.qseg_items, (int)a.n_qseg,
-                       a.H, a.F, a.scale * kLog2e, a.scale);
+                       (const float *)a.dax, (float *)a.du, a.ax, a.part_du, a.part_ax,
+                       a.qseg_items, (int)a.n_qseg, a.H, a.F, a.scale * kLog2e, a.scale);
+    launch_du_combine<float>(a, st);
   }
   if (a.n_kv > 0) {
     const int smem = F32Smem<FP>::kDxBytes;

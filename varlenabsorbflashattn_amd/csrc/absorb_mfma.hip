@@ -49,13 +49,18 @@ using namespace absorb;
 // With the folded projection the same launch also writes
 // W_K [F, H, DH] -> wkt [H, FP, DHP] (DHP = max(DH, 32); zeros at f >= F and
 // d >= DH): the rows of one head contiguous, so the u product's A operand
-// (16 f rows x 16 bytes per lane group) reads whole cache lines.
+// (16 f rows x 16 bytes per lane group) reads whole cache lines; and, when the
+// whole op runs in one call, W_Q [DQ, H*DH] -> wqt [H*DH, DQ] for the q_proj
+// row GEMM that follows (one launch for the three weights: 16 small samples'
+// forward takes 4 launches instead of 5).
 template <typename T>
 __global__ __launch_bounds__(256) void transpose_w_kernel(const T *__restrict__ wv,
                                                           T *__restrict__ wvt,
                                                           const T *__restrict__ wk,
-                                                          T *__restrict__ wkt, int H, int F,
-                                                          int DH, int FP, int DHP) {
+                                                          T *__restrict__ wkt,
+                                                          const T *__restrict__ wq,
+                                                          T *__restrict__ wqt, int H, int F,
+                                                          int DH, int FP, int DHP, int DQ) {
   const int64_t nv = (int64_t)H * DH * FP;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < nv) {
@@ -68,8 +73,13 @@ __global__ __launch_bounds__(256) void transpose_w_kernel(const T *__restrict__ 
     return;
   }
   if (wkt == nullptr) return;
-  const int64_t j = i - nv;
-  if (j >= (int64_t)H * FP * DHP) return;
+  const int64_t j = i - nv, nk = (int64_t)H * FP * DHP;
+  if (j >= nk) {
+    const int64_t e = j - nk;
+    if (wqt != nullptr && e < (int64_t)H * DH * DQ)
+      wqt[e] = wq[(e % DQ) * ((int64_t)H * DH) + e / DQ];
+    return;
+  }
   const int d = (int)(j % DHP);
   const int f = (int)((j / DHP) % FP);
   const int h = (int)(j / ((int64_t)DHP * FP));
@@ -527,10 +537,17 @@ void launch_mfma_absorb_fwd(const AbsorbArgs &a, hipStream_t st) {
   const int FP = padded_f(a.F);
   T *wvt = reinterpret_cast<T *>(a.wvt);
   const int DHP = a.DH < 32 ? 32 : a.DH;
-  const int64_t n = (int64_t)a.H * a.DH * FP + (a.fold ? (int64_t)a.H * FP * DHP : 0);
+  const int64_t n = (int64_t)a.H * a.DH * FP + (a.fold ? (int64_t)a.H * FP * DHP : 0) +
+                    (a.wqt != nullptr ? (int64_t)a.H * a.DH * a.DQ : 0);
   hipLaunchKernelGGL(transpose_w_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                      (const T *)a.wv, wvt, (const T *)a.wk,
-                     a.fold ? reinterpret_cast<T *>(a.wkt) : nullptr, a.H, a.F, a.DH, FP, DHP);
+                     a.fold ? reinterpret_cast<T *>(a.wkt) : nullptr, (const T *)a.wq,
+                     reinterpret_cast<T *>(a.wqt), a.H, a.F, a.DH, FP, DHP, a.DQ);
+  if (a.wqt != nullptr) {  // q_proj [T, HD] = q_raw [T, DQ] . W_Q, through W_Q^T
+    const int HD = a.H * a.DH;
+    launch_rowgemm<T>(RowGemm{a.q_raw, a.wqt, const_cast<void *>(a.u), a.T_qp, 1, HD, a.DQ, a.DQ,
+                              0, 0, a.DQ, HD, 0}, st);
+  }
   if (a.n_items == 0) return;
   if (mfma_absorb_unprojected(a.H, a.F, a.DH, a.fold)) {
     switch (FP) {

@@ -251,7 +251,7 @@ void varlen_bwd_all(const VarlenArgs &a, hipStream_t st) {
 // ---- absorb ---------------------------------------------------------------
 struct AbsorbWs {
   float *part_o = nullptr, *part_lse = nullptr, *delta = nullptr, *dax = nullptr, *ax = nullptr,
-        *dwv_part = nullptr;
+        *dwv_part = nullptr, *part_du = nullptr, *part_ax = nullptr;
   void *wvt = nullptr, *wkt = nullptr, *axf = nullptr;
   // D_KV padded to a multiple of 8: copies of u, X, W_V and (backward) the
   // padded du, dX, dW_V
@@ -322,6 +322,8 @@ AbsorbWs carve_absorb(void *ws, const vafa_plan_info *info, int64_t F0, int64_t 
     w.tchunk = Tq > 0 ? (Tq + kDwvChunks - 1) / kDwvChunks : 0;
     w.n_tchunks = Tq > 0 ? (Tq + w.tchunk - 1) / w.tchunk : 0;
     w.dwv_part = c.take<float>((w.n_tchunks > 0 ? w.n_tchunks : 1) * F * H * DH * 4);
+    w.part_du = c.take<float>(info->n_fpart_rows * H * F * 4);
+    w.part_ax = c.take<float>(info->n_fpart_rows * H * F * 4);
   }
   w.bytes = c.used;
   return w;
@@ -781,6 +783,22 @@ int64_t vafa_absorb_fwd_fold_workspace(const vafa_plan_info *info, int64_t D_KV,
   return carve_absorb(nullptr, info, D_KV, D_H, false, true).bytes;
 }
 
+static AbsorbArgs fold_args(const void *q_proj, const void *W_K, const void *X, const void *W_V,
+                            void *O, float *lse, const int32_t *plan_dev,
+                            const vafa_plan_info *info, int64_t D_KV, int64_t D_H, float scale,
+                            const AbsorbWs &w) {
+  AbsorbArgs a{};
+  a.u = q_proj; a.wk = W_K; a.wkt = w.wkt; a.fold = true;
+  a.X = X; a.wv = W_V; a.O = O; a.lse = lse;
+  a.part_o = w.part_o; a.part_lse = w.part_lse; a.wvt = w.wvt;
+  a.items = plan_dev + info->off_fwd; a.n_items = info->n_fwd;
+  a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
+  a.comb_rows = (int)info->max_comb_rows;
+  a.T_q = info->T_q; a.T_k = info->T_k;
+  a.H = (int)info->H; a.F = (int)D_KV; a.DH = (int)D_H; a.scale = scale;
+  return a;
+}
+
 int vafa_absorb_fwd_fold(const void *q_proj, const void *W_K, const void *X, const void *W_V,
                          void *O, float *lse, const int32_t *plan_dev,
                          const vafa_plan_info *info, int64_t D_KV, int64_t D_H, int32_t dtype,
@@ -798,17 +816,54 @@ int vafa_absorb_fwd_fold(const void *q_proj, const void *W_K, const void *X, con
   if (workspace_bytes < w.bytes || (w.bytes > 0 && workspace == nullptr))
     return fail(VAFA_ERR_WORKSPACE, "workspace of %lld bytes, %lld needed",
                 (long long)workspace_bytes, (long long)w.bytes);
-  AbsorbArgs a{};
-  a.u = q_proj; a.wk = W_K; a.wkt = w.wkt; a.fold = true;
-  a.X = X; a.wv = W_V; a.O = O; a.lse = lse;
-  a.part_o = w.part_o; a.part_lse = w.part_lse; a.wvt = w.wvt;
-  a.items = plan_dev + info->off_fwd; a.n_items = info->n_fwd;
-  a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
-  a.comb_rows = (int)info->max_comb_rows;
-  a.T_q = info->T_q; a.T_k = info->T_k;
-  a.H = (int)info->H; a.F = (int)D_KV; a.DH = (int)D_H; a.scale = scale;
+  const AbsorbArgs a =
+      fold_args(q_proj, W_K, X, W_V, O, lse, plan_dev, info, D_KV, D_H, scale, w);
   if (int rc = by_dtype<AFwd>(dtype, a, (hipStream_t)stream)) return rc;
   return check_launch("vafa_absorb_fwd_fold");
+}
+
+// W_Q^T leads the folded forward's workspace.
+static int64_t full_wqt_bytes(const vafa_plan_info *info, int64_t D_Q, int64_t D_H) {
+  return align_up(info->H * D_H * D_Q * 2);
+}
+
+int64_t vafa_absorb_fwd_full_workspace(const vafa_plan_info *info, int64_t D_Q, int64_t D_KV,
+                                       int64_t D_H) {
+  if (check_info(info, 2)) return -1;
+  if (check_project_dims("fwd_full_workspace", 0, info->H, D_Q, D_KV, D_H)) return -1;
+  return full_wqt_bytes(info, D_Q, D_H) +
+         carve_absorb(nullptr, info, D_KV, D_H, false, true).bytes;
+}
+
+int vafa_absorb_fwd_full(const void *q_raw, const void *X, const void *W_Q, const void *W_K,
+                         const void *W_V, void *q_proj, void *O, float *lse, int64_t T_q,
+                         const int32_t *plan_dev, const vafa_plan_info *info, int64_t D_Q,
+                         int64_t D_KV, int64_t D_H, int32_t dtype, float scale, void *workspace,
+                         int64_t workspace_bytes, void *stream) {
+  if (int rc = check_info(info, 2)) return rc;
+  if (int rc = check_absorb_dims(D_KV, D_H)) return rc;
+  if (int rc = check_project_dims("absorb_fwd_full", T_q, info->H, D_Q, D_KV, D_H)) return rc;
+  if (info->T_q > T_q)
+    return fail(VAFA_ERR_VALUE, "absorb_fwd_full: the plan addresses %lld query tokens of %lld",
+                (long long)info->T_q, (long long)T_q);
+  if (!fold_supported(info->H, D_KV, D_H, dtype))
+    return fail(VAFA_ERR_VALUE,
+                "absorb_fwd_full: H=%lld, D_KV=%lld, D_H=%lld, dtype %d is not a shape of the "
+                "folded kernel (vafa_absorb_fold_supported)",
+                (long long)info->H, (long long)D_KV, (long long)D_H, (int)dtype);
+  if (int rc = check_aligned("absorb_fwd_full",
+                             {q_raw, X, W_Q, W_K, W_V, q_proj, O, workspace}))
+    return rc;
+  const int64_t lead = full_wqt_bytes(info, D_Q, D_H);
+  AbsorbWs w = carve_absorb(workspace ? static_cast<char *>(workspace) + lead : nullptr, info,
+                            D_KV, D_H, false, true);
+  if (workspace == nullptr || workspace_bytes < lead + w.bytes)
+    return fail(VAFA_ERR_WORKSPACE, "workspace of %lld bytes, %lld needed",
+                (long long)workspace_bytes, (long long)(lead + w.bytes));
+  AbsorbArgs a = fold_args(q_proj, W_K, X, W_V, O, lse, plan_dev, info, D_KV, D_H, scale, w);
+  a.q_raw = q_raw; a.wq = W_Q; a.wqt = workspace; a.T_qp = T_q; a.DQ = (int)D_Q;
+  if (int rc = by_dtype<AFwd>(dtype, a, (hipStream_t)stream)) return rc;
+  return check_launch("vafa_absorb_fwd_full");
 }
 
 int vafa_absorb_project_u(const void *q_proj, const void *W_K, void *u, int64_t T_q, int64_t H,
@@ -894,6 +949,9 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
                     int64_t workspace_bytes, void *stream) {
   if (int rc = check_info(info, 2)) return rc;
   if (int rc = check_absorb_dims(D_KV, D_H)) return rc;
+  if (info->n_dqc > 0 && info->H > kAbsorbRows)
+    return fail(VAFA_ERR_VALUE, "plan splits token tiles, which H=%lld does not run",
+                (long long)info->H);
   AbsorbWs w = carve_absorb(workspace, info, D_KV, D_H, true);
   if (workspace_bytes < w.bytes || (w.bytes > 0 && workspace == nullptr))
     return fail(VAFA_ERR_WORKSPACE, "workspace of %lld bytes, %lld needed",
@@ -914,11 +972,17 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
   }
   a.delta = w.delta; a.dax = w.dax; a.ax = w.ax; a.dwv_part = w.dwv_part;
   a.n_tchunks = w.n_tchunks; a.tchunk = w.tchunk;
+  a.part_du = w.part_du; a.part_ax = w.part_ax;
+  a.qtc_items = plan_dev + info->off_dqc; a.n_qtc = info->n_dqc;
+  a.qtc_rows = (int)info->max_dqc_rows;
   a.items = plan_dev + info->off_fwd; a.n_items = info->n_fwd;
   a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
   a.comb_rows = (int)info->max_comb_rows;
   a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
   a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
+  if (info->n_dq > 0) {  // the du pass splits key ranges
+    a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
+  }
   a.T_q = info->T_q; a.T_k = info->T_k;
   a.H = (int)info->H; a.F = (int)F; a.DH = (int)D_H; a.scale = scale;
   if (int rc = by_dtype<ABwd>(dtype, a, st)) return rc;

@@ -53,6 +53,7 @@ struct AbsorbArgs {
   void *dax;                  // dO W_V^T [T_q, H, F] in the input dtype (backward)
   float *ax;                  // aX [T_q, H, F] fp32 (backward, for dW_V)
   float *dwv_part;            // [n_tchunks, F, H, D_H] fp32 (backward)
+  float *part_du, *part_ax;   // du / aX partials of split token tiles [rows, H, F] fp32
   void *wvt;                  // W_V re-laid out as [H, D_H, F padded to 32] (forward)
   // forward with mfma_absorb_unprojected: rounded aX/l rows [T_q, H, FP] in
   // wvt's f order (part_o then holds [rows, H, FP] unprojected partials)
@@ -64,10 +65,19 @@ struct AbsorbArgs {
   const void *wk;
   void *wkt;
   bool fold;
+  // whole op (folded forward with wqt set): q_raw [T_qp, DQ] and W_Q [DQ, H,
+  // D_H]; q_proj is formed into `u` through W_Q^T in wqt
+  const void *q_raw, *wq;
+  void *wqt;
+  int64_t T_qp;
+  int DQ;
   const int32_t *items, *comb_items, *kv_items, *qseg_items;
   int64_t n_items, n_comb, n_kv, n_qseg;
   int64_t n_kv_res;           // leading kv items for absorb_dx_res_kernel
   int comb_rows;              // most tokens of one combine item
+  const int32_t *qtc_items;   // split token tiles of the du pass
+  int64_t n_qtc;
+  int qtc_rows;               // most tokens of one of them
   int64_t T_q, T_k;
   int64_t n_tchunks, tchunk;
   int H, F, DH;
@@ -127,6 +137,10 @@ void launch_unpad_cols(const void *src, void *dst, int64_t rows, int64_t n, int6
 // out[o] = sum_c part[c * n_out + o] in chunk order, rounded to T
 template <typename T>
 void launch_chunk_sum(const float *part, void *out, int64_t n_out, int64_t n_chunks, hipStream_t);
+// du (rounded to T) and aX of the du pass's split token tiles: ordered sums of
+// their key chunks' fp32 partials (F % 4 == 0)
+template <typename T>
+void launch_du_combine(const AbsorbArgs &, hipStream_t);
 // dAX = dO W_V^T, fp32 [T_q, H, F]
 template <typename T>
 void launch_absorb_dax(const AbsorbArgs &, hipStream_t);

@@ -46,6 +46,20 @@ struct Item {
   int64_t cost;
 };
 
+// A plan section: its items and the order in which they are laid out (kNoop:
+// an empty slot of the XCD-aware layout).
+constexpr uint32_t kNoop = UINT32_MAX;
+struct Section {
+  std::vector<Item> items;
+  std::vector<uint32_t> order;
+  void push_back(const Item &it) { items.push_back(it); }
+  // items in the order they were pushed
+  void keep_order() {
+    order.resize(items.size());
+    std::iota(order.begin(), order.end(), 0u);
+  }
+};
+
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int64_t round_up(int64_t a, int64_t b) { return cdiv(a, b) * b; }
 
@@ -99,9 +113,34 @@ void varlen_tiles(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t 
   *xcd_heads = work > 0.0 && 2.0 * long_q < work ? 1 : 0;
 }
 
-void sort_lpt(std::vector<Item> &items) {
-  std::stable_sort(items.begin(), items.end(),
-                   [](const Item &a, const Item &b) { return a.cost > b.cost; });
+// Indices of `cost` in descending order, equal costs in index order: a
+// radix sort (a launch of thousands of samples sorts up to 100k items).
+std::vector<uint32_t> order_lpt(const std::vector<int64_t> &cost) {
+  const size_t n = cost.size();
+  std::vector<uint32_t> idx(n), tmp(n);
+  std::iota(idx.begin(), idx.end(), 0u);
+  if (n < 2) return idx;
+  const auto mm = std::minmax_element(cost.begin(), cost.end());
+  const int64_t top = *mm.second;
+  const uint64_t span = (uint64_t)(top - *mm.first);
+  constexpr int kBits = 11;
+  for (int shift = 0; shift < 64 && (span >> shift) != 0; shift += kBits) {
+    auto digit = [&](uint32_t i) {
+      return (uint32_t)((uint64_t)(top - cost[i]) >> shift) & ((1u << kBits) - 1);
+    };
+    uint32_t at[(1 << kBits) + 1] = {0};
+    for (uint32_t i : idx) ++at[digit(i) + 1];
+    for (int d = 0; d < (1 << kBits); ++d) at[d + 1] += at[d];
+    for (uint32_t i : idx) tmp[at[digit(i)]++] = i;
+    idx.swap(tmp);
+  }
+  return idx;
+}
+
+void sort_lpt(Section &s) {
+  std::vector<int64_t> cost(s.items.size());
+  for (size_t i = 0; i < cost.size(); ++i) cost[i] = s.items[i].cost;
+  s.order = order_lpt(cost);
 }
 
 // Items that read the same key range (same segment and split, different
@@ -109,58 +148,50 @@ void sort_lpt(std::vector<Item> &items) {
 // least-loaded XCD and the grid is laid out in rounds of kXcds slots, slot x
 // running on XCD x, so the members of a bundle run back to back on one XCD
 // and share its L2.  Empty slots are padded with no-op items (t0 == t1).
-std::vector<Item> xcd_bundle(const std::vector<Item> &items) {
-  std::vector<std::vector<Item>> bundles;
+void xcd_bundle(Section &s) {
+  const std::vector<Item> &items = s.items;
+  std::vector<uint32_t> first;  // a bundle's first item; its members follow it
   std::vector<int64_t> cost;
-  for (const Item &it : items) {
+  for (size_t i = 0; i < items.size(); ++i) {
     // split items of one tile are emitted consecutively per (segment, split)
-    bool joined = false;
-    if (!bundles.empty()) {
-      const Item &h = bundles.back().front();
-      joined = h.v[5] == it.v[5] && h.v[6] == it.v[6] && h.v[2] == it.v[2] && h.v[3] == it.v[3];
-    }
+    const Item &it = items[i];
+    const bool joined = !first.empty() && [&](const Item &h) {
+      return h.v[5] == it.v[5] && h.v[6] == it.v[6] && h.v[2] == it.v[2] && h.v[3] == it.v[3];
+    }(items[first.back()]);
     if (!joined) {
-      bundles.emplace_back();
+      first.push_back((uint32_t)i);
       cost.push_back(0);
     }
-    bundles.back().push_back(it);
     cost.back() += it.cost;
   }
-  std::vector<size_t> order(bundles.size());
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(),
-                   [&](size_t a, size_t b) { return cost[a] > cost[b]; });
-  std::vector<std::vector<Item>> q(kXcds);
-  std::vector<int64_t> load(kXcds, 0);
-  for (size_t b : order) {
-    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    for (const Item &it : bundles[b]) q[x].push_back(it);
+  std::vector<uint32_t> q[kXcds];
+  int64_t load[kXcds] = {0};
+  for (uint32_t b : order_lpt(cost)) {
+    const int x = (int)(std::min_element(load, load + kXcds) - load);
+    const uint32_t end = b + 1 < first.size() ? first[b + 1] : (uint32_t)items.size();
+    for (uint32_t i = first[b]; i < end; ++i) q[x].push_back(i);
     load[x] += cost[b];
   }
   size_t rounds = 0;
   for (const auto &v : q) rounds = std::max(rounds, v.size());
-  std::vector<Item> out;
-  out.reserve(rounds * kXcds);
-  const Item noop{{0, 0, 0, 0, -1, -1, 0, 1}, 0};
+  s.order.reserve(rounds * kXcds);
   for (size_t r = 0; r < rounds; ++r)
-    for (int x = 0; x < kXcds; ++x) out.push_back(r < q[x].size() ? q[x][r] : noop);
-  return out;
+    for (int x = 0; x < kXcds; ++x) s.order.push_back(r < q[x].size() ? q[x][r] : kNoop);
 }
 
-int64_t max_rows(const std::vector<Item> &comb) {
+int64_t max_rows(const Section &comb) {
   // combine items start {q0, q1, ...} in every plan
   int64_t m = 0;
-  for (const Item &it : comb) m = std::max<int64_t>(m, it.v[1] - it.v[0]);
+  for (const Item &it : comb.items) m = std::max<int64_t>(m, it.v[1] - it.v[0]);
   return m;
 }
 
 // Lays the sections out back to back: fwd, comb, kv, qt, then the varlen
 // backward's dq, dqc, fkv, fcomb.
-int emit(const std::vector<Item> &fwd, const std::vector<Item> &comb,
-         const std::vector<Item> &kv, const std::vector<Item> &qt, const std::vector<Item> &dq,
-         const std::vector<Item> &dqc, const std::vector<Item> &fkv,
-         const std::vector<Item> &fcomb, int32_t *plan, int64_t cap, vafa_plan_info *info) {
-  const std::vector<Item> *secs[] = {&fwd, &comb, &kv, &qt, &dq, &dqc, &fkv, &fcomb};
+int emit(const Section &fwd, const Section &comb, const Section &kv, const Section &qt,
+         const Section &dq, const Section &dqc, const Section &fkv, const Section &fcomb,
+         int32_t *plan, int64_t cap, vafa_plan_info *info) {
+  const Section *secs[] = {&fwd, &comb, &kv, &qt, &dq, &dqc, &fkv, &fcomb};
   int64_t *offs[] = {&info->off_fwd, &info->off_comb, &info->off_kv, &info->off_qt,
                      &info->off_dq, &info->off_dqc, &info->off_fkv, &info->off_fcomb};
   int64_t *counts[] = {&info->n_fwd, &info->n_comb, &info->n_kv, &info->n_qt,
@@ -168,7 +199,7 @@ int emit(const std::vector<Item> &fwd, const std::vector<Item> &comb,
   int64_t off = 0;
   for (int i = 0; i < 8; ++i) {
     *offs[i] = off;
-    *counts[i] = (int64_t)secs[i]->size();
+    *counts[i] = (int64_t)secs[i]->order.size();
     off += *counts[i] * VAFA_ITEM_INTS;
   }
   info->plan_ints = off;
@@ -180,9 +211,10 @@ int emit(const std::vector<Item> &fwd, const std::vector<Item> &comb,
     return fail(VAFA_ERR_CAPACITY, "plan buffer holds %lld int32, %lld needed",
                 (long long)cap, (long long)info->plan_ints);
   int32_t *p = plan;
-  for (const auto *sec : secs)
-    for (const Item &it : *sec) {
-      std::memcpy(p, it.v, sizeof(it.v));
+  const Item noop{{0, 0, 0, 0, -1, -1, 0, 1}, 0};
+  for (const Section *sec : secs)
+    for (uint32_t i : sec->order) {
+      std::memcpy(p, i == kNoop ? noop.v : sec->items[i].v, sizeof(noop.v));
       p += VAFA_ITEM_INTS;
     }
   return VAFA_OK;
@@ -322,7 +354,7 @@ int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   info->q_tile = BM;
   info->k_tile = BK;
   info->xcd_heads = xcd_heads;
-  std::vector<Item> fwd, comb, kv, fkv, fcomb;
+  Section fwd, comb, kv, fkv, fcomb, dq, dqc;
   std::vector<char> fused(n1 > 1 ? n1 - 1 : 0, 0);
   int64_t prow = 0, fprow = 0;
   int64_t max_split = 1;
@@ -375,11 +407,14 @@ int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   sort_lpt(fwd);
   sort_lpt(kv);
   sort_lpt(fkv);
-  std::vector<Item> dq, dqc;
-  for (const Item &it : fwd)
-    if (!fused[it.v[5]]) dq.push_back(it);
-  for (const Item &it : comb)
+  comb.keep_order();
+  fcomb.keep_order();
+  for (uint32_t i : fwd.order)
+    if (!fused[fwd.items[i].v[5]]) dq.push_back(fwd.items[i]);
+  for (const Item &it : comb.items)
     if (!fused[it.v[4]]) dqc.push_back(it);
+  dq.keep_order();
+  dqc.keep_order();
   info->n_part_rows = prow;
   info->n_fpart_rows = fprow;
   info->max_split = max_split;
@@ -399,6 +434,11 @@ int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
 //                 segment's whole token range [t0, t1).
 //   qt section  : {t0, t1, k0, k1, -1, seg, 0, 1} unsplit token tiles with the
 //                 segment's whole key range (backward dU pass).
+//   dq, dqc     : where the dU pass splits key ranges (its own policy), the
+//                 items it runs instead of qt, {t0, t1, k0, k1, pbase, seg,
+//                 split, nsplit} with fp32 du / aX partials in rows pbase + r
+//                 (n_fpart_rows in all), and one item per split tile, laid out
+//                 as the comb items.
 int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
                      int64_t D_KV, int64_t D_H, int32_t *plan, int64_t plan_cap,
                      vafa_plan_info *info) {
@@ -408,21 +448,28 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   (void)D_KV;
   (void)D_H;
   const int64_t TT = std::max<int64_t>(1, kAbsorbRows / H);
-  const int64_t BK = kAbsorbKTile;
-  // Key chunk of split segments, from the launch's total work: a chunk holds
-  // kAbsorbSplitSlack times the average keys per resident forward workgroup
-  // (never below kAbsorbPolicy.long_chunk), and only longer key ranges split.
-  // Longest-first order starts such items at once, so they end within the
-  // kernel; every extra item costs a prologue, an epilogue and a combine.
-  SplitPolicy pol = kAbsorbPolicy;
-  {
-    int64_t work = 0;  // sum over segments of (token tiles x keys)
-    for (int64_t s = 0; s + 1 < n1; ++s)
-      if (cu_q[s + 1] > cu_q[s]) work += cdiv(cu_q[s + 1] - cu_q[s], TT) * (cu_k[s + 1] - cu_k[s]);
-    const int64_t chunk = round_up(cdiv(kAbsorbSplitSlack * work, kAbsorbSlots), pol.align);
-    pol.long_chunk = std::max<int64_t>(pol.long_chunk, chunk);
-    pol.long_threshold = pol.long_chunk;
+  const int64_t BK = cu_k[n1 - 1] <= kAbsorbSmallKeys ? kAbsorbSmallKTile : kAbsorbKTile;
+  // Key chunks of split segments, from the launch's total work: a chunk holds
+  // a multiple of the average keys per resident workgroup (never below the
+  // policy's long_chunk), and only longer key ranges split.  Longest-first
+  // order starts such items at once, so they end within the kernel; every
+  // extra item costs a prologue, an epilogue and a combine.
+  SplitPolicy pol = kAbsorbPolicy, du_pol = kAbsorbDuPolicy;
+  int64_t work = 0, n_tiles = 0;  // sum over segments of (token tiles x keys), and of tiles
+  for (int64_t s = 0; s + 1 < n1; ++s) {
+    const int64_t tiles = cdiv(cu_q[s + 1] - cu_q[s], TT);
+    n_tiles += tiles;
+    work += tiles * (cu_k[s + 1] - cu_k[s]);
   }
+  auto raise_chunk = [work](SplitPolicy &p, int64_t slack, int64_t slots) {
+    p.long_chunk = std::max<int64_t>(p.long_chunk, round_up(cdiv(slack * work, slots), p.align));
+    p.long_threshold = p.long_chunk;
+  };
+  raise_chunk(pol, kAbsorbSlack2, 2 * kAbsorbSlots);
+  raise_chunk(du_pol, kAbsorbDuSlack, kAbsorbDuSlots);
+  bool du_split = false;  // some token tile's range is split
+  for (int64_t s = 0; s + 1 < n1 && H <= kAbsorbRows && !du_split; ++s)
+    du_split = cu_q[s + 1] > cu_q[s] && cu_k[s + 1] - cu_k[s] > du_pol.long_threshold;
   std::memset(info, 0, sizeof(*info));
   info->magic = VAFA_PLAN_MAGIC;
   info->kind = 2;
@@ -432,21 +479,48 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   info->H = H;
   info->q_tile = TT;
   info->k_tile = BK;
-  std::vector<Item> fwd, comb, kv, qt;
-  int64_t prow = 0, max_split = 1;
+  Section fwd, comb, kv, qt, qs, qsc;
+  fwd.items.reserve(n_tiles);
+  qt.items.reserve(n_tiles);
+  kv.items.reserve(cu_k[n1 - 1] / BK + n1);
+  int64_t prow = 0, qprow = 0, max_split = 1;
   for (int64_t s = 0; s + 1 < n1; ++s) {
     const int64_t q0 = cu_q[s], q1 = cu_q[s + 1], k0 = cu_k[s], k1 = cu_k[s + 1];
     const int64_t lq = q1 - q0, lk = k1 - k0;
     // one split decision per segment (its tiles share the key ranges)
     int64_t ns = 1, chunk = lk;
-    if (lq > 0) key_split(std::min<int64_t>(lq, TT) * H, lk, pol, &ns, &chunk);
+    if (lq > 0) {
+      // chunks below kAbsorbWideChunk only as far as kAbsorbFineSplits of them
+      // cover the range
+      SplitPolicy p = pol;
+      p.long_chunk = std::max(p.long_chunk,
+                              std::min(kAbsorbWideChunk, cdiv(lk, kAbsorbFineSplits)));
+      p.long_threshold = p.long_chunk;
+      key_split(std::min<int64_t>(lq, TT) * H, lk, p, &ns, &chunk);
+    }
     max_split = std::max(max_split, ns);
+    // the du pass's own split; the wave-per-row kernels (H > kAbsorbRows) walk
+    // whole key ranges
+    int64_t du_ns = 1, du_chunk = lk;
+    if (du_split && lq > 0) key_split(kAbsorbRows, lk, du_pol, &du_ns, &du_chunk);
     const int64_t seg_prow = prow;
     for (int64_t t = q0; t < q1; t += TT) {
       const int64_t te = std::min(t + TT, q1), ntok = te - t;
       const int64_t row_cost = round_up(ntok * H, 32);
       qt.push_back(Item{{(int32_t)t, (int32_t)te, (int32_t)k0, (int32_t)k1, -1, (int32_t)s, 0, 1},
                         (lk + pol.item_overhead) * row_cost});
+      for (int64_t j = 0; du_split && j < du_ns; ++j) {
+        const int64_t a = k0 + j * du_chunk, b = du_ns > 1 ? std::min(k1, a + du_chunk) : k1;
+        const int32_t pb = du_ns > 1 ? (int32_t)(qprow + j * ntok) : -1;
+        qs.push_back(Item{{(int32_t)t, (int32_t)te, (int32_t)a, (int32_t)b, pb, (int32_t)s,
+                           (int32_t)j, (int32_t)du_ns},
+                          ((b - a) + du_pol.item_overhead) * row_cost});
+      }
+      if (du_ns > 1) {
+        qsc.push_back(Item{{(int32_t)t, (int32_t)te, (int32_t)qprow, (int32_t)du_ns, (int32_t)s, 0,
+                            0, 0}, 0});
+        qprow += du_ns * ntok;
+      }
       if (ns > 1) {
         Item c{{(int32_t)t, (int32_t)te, (int32_t)prow, (int32_t)ns, (int32_t)s, 0, 0, 0}, 0};
         comb.push_back(c);
@@ -475,17 +549,22 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
       kv.push_back(it);
     }
   }
-  fwd = xcd_bundle(fwd);
+  xcd_bundle(fwd);
   sort_lpt(kv);
   // resident-row items first, so each dX kernel is launched over its own items
-  const auto res_end = std::stable_partition(kv.begin(), kv.end(), [H](const Item &it) {
+  const auto res_end = std::stable_partition(kv.order.begin(), kv.order.end(), [&](uint32_t i) {
+    const Item &it = kv.items[i];
     return (int64_t)(it.v[3] - it.v[2]) * H <= kDxResidentRows;
   });
-  info->n_kv_res = (int64_t)(res_end - kv.begin());
+  info->n_kv_res = (int64_t)(res_end - kv.order.begin());
   sort_lpt(qt);
+  sort_lpt(qs);
+  comb.keep_order();
+  qsc.keep_order();
   info->n_part_rows = prow;
+  info->n_fpart_rows = qprow;
   info->max_split = max_split;
-  return emit(fwd, comb, kv, qt, {}, {}, {}, {}, plan, plan_cap, info);
+  return emit(fwd, comb, kv, qt, qs, qsc, {}, {}, plan, plan_cap, info);
 }
 
 }  // extern "C"

@@ -12,10 +12,17 @@ namespace vafa {
 constexpr int kVarlenTile = 128;
 constexpr int kVarlenWideTile = 256;
 // Absorb: a forward workgroup covers up to kAbsorbRows (token, head) rows;
-// a dX workgroup covers up to kAbsorbKTile keys of one sample (four 128-key
-// sub-tiles on the matrix-core path).
+// a dX workgroup covers up to kAbsorbKTile keys of one sample (two 128-key
+// sub-tiles on the matrix-core path), kAbsorbSmallKTile in launches of at most
+// kAbsorbSmallKeys keys, whose dX grid would leave CUs idle.  GPU time of
+// forward + backward, us, at 512 / 256 / 128 keys: C4 (648k keys) 543 / 543 /
+// 547, 1127 samples of <= 2048 keys (1.37M) 969 / 949 / 994, 256 and 64 C4
+// samples (80k, 20k) 162 / 155 / 157 and 131 / 121 / 115, 512 C4 samples in
+// fp32 (157k) 984 / 938 / 893.
 constexpr int kAbsorbRows = 64;
-constexpr int kAbsorbKTile = 512;
+constexpr int kAbsorbKTile = 256;
+constexpr int kAbsorbSmallKTile = 128;
+constexpr int64_t kAbsorbSmallKeys = 192 * 1024;
 
 struct SplitPolicy {
   // Query tiles with at most `decode_rows` rows against >= decode_min_keys
@@ -29,16 +36,33 @@ struct SplitPolicy {
 };
 
 constexpr SplitPolicy kVarlenPolicy{16, 1024, 2048, 4, 16, 4096, 4096, 64, 64};
-// Absorb: long_chunk is the smallest key chunk; the planner raises chunk and
-// threshold with the launch's total work (see vafa_plan_absorb).
-constexpr SplitPolicy kAbsorbPolicy{0, 1 << 30, 1024, 1, 16, 1024, 1024, 64, 32};
-// Resident absorb forward workgroups on the MI355X (256 CUs x 3), and the
-// multiple of the average keys per workgroup that a key range may hold
-// before it is split (measured: splitting configs[4]'s <= 8192-key samples
-// into 1024-key chunks cost 10%, configs[3]'s <= 2000-key samples at 1024
-// keys 4%).
+// Absorb forward key splits.  A chunk holds kAbsorbSlack2 / 2 times the
+// average keys per resident forward workgroup (256 CUs x 3 on the MI355X), so
+// large launches stay whole (splitting C5's <= 8192-key samples into 1024-key
+// chunks cost 10%, C4's <= 2000-key samples at 1024 keys 4%), and a small
+// launch splits down to long_chunk keys, where one workgroup's walk over the
+// longest sample is the launch's whole time.  Chunks below kAbsorbWideChunk
+// are taken only while kAbsorbFineSplits of them cover the range (each costs a
+// prologue, an epilogue and a partial row set).  GPU time of the forward, us,
+// with chunks of at least 1024 keys at 3x the average -> this rule: 16 C4
+// samples 43.7 -> 31.5, 256 / 512 skewed (C5) samples 157 / 275 -> 139 / 236,
+// 512 C4 samples in fp32 246 -> 235, C4 and C5 themselves unchanged; smallest
+// chunk 128 / 256 / 512: 31.4 / 33.9 / 38.2 on the 16 samples.
+constexpr SplitPolicy kAbsorbPolicy{0, 1 << 30, 128, 1, 16, 128, 128, 64, 32};
+constexpr int64_t kAbsorbWideChunk = 1024;
+constexpr int64_t kAbsorbFineSplits = 16;
 constexpr int64_t kAbsorbSlots = 768;
-constexpr int64_t kAbsorbSplitSlack = 3;
+constexpr int64_t kAbsorbSlack2 = 5;
+// Absorb backward, dU pass: two resident workgroups per CU; a chunk holds
+// kAbsorbDuSlack times the average keys per workgroup.  A split tile writes
+// and re-reads 8 bytes of fp32 partials per (row, feature), so chunks stay at
+// 256 keys and up.  GPU time of forward + backward, us, whole ranges -> split:
+// 64 / 256 / 700 C4 samples 158 / 201 / 257 -> 131 / 162 / 234, 512 and 64 C4
+// samples in fp32 1318 -> 985 and 872 -> 548; all of C4 unchanged (544, whole
+// at this slack; 553 at half of it).
+constexpr SplitPolicy kAbsorbDuPolicy{0, 1 << 30, 256, 1, 16, 256, 256, 64, 32};
+constexpr int64_t kAbsorbDuSlots = 512;
+constexpr int64_t kAbsorbDuSlack = 2;
 
 // Varlen backward, fused K-major path (dQ, dK, dV in one kernel, fp32 dQ
 // partials per key chunk summed in order): segments with at most kFusedMaxQ

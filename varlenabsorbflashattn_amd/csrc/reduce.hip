@@ -183,6 +183,44 @@ __global__ __launch_bounds__(64 * kCombRows) void sum_combine_kernel(
   }
 }
 
+// Split token tiles of the absorb du pass: du = sum_s part_du[s] (partials
+// carry the scale) rounded to T, aX = sum_s part_ax[s], in split order.  A
+// tile's rows are contiguous in the outputs and in each split's partials, so a
+// block walks one 16-byte chunk per thread over them, kCombBatch splits' loads
+// in flight; blockIdx.y selects du or aX.
+template <typename T>
+__global__ __launch_bounds__(256) void absorb_du_combine_kernel(
+    const float *__restrict__ part_du, const float *__restrict__ part_ax, T *__restrict__ du,
+    float *__restrict__ ax, const int32_t *__restrict__ items, int H, int F, int blocks) {
+  const int item = (int)blockIdx.x / blocks, b = (int)blockIdx.x - item * blocks;
+  const PlanItem it = load_item(items, item);
+  const int t0 = it.v[0], t1 = it.v[1], pbase = it.v[2], ns = it.v[3];
+  const int64_t n = (int64_t)(t1 - t0) * H * F;  // elements of the tile and of one split
+  const int64_t e = ((int64_t)b * 256 + threadIdx.x) * 4;
+  if (e >= n) return;
+  const float *src = (blockIdx.y ? part_ax : part_du) + (int64_t)pbase * H * F + e;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 0; j0 < ns; j0 += kCombBatch) {
+    f32x4 v[kCombBatch];
+#pragma unroll
+    for (int j = 0; j < kCombBatch; ++j)
+      v[j] = *reinterpret_cast<const f32x4 *>(src + (j0 + j < ns ? j0 + j : ns - 1) * n);
+#pragma unroll
+    for (int j = 0; j < kCombBatch; ++j)
+      if (j0 + j < ns) acc += v[j];
+  }
+  const int64_t o = (int64_t)t0 * H * F + e;
+  if (blockIdx.y) {
+    *reinterpret_cast<f32x4 *>(ax + o) = acc;
+  } else {
+    typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
+    T4 w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = from_f<T>(acc[i]);
+    *reinterpret_cast<T4 *>(du + o) = w;
+  }
+}
+
 // dAX[t,h,f] = sum_d dO[t,h,d] W_V[f,h,d]; one block per (t, h) row.
 template <typename T>
 __global__ __launch_bounds__(256) void absorb_dax_kernel(const T *__restrict__ dO,
@@ -522,6 +560,14 @@ void launch_sum_combine(const float *part, void *out, const int32_t *comb_items,
 }
 
 template <typename T>
+void launch_du_combine(const AbsorbArgs &a, hipStream_t st) {
+  if (a.n_qtc == 0) return;
+  const int blocks = (int)blocks_for(((int64_t)a.qtc_rows * a.H * a.F + 3) / 4);
+  hipLaunchKernelGGL(absorb_du_combine_kernel<T>, dim3((unsigned)(a.n_qtc * blocks), 2), dim3(256),
+                     0, st, a.part_du, a.part_ax, (T *)a.du, a.ax, a.qtc_items, a.H, a.F, blocks);
+}
+
+template <typename T>
 void launch_absorb_dax(const AbsorbArgs &a, hipStream_t st) {
   if (a.T_q == 0) return;
   hipLaunchKernelGGL(absorb_dax_kernel<T>, dim3((unsigned)(a.T_q * a.H)), dim3(256), 0, st,
@@ -622,6 +668,7 @@ void launch_unpad16(const void *src, void *dst, int64_t rows, int elem_bytes, hi
                                       const int32_t *, int64_t, int, int, int, hipStream_t);\
   template void launch_sum_combine<T>(const float *, void *, const int32_t *, int64_t, int, \
                                       int, int, hipStream_t);                               \
+  template void launch_du_combine<T>(const AbsorbArgs &, hipStream_t);                      \
   template void launch_absorb_dax<T>(const AbsorbArgs &, hipStream_t);                      \
   template void launch_absorb_dwv<T>(const AbsorbArgs &, hipStream_t);                      \
   template void launch_wgrad<T, T>(const void *, const void *, float *, void *, int64_t,    \
