@@ -322,6 +322,21 @@ VAFA_API int vafa_absorb_project_bwd(const void *q_raw, const void *W_Q, const v
                                      int64_t D_KV, int64_t D_H, int32_t dtype, void *workspace,
                                      int64_t workspace_bytes, void *stream);
 
+/* The projections and their backward on fp32 operands (fp32 matrix cores,
+ * IEEE products; the reference's documented fp32 call): any D_Q and D_KV, D_H a
+ * multiple of 8, 16-byte aligned operands.  u may be NULL in the forward, any
+ * of dq_raw, dW_Q, dW_K in the backward, which alone needs a workspace. */
+VAFA_API int64_t vafa_absorb_project_f32_workspace(int64_t T_q, int64_t H, int64_t D_Q,
+                                                   int64_t D_KV, int64_t D_H);
+VAFA_API int vafa_absorb_project_f32_fwd(const float *q_raw, const float *W_Q, const float *W_K,
+                                         float *q_proj, float *u, int64_t T_q, int64_t H,
+                                         int64_t D_Q, int64_t D_KV, int64_t D_H, void *stream);
+VAFA_API int vafa_absorb_project_f32_bwd(const float *q_raw, const float *W_Q, const float *W_K,
+                                         const float *q_proj, const float *du, float *dq_raw,
+                                         float *dW_Q, float *dW_K, int64_t T_q, int64_t H,
+                                         int64_t D_Q, int64_t D_KV, int64_t D_H, void *workspace,
+                                         int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -443,6 +443,49 @@ def test_project_fwd_bwd_kernels(device, T, d_q, d_kv, H, D_H, dtype):
             (name, float((err - bound).max()), float(err.max()))
 
 
+# D_Q above 512: dW_Q over 256-column slices, the last of 8, 256 and 200 columns
+@pytest.mark.parametrize("T,d_q", [(130, 520), (33, 768), (700, 968)])
+def test_project_wide_dq(device, T, d_q):
+    test_project_fwd_bwd_kernels(device, T, d_q, 64, 2, 32, torch.bfloat16)
+
+
+# fp32 projections: any width (16-byte and single-element accesses), token and
+# column remainders, no tokens.  Each output is a sum of K fp32 products: within
+# (K + 1) ulp of the sum of their magnitudes, for the two chained products twice
+# that; the backward repeats bit for bit.
+@pytest.mark.parametrize("T,d_q,d_kv,H,D_H", [(300, 256, 256, 8, 32), (33, 968, 250, 8, 32),
+                                              (31, 5, 3, 3, 16), (1, 64, 65, 1, 64),
+                                              (0, 64, 64, 2, 32), (97, 20, 12, 2, 128)])
+def test_project_f32(device, T, d_q, d_kv, H, D_H):
+    from varlenabsorbflashattn_amd.absorb import _project_native, _project_u
+    print(f"[project f32] T={T} d_q={d_q} d_kv={d_kv} H={H} D_H={D_H}", flush=True)
+    g = torch.Generator().manual_seed(T + d_q)
+    ins = [torch.randn(T, d_q, generator=g),
+           torch.randn(d_q, H, D_H, generator=g) / math.sqrt(d_q),
+           torch.randn(d_kv, H, D_H, generator=g) / math.sqrt(d_kv)]
+    du = torch.randn(T, H, d_kv, generator=g)
+    dev = [t.to(device).requires_grad_(True) for t in ins]
+    assert _project_native(*dev)
+    u = _project_u(*dev)
+    grads = torch.autograd.grad(u, dev, du.to(device), retain_graph=True)
+    again = torch.autograd.grad(u, dev, du.to(device))
+    assert all(torch.equal(a, b) for a, b in zip(grads, again))
+    q, wq, wk = (t.double() for t in ins)
+    dd = du.double()
+
+    def both(q, wq, wk, dd):  # u, dq_raw, dW_Q, dW_K
+        qp = torch.einsum("tc,chd->thd", q, wq)
+        dqp = torch.einsum("thf,fhd->thd", dd, wk)
+        return (torch.einsum("thd,fhd->thf", qp, wk), torch.einsum("thd,chd->tc", dqp, wq),
+                torch.einsum("tc,thd->chd", q, dqp), torch.einsum("thf,thd->fhd", dd, qp))
+
+    ref, mag = both(q, wq, wk, dd), both(*(t.abs() for t in (q, wq, wk, dd)))
+    k = (d_q + D_H, d_kv + H * D_H, d_kv + T, T + d_q)
+    for got, r, m, n in zip((u, *grads), ref, mag, k):
+        err = (got.detach().cpu().double() - r).abs()
+        assert got.shape == r.shape and (err <= (n + 2) * 2.0 ** -24 * m).all()
+
+
 def test_project_rejects_bad_shapes(device):
     """Unsupported widths and dtypes return an error, and nothing runs."""
     from varlenabsorbflashattn_amd import _lib

@@ -5,7 +5,7 @@
 the matrix-core shapes it forms ``q_proj = q_raw W_Q`` and runs the attention
 with ``u = q_proj W_K^T`` formed inside the attention kernel (u never reaches
 memory in the forward); otherwise it projects ``u`` per head (this library's
-projection kernels, or torch GEMMs for fp32 / odd widths, as in
+projection kernels, or torch GEMMs for odd 16-bit widths, as in
 ta/interface.py:429-435) and calls ``target_attn_inner``, whose forward and
 backward run in ``libvafa.so``:
 scores are taken directly against the raw ``X`` rows, ``aX = softmax(u X^T) X``
@@ -248,21 +248,27 @@ def target_attn_inner(
 
 
 def _project_native(q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -> bool:
-    """Whether ``vafa_absorb_project_fwd/_bwd`` take these operands: CUDA,
-    one 16-bit dtype, D_Q, D_KV and D_H multiples of 8."""
+    """Whether this library's projection kernels take these operands: CUDA,
+    one dtype, D_H a multiple of 8 and, in 16 bits, D_Q and D_KV too."""
     d_q = q_raw.shape[1]
     d_kv, _, D_H = W_K.shape
-    return (q_raw.is_cuda and q_raw.dtype in (torch.bfloat16, torch.float16)
-            and W_Q.dtype == q_raw.dtype and W_K.dtype == q_raw.dtype
-            and d_q % 8 == 0 and d_kv % 8 == 0 and D_H % 8 == 0)
+    if not (q_raw.is_cuda and W_Q.device == W_K.device == q_raw.device
+            and W_Q.dtype == W_K.dtype == q_raw.dtype and D_H % 8 == 0):
+        return False
+    if q_raw.dtype == torch.float32:
+        # (autocast applies to the torch formulation only)
+        return (0 < d_q <= 65536 and 0 < d_kv <= 65536 and W_Q.shape[1] * D_H <= 65536
+                and W_Q.shape[1] <= 1024 and not torch.is_autocast_enabled())
+    return (q_raw.dtype in (torch.bfloat16, torch.float16)
+            and d_q % 8 == 0 and d_kv % 8 == 0)
 
 
 class _Project(torch.autograd.Function):
     """q_proj = q_raw W_Q, u[t,h,:] = q_proj[t,h,:] W_K[:,h,:]^T
-    (ta/interface.py:434-435) for 16-bit operands, forward and backward on
-    the row-GEMM and weight-gradient kernels of ``vafa_absorb_project_fwd`` /
-    ``vafa_absorb_project_bwd``.  Each product is rounded once to the input
-    dtype, as the reference's 16-bit GEMMs and their autograd backward
+    (ta/interface.py:434-435), forward and backward on the row-GEMM and
+    weight-gradient kernels of ``vafa_absorb_project_fwd`` / ``_bwd`` (16-bit)
+    and ``vafa_absorb_project_f32_fwd`` / ``_bwd``.  Each product is rounded
+    once to the input dtype, as the reference's GEMMs and their autograd backward
     (dq_proj = du W_K per head, dq_raw = dq_proj W_Q^T, dW_Q = q_raw^T dq_proj,
     dW_K = du^T q_proj per head); the weight gradients are summed over fixed
     token chunks in order (deterministic)."""
@@ -278,11 +284,16 @@ class _Project(torch.autograd.Function):
         W_K = _aligned(W_K.contiguous())
         q_proj = torch.empty((T_q, H * D_H), dtype=q_raw.dtype, device=q_raw.device)
         u = torch.empty((T_q, H, d_kv), dtype=q_raw.dtype, device=q_raw.device)
-        ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 0), q_raw.device)
-        _lib.check(L.vafa_absorb_project_fwd(
-            q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), u.data_ptr(),
-            T_q, H, d_q, d_kv, D_H, _lib.dtype_code(q_raw.dtype), ws.data_ptr(), ws.numel(),
-            _lib.stream_ptr(q_raw.device)))
+        args = (q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), u.data_ptr(),
+                T_q, H, d_q, d_kv, D_H)
+        st = _lib.stream_ptr(q_raw.device)
+        if q_raw.dtype == torch.float32:
+            _lib.check(L.vafa_absorb_project_f32_fwd(*args, st))
+        else:
+            ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 0),
+                            q_raw.device)
+            _lib.check(L.vafa_absorb_project_fwd(*args, _lib.dtype_code(q_raw.dtype),
+                                                 ws.data_ptr(), ws.numel(), st))
         ctx.save_for_backward(q_raw, W_Q, W_K, q_proj)
         return u
 
@@ -297,15 +308,17 @@ class _Project(torch.autograd.Function):
         dwq = torch.empty_like(W_Q) if need_wq else None
         dwk = torch.empty_like(W_K) if need_wk else None
         L = _lib.lib()
-        ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 1), du.device)
-
-        def ptr(t):
-            return t.data_ptr() if t is not None else None
-
-        _lib.check(L.vafa_absorb_project_bwd(
-            q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), du.data_ptr(),
-            ptr(dq), ptr(dwq), ptr(dwk), T_q, H, d_q, d_kv, D_H, _lib.dtype_code(du.dtype),
-            ws.data_ptr(), ws.numel(), _lib.stream_ptr(du.device)))
+        args = (q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), du.data_ptr(),
+                _lib.ptr(dq), _lib.ptr(dwq), _lib.ptr(dwk), T_q, H, d_q, d_kv, D_H)
+        st = _lib.stream_ptr(du.device)
+        if du.dtype == torch.float32:
+            ws = _workspace(L.vafa_absorb_project_f32_workspace(T_q, H, d_q, d_kv, D_H),
+                            du.device)
+            _lib.check(L.vafa_absorb_project_f32_bwd(*args, ws.data_ptr(), ws.numel(), st))
+        else:
+            ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 1), du.device)
+            _lib.check(L.vafa_absorb_project_bwd(*args, _lib.dtype_code(du.dtype), ws.data_ptr(),
+                                                 ws.numel(), st))
         return dq, dwq, dwk
 
 
@@ -314,7 +327,7 @@ def _fold_native(q_raw, X, W_Q, W_K, W_V) -> bool:
     kernel (vafa_absorb_fwd_fold): the native projection's operands, X and
     W_V of the same dtype on the same device, and a shape of the folded
     matrix-core kernel."""
-    if not _project_native(q_raw, W_Q, W_K):
+    if q_raw.dtype == torch.float32 or not _project_native(q_raw, W_Q, W_K):
         return False
     if X.dtype != q_raw.dtype or W_V.dtype != q_raw.dtype or not (X.is_cuda and W_V.is_cuda):
         return False
@@ -390,9 +403,10 @@ def _project_u(q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -> tor
     """u[t,h,:] = (q_raw[t] W_Q[:,h,:]) W_K[:,h,:]^T (ta/interface.py:434-435),
     contiguous ``[T_q, H, d_kv]``.
 
-    16-bit operands with D_Q, D_KV, D_H multiples of 8 run on ``_Project``
-    (both directions in this library's kernels).  Other operands (fp32, odd
-    widths) take the reference's own formulation on torch's GEMMs: q_proj =
+    CUDA operands run on ``_Project`` (both directions in this library's
+    kernels) in fp32 and, with D_Q, D_KV, D_H multiples of 8, in 16 bits.
+    Other operands (odd 16-bit widths, the CPU) take the reference's own
+    formulation on torch's GEMMs: q_proj =
     q_raw @ W_Q, then u = q_proj @ blockdiag(W_K[:,h,:]^T), ONE GEMM that
     writes u token-major (for finite q_proj the zero blocks add exact zeros
     to each fp32 sum, so every u element is the same sum of products as per

@@ -274,7 +274,8 @@ struct WgSmem {
 template <typename T, int FP, bool DQ>
 __global__ __launch_bounds__(256) void wgrad_kernel(
     const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ Wt, T *__restrict__ dq,
-    float *__restrict__ part, int64_t T_q, int64_t tchunk, int G, int F, int DH, int n_db) {
+    float *__restrict__ part, int64_t T_q, int64_t tchunk, int G, int lda, int DH, int n_db,
+    int n_fb) {
   using M16 = Mfma16<T>;
   using v8 = typename Mfma<T>::v8;
   using S = WgSmem<FP>;
@@ -286,11 +287,15 @@ __global__ __launch_bounds__(256) void wgrad_kernel(
   int64_t b = blockIdx.x;
   const int db = (int)(b % n_db);
   b /= n_db;
+  const int fb = (int)(b % n_fb);  // FP-wide slice of A's columns
+  b /= n_fb;
   const int g = (int)(b % G);
   const int64_t c = b / G;
   const int64_t ta = c * tchunk, tb = ta + tchunk < T_q ? ta + tchunk : T_q;
   const int d0 = db * kWgDB;
   const int dn = DH - d0 < kWgDB ? DH - d0 : kWgDB;
+  A += fb * FP;
+  const int F = lda - fb * FP < FP ? lda - fb * FP : FP;  // columns of this slice
 
   constexpr int kACh = FP / 8;                    // 16-byte chunks per A row
   constexpr int kAPer = kWgTok * kACh / 256;      // A chunks per thread
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(256) void wgrad_kernel(
       const int idx = i * 256 + tid, r = idx / kACh, ch = idx % kACh;
       const int64_t t = t0 + r;
       const bool ok = t < tb && ch * 8 < F;
-      const u32x4 v = *reinterpret_cast<const u32x4 *>(A + (ok ? (t * G + g) * F + ch * 8 : 0));
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(A + (ok ? (t * G + g) * lda + ch * 8 : 0));
       ra[i] = ok ? v : u32x4{0u, 0u, 0u, 0u};
     }
     {
@@ -403,9 +408,101 @@ __global__ __launch_bounds__(256) void wgrad_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int f = 16 * (wave + 4 * j) + 4 * lq + r;
-        if (f < F) part[((c * F + f) * G + g) * DH + d0 + d] = acc[j][dt][r];
+        if (f < F) part[((c * lda + fb * FP + f) * G + g) * DH + d0 + d] = acc[j][dt][r];
       }
     }
+}
+
+// The row GEMM in fp32 (v_mfma_f32_16x16x4_f32): Y[t, g, j] = sum_k X[t, g, k]
+// W[g, j, k] (W rows along k), or with KJ = true W[g, k, j] (rows along j, so
+// q_proj and dq_proj need no transposed copy).  A workgroup covers 32 tokens x
+// 64 columns, a wave 16 columns: the products are small (2397 tokens x 256 x
+// 256: 0.3 GFLOP) and latency-bound, so operands go straight from L2 to
+// registers, 64 k per batch.  In product i of a 16-wide k block lane group lq
+// holds k = 4*lq + i, so a lane's operand is 16 contiguous bytes along k.  Any
+// width runs: VEC = 16-byte accesses where every stride is a multiple of 4.
+// 2397 tokens, D_Q = D_KV = 256 forward and backward: torch's GEMMs, block
+// diagonal and copies took 285 us of GPU time, these kernels and the weight
+// gradients 108.
+template <bool KJ, bool VEC>
+__global__ __launch_bounds__(256) void rowgemm_f32_kernel(
+    const float *__restrict__ X, const float *__restrict__ W, float *__restrict__ Y, int64_t T_q,
+    int G, int J, int K, int64_t ldx, int64_t xs, int64_t ws, int64_t ldw, int64_t ldy,
+    int64_t ys, int n_jb) {
+  constexpr int kU = 4;  // 16-wide k blocks per batch of loads
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
+  int64_t b = blockIdx.x;
+  const int j0 = (int)(b % n_jb) * 64 + (tid >> 6) * 16;
+  b /= n_jb;
+  const int g = (int)(b % G);
+  const int64_t tb = (b / G) * kRgTok;
+  if (j0 >= J) return;
+  const int j = j0 + l16;
+  const float *wg = W + g * ws + (j < J ? (KJ ? j : j * ldw) : 0);
+  const float *xr[2];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const int64_t t = tb + 16 * hf + l16;
+    xr[hf] = X + (t < T_q ? t : T_q - 1) * ldx + g * xs;
+  }
+  // four elements at k .. k+3 of a row (zero past K); clamped loads, then the
+  // select, so that a batch is one round trip
+  auto row4 = [&](const float *row, int k) {
+    f32x4 v;
+    if constexpr (VEC) {
+      v = *reinterpret_cast<const f32x4 *>(row + (k < K ? k : 0));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = k < K ? v[i] : 0.f;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = row[k + i < K ? k + i : 0];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = k + i < K ? v[i] : 0.f;
+    }
+    return v;
+  };
+  auto w4 = [&](int k) {
+    if constexpr (!KJ) return row4(wg, k);
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = wg[(k + i < K ? k + i : 0) * ldw];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < K ? v[i] : 0.f;
+    return v;
+  };
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int kb = 0; kb < K; kb += 16 * kU) {
+    f32x4 wv[kU], xv[kU][2];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int k = kb + 16 * u + 4 * lq;
+      wv[u] = w4(k);
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) xv[u][hf] = row4(xr[hf], k);
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+          acc[hf] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][i], xv[u][hf][i], acc[hf], 0, 0, 0);
+  }
+  // lane: columns j0 + 4*lq + r of token tb + 16*hf + l16
+  const int jo = j0 + 4 * lq;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const int64_t t = tb + 16 * hf + l16;
+    if (t >= T_q || jo >= J) continue;
+    float *y = Y + t * ldy + g * ys + jo;
+    if constexpr (VEC) {
+      *reinterpret_cast<f32x4 *>(y) = acc[hf];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (jo + r < J) y[r] = acc[hf][r];
+    }
+  }
 }
 
 // dst[c, r] = src[r, c] for a [R, C] matrix.
@@ -452,24 +549,41 @@ void rowgemm_ks(const RowGemm &p, hipStream_t st) {
 
 template <typename T, int FP>
 void wgrad_fp(const Wgrad &p, hipStream_t st) {
-  const int n_db = (p.DH + kWgDB - 1) / kWgDB;
-  const int64_t wgs = p.n_chunks * p.G * n_db;
+  const int n_db = (p.DH + kWgDB - 1) / kWgDB, n_fb = (p.F + FP - 1) / FP;
+  const int64_t wgs = p.n_chunks * p.G * n_db * n_fb;
   if (wgs == 0) return;
   constexpr int smem = WgSmem<FP>::kBytes;
   if (p.dq != nullptr) {
     allow_dynamic_lds(reinterpret_cast<const void *>(&wgrad_kernel<T, FP, true>), smem);
     hipLaunchKernelGGL((wgrad_kernel<T, FP, true>), dim3((unsigned)wgs), dim3(256), smem, st,
                        (const T *)p.A, (const T *)p.B, (const T *)p.Wt, (T *)p.dq, p.part, p.T_q,
-                       p.tchunk, p.G, p.F, p.DH, n_db);
+                       p.tchunk, p.G, p.F, p.DH, n_db, n_fb);
   } else {
     allow_dynamic_lds(reinterpret_cast<const void *>(&wgrad_kernel<T, FP, false>), smem);
     hipLaunchKernelGGL((wgrad_kernel<T, FP, false>), dim3((unsigned)wgs), dim3(256), smem, st,
                        (const T *)p.A, (const T *)p.B, nullptr, nullptr, p.part, p.T_q,
-                       p.tchunk, p.G, p.F, p.DH, n_db);
+                       p.tchunk, p.G, p.F, p.DH, n_db, n_fb);
   }
 }
 
 }  // namespace
+
+void launch_rowgemm_f32(const RowGemm &p, bool kj, hipStream_t st) {
+  const int n_jb = (p.J + 63) / 64;
+  const int64_t wgs = (p.T_q + kRgTok - 1) / kRgTok * p.G * n_jb;
+  if (wgs == 0) return;
+  const bool vec = p.J % 4 == 0 && p.K % 4 == 0 && p.ldx % 4 == 0 && p.xs % 4 == 0 &&
+                   p.ws % 4 == 0 && p.ldw % 4 == 0 && p.ldy % 4 == 0 && p.ys % 4 == 0;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, st, (const float *)p.X,
+                       (const float *)p.W, (float *)p.Y, p.T_q, p.G, p.J, p.K, p.ldx, p.xs, p.ws,
+                       p.ldw, p.ldy, p.ys, n_jb);
+  };
+  if (kj)
+    vec ? run(rowgemm_f32_kernel<true, true>) : run(rowgemm_f32_kernel<true, false>);
+  else
+    vec ? run(rowgemm_f32_kernel<false, true>) : run(rowgemm_f32_kernel<false, false>);
+}
 
 bool rowgemm_supported(const RowGemm &p) {
   const bool pos = p.T_q >= 0 && p.G >= 1 && p.J >= 1 && p.K >= 8;
@@ -489,14 +603,18 @@ void launch_rowgemm(const RowGemm &p, hipStream_t st) {
   else rowgemm_ks<T, 1>(p, st);
 }
 
-bool wgrad16_supported(int F) { return F >= 8 && F <= 512 && F % 8 == 0; }
+// Above 512 columns A is taken in slices of kWgSlice (without the fused dq
+// product, which reduces over all of them).  dW_Q at D_Q = 968, 6918 tokens:
+// 96 us on the fp32-product kernel, 27 here.
+bool wgrad16_supported(int F, bool dq) { return F >= 8 && F % 8 == 0 && (F <= 512 || !dq); }
+int wgrad16_slices(int F) { return F <= 512 ? 1 : (F + 255) / 256; }
 
 template <typename T>
 void launch_wgrad16(const Wgrad &p, hipStream_t st) {
   if (p.F <= 64) wgrad_fp<T, 64>(p, st);
   else if (p.F <= 128) wgrad_fp<T, 128>(p, st);
-  else if (p.F <= 256) wgrad_fp<T, 256>(p, st);
-  else wgrad_fp<T, 512>(p, st);
+  else if (p.F > 256 && p.F <= 512) wgrad_fp<T, 512>(p, st);
+  else wgrad_fp<T, 256>(p, st);
   launch_chunk_sum<T>(p.part, p.out, (int64_t)p.F * p.G * p.DH, p.n_chunks, st);
 }
 

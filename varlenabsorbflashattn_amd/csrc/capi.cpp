@@ -432,17 +432,20 @@ int scratch_ptr(void **out) {
 }
 
 
-// Projection shapes: every dimension a positive multiple of 8 (16-byte rows
-// for the row GEMM's loads), H * D_H and the token count within int range.
+// Projection shapes: H * D_H and the token count within int range, D_H a
+// positive multiple of 8, and in 16 bits D_Q and D_KV too (16-byte rows for the
+// row GEMM's loads; the fp32 kernels take any width).
 int check_project_dims(const char *what, int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV,
-                       int64_t D_H) {
-  const bool ok = T_q >= 0 && T_q < (1ll << 31) && H >= 1 && H <= 1024 && D_Q >= 8 &&
-                  D_Q <= 65536 && D_Q % 8 == 0 && D_KV >= 8 && D_KV <= 65536 && D_KV % 8 == 0 &&
-                  D_H >= 8 && D_H % 8 == 0 && H * D_H <= 65536;
+                       int64_t D_H, int32_t dtype = VAFA_BF16) {
+  const int64_t al = dtype == VAFA_F32 ? 1 : 8;
+  const bool ok = T_q >= 0 && T_q < (1ll << 31) && H >= 1 && H <= 1024 && D_Q >= al &&
+                  D_Q <= 65536 && D_Q % al == 0 && D_KV >= al && D_KV <= 65536 &&
+                  D_KV % al == 0 && D_H >= 8 && D_H % 8 == 0 && H * D_H <= 65536;
   if (!ok)
     return fail(VAFA_ERR_VALUE, "%s: T_q=%lld H=%lld D_Q=%lld D_KV=%lld D_H=%lld not supported "
-                "(D_Q, D_KV, D_H positive multiples of 8, H*D_H <= 65536)", what, (long long)T_q,
-                (long long)H, (long long)D_Q, (long long)D_KV, (long long)D_H);
+                "(D_H and, in 16 bits, D_Q and D_KV positive multiples of 8, H*D_H <= 65536)",
+                what, (long long)T_q, (long long)H, (long long)D_Q, (long long)D_KV,
+                (long long)D_H);
   return VAFA_OK;
 }
 
@@ -461,17 +464,20 @@ void project_u(const void *q_proj, const void *W_K, void *u, int64_t T_q, int H,
   launch_rowgemm<T>(RowGemm{q_proj, W_K, u, T_q, H, F, DH, HD, DH, DH, HD, (int64_t)H * F, F}, st);
 }
 
-// Token chunks of a projection weight gradient: on the 16-bit kernel a
-// multiple of 32 tokens, about kWgradWgs workgroups in all (wgs_per_chunk per
-// chunk); on the fp32-product fallback (F > 512) 64 chunks.
+// Token chunks of a projection weight gradient: a multiple of 32 tokens, about
+// kWgradWgs workgroups in all (wgs_per_chunk per chunk); on the fp32-product
+// kernel (fp32 operands; 16-bit dW_K above 512 features) 64 chunks, 32 for fp32
+// operands (one wave per 32 x 32 outputs: 64 and more waves a chunk).
 constexpr int64_t kWgradWgs = 512;
 struct Chunks {
   int64_t tchunk = 0, n = 0;
 };
-Chunks wgrad_chunks(int64_t T_q, int64_t F, int64_t wgs_per_chunk) {
+Chunks wgrad_chunks(int64_t T_q, int64_t F, int64_t wgs_per_chunk, bool dq, bool f32) {
   Chunks c;
   if (T_q <= 0) return c;
-  if (!wgrad16_supported((int)F)) {
+  if (f32) {
+    c.tchunk = (T_q + 31) / 32;
+  } else if (!wgrad16_supported((int)F, dq)) {
     c.tchunk = (T_q + 63) / 64;
   } else {
     const int64_t tiles = (T_q + 31) / 32;
@@ -492,15 +498,15 @@ struct ProjectWs {
 };
 
 ProjectWs carve_project(void *ws, int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV, int64_t D_H,
-                        bool bwd) {
+                        bool bwd, bool f32) {
   Carver c(ws);
   ProjectWs w;
   const int64_t HD = H * D_H;
-  w.wt = c.take<void>(HD * (bwd ? D_KV : D_Q) * 2);
+  if (!f32) w.wt = c.take<void>(HD * (bwd ? D_KV : D_Q) * 2);
   if (bwd) {
-    w.dq_proj = c.take<void>(T_q * HD * 2);
-    w.ck = wgrad_chunks(T_q, D_KV, H * ((D_H + 31) / 32));
-    w.cq = wgrad_chunks(T_q, D_Q, (HD + 31) / 32);
+    w.dq_proj = c.take<void>(T_q * HD * (f32 ? 4 : 2));
+    w.ck = wgrad_chunks(T_q, D_KV, H * ((D_H + 31) / 32), true, f32);
+    w.cq = wgrad_chunks(T_q, D_Q, (HD + 31) / 32 * wgrad16_slices((int)D_Q), false, f32);
     const int64_t pk = w.ck.n * D_KV * HD, pq = w.cq.n * D_Q * HD;
     w.part = c.take<float>((pk > pq ? pk : pq) * 4 + 4);
   }
@@ -528,7 +534,7 @@ void project_bwd(const void *q_raw, const void *W_Q, const void *W_K, const void
   if (need_dq) launch_transpose2d<T>(W_K, w.wt, F, HD, st);
   // dW_K[f, h, d] = sum_t du[t, h, f] q_proj[t, h, d], and on the 16-bit
   // kernel dq_proj[t, h, d] = sum_f du[t, h, f] W_K[f, h, d] from the same du reads
-  const bool fused = wgrad16_supported(F) && dW_K != nullptr;
+  const bool fused = wgrad16_supported(F, true) && dW_K != nullptr;
   if (fused) {
     launch_wgrad16<T>(Wgrad{du, q_proj, w.wt, need_dq ? w.dq_proj : nullptr, dW_K, w.part, T_q,
                             w.ck.tchunk, w.ck.n, H, F, DH}, st);
@@ -542,12 +548,39 @@ void project_bwd(const void *q_raw, const void *W_Q, const void *W_K, const void
   if (dq_raw != nullptr)  // dq_raw [T, DQ] = dq_proj [T, HD] . W_Q [DQ, HD]^T
     launch_rowgemm<T>(RowGemm{w.dq_proj, W_Q, dq_raw, T_q, 1, DQ, HD, HD, 0, 0, HD, DQ, 0}, st);
   if (dW_Q != nullptr) {  // dW_Q[c, hd] = sum_t q_raw[t, c] dq_proj[t, hd]
-    if (wgrad16_supported(DQ))
+    if (wgrad16_supported(DQ, false))
       launch_wgrad16<T>(Wgrad{q_raw, w.dq_proj, nullptr, nullptr, dW_Q, w.part, T_q, w.cq.tchunk,
                               w.cq.n, 1, DQ, HD}, st);
     else
       launch_wgrad<T, T>(q_raw, w.dq_proj, w.part, dW_Q, T_q, w.cq.tchunk, w.cq.n, 1, DQ, HD, st);
   }
+}
+
+// The same products on fp32 operands (weights read in place).
+void project_fwd_f32(const void *q_raw, const void *W_Q, const void *W_K, void *q_proj, void *u,
+                     int64_t T_q, int H, int DQ, int F, int DH, hipStream_t st) {
+  const int HD = H * DH;
+  launch_rowgemm_f32(RowGemm{q_raw, W_Q, q_proj, T_q, 1, HD, DQ, DQ, 0, 0, HD, HD, 0}, true, st);
+  if (u != nullptr)
+    launch_rowgemm_f32(RowGemm{q_proj, W_K, u, T_q, H, F, DH, HD, DH, DH, HD, (int64_t)H * F, F},
+                       false, st);
+}
+
+void project_bwd_f32(const void *q_raw, const void *W_Q, const void *W_K, const void *q_proj,
+                     const void *du, void *dq_raw, void *dW_Q, void *dW_K, int64_t T_q, int H,
+                     int DQ, int F, int DH, const ProjectWs &w, hipStream_t st) {
+  const int HD = H * DH;
+  if (dW_K != nullptr)
+    launch_wgrad<float, float>(du, q_proj, w.part, dW_K, T_q, w.ck.tchunk, w.ck.n, H, F, DH, st);
+  if (dq_raw == nullptr && dW_Q == nullptr) return;
+  launch_rowgemm_f32(RowGemm{du, W_K, w.dq_proj, T_q, H, DH, F, (int64_t)H * F, F, DH, HD, HD, DH},
+                     true, st);
+  if (dq_raw != nullptr)
+    launch_rowgemm_f32(RowGemm{w.dq_proj, W_Q, dq_raw, T_q, 1, DQ, HD, HD, 0, 0, HD, DQ, 0},
+                       false, st);
+  if (dW_Q != nullptr)
+    launch_wgrad<float, float>(q_raw, w.dq_proj, w.part, dW_Q, T_q, w.cq.tchunk, w.cq.n, 1, DQ, HD,
+                               st);
 }
 
 }  // namespace
@@ -886,7 +919,7 @@ int vafa_absorb_project_u(const void *q_proj, const void *W_K, void *u, int64_t 
 int64_t vafa_absorb_project_workspace(int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV,
                                       int64_t D_H, int32_t backward) {
   if (check_project_dims("project_workspace", T_q, H, D_Q, D_KV, D_H) != VAFA_OK) return -1;
-  return carve_project(nullptr, T_q, H, D_Q, D_KV, D_H, backward != 0).bytes;
+  return carve_project(nullptr, T_q, H, D_Q, D_KV, D_H, backward != 0, false).bytes;
 }
 
 int vafa_absorb_project_fwd(const void *q_raw, const void *W_Q, const void *W_K, void *q_proj,
@@ -895,7 +928,7 @@ int vafa_absorb_project_fwd(const void *q_raw, const void *W_Q, const void *W_K,
                             void *stream) {
   if (int rc = check_project_dims("project_fwd", T_q, H, D_Q, D_KV, D_H)) return rc;
   if (int rc = check_aligned("project_fwd", {q_raw, W_Q, W_K, q_proj, u, workspace})) return rc;
-  const ProjectWs w = carve_project(workspace, T_q, H, D_Q, D_KV, D_H, false);
+  const ProjectWs w = carve_project(workspace, T_q, H, D_Q, D_KV, D_H, false, false);
   if (workspace_bytes < w.bytes || workspace == nullptr)
     return fail(VAFA_ERR_WORKSPACE, "project_fwd: workspace of %lld bytes, %lld needed",
                 (long long)workspace_bytes, (long long)w.bytes);
@@ -922,7 +955,7 @@ int vafa_absorb_project_bwd(const void *q_raw, const void *W_Q, const void *W_K,
   if (int rc = check_aligned("project_bwd", {q_raw, W_Q, W_K, q_proj, du, dq_raw, dW_Q, dW_K,
                                              workspace}))
     return rc;
-  const ProjectWs w = carve_project(workspace, T_q, H, D_Q, D_KV, D_H, true);
+  const ProjectWs w = carve_project(workspace, T_q, H, D_Q, D_KV, D_H, true, false);
   if (workspace_bytes < w.bytes || workspace == nullptr)
     return fail(VAFA_ERR_WORKSPACE, "project_bwd: workspace of %lld bytes, %lld needed",
                 (long long)workspace_bytes, (long long)w.bytes);
@@ -940,6 +973,40 @@ int vafa_absorb_project_bwd(const void *q_raw, const void *W_Q, const void *W_K,
       return fail(VAFA_ERR_VALUE, "project_bwd: 16-bit dtypes only (got %d)", (int)dtype);
   }
   return check_launch("vafa_absorb_project_bwd");
+}
+
+int64_t vafa_absorb_project_f32_workspace(int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV,
+                                          int64_t D_H) {
+  if (check_project_dims("project_f32_workspace", T_q, H, D_Q, D_KV, D_H, VAFA_F32)) return -1;
+  return carve_project(nullptr, T_q, H, D_Q, D_KV, D_H, true, true).bytes;
+}
+
+int vafa_absorb_project_f32_fwd(const float *q_raw, const float *W_Q, const float *W_K,
+                                float *q_proj, float *u, int64_t T_q, int64_t H, int64_t D_Q,
+                                int64_t D_KV, int64_t D_H, void *stream) {
+  if (int rc = check_project_dims("project_f32_fwd", T_q, H, D_Q, D_KV, D_H, VAFA_F32)) return rc;
+  if (int rc = check_aligned("project_f32_fwd", {q_raw, W_Q, W_K, q_proj, u})) return rc;
+  project_fwd_f32(q_raw, W_Q, W_K, q_proj, u, T_q, (int)H, (int)D_Q, (int)D_KV, (int)D_H,
+                  (hipStream_t)stream);
+  return check_launch("vafa_absorb_project_f32_fwd");
+}
+
+int vafa_absorb_project_f32_bwd(const float *q_raw, const float *W_Q, const float *W_K,
+                                const float *q_proj, const float *du, float *dq_raw, float *dW_Q,
+                                float *dW_K, int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV,
+                                int64_t D_H, void *workspace, int64_t workspace_bytes,
+                                void *stream) {
+  if (int rc = check_project_dims("project_f32_bwd", T_q, H, D_Q, D_KV, D_H, VAFA_F32)) return rc;
+  if (int rc = check_aligned("project_f32_bwd",
+                             {q_raw, W_Q, W_K, q_proj, du, dq_raw, dW_Q, dW_K, workspace}))
+    return rc;
+  const ProjectWs w = carve_project(workspace, T_q, H, D_Q, D_KV, D_H, true, true);
+  if (workspace_bytes < w.bytes || workspace == nullptr)
+    return fail(VAFA_ERR_WORKSPACE, "project_f32_bwd: workspace of %lld bytes, %lld needed",
+                (long long)workspace_bytes, (long long)w.bytes);
+  project_bwd_f32(q_raw, W_Q, W_K, q_proj, du, dq_raw, dW_Q, dW_K, T_q, (int)H, (int)D_Q,
+                  (int)D_KV, (int)D_H, w, (hipStream_t)stream);
+  return check_launch("vafa_absorb_project_f32_bwd");
 }
 
 int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O,

@@ -175,7 +175,7 @@ struct RowGemm {
 };
 bool rowgemm_supported(const RowGemm &);
 // Weight gradient out[f, g, d] = sum_t A[t, g, f] B[t, g, d] on 16-bit
-// matrix cores (A [T, G, F] with F <= 512, B [T, G, DH]): fp32 partials over
+// matrix cores (A [T, G, F], B [T, G, DH]): fp32 partials over
 // n_chunks chunks of tchunk tokens (a multiple of 32; part holds n_chunks * F
 // * G * DH floats) summed in chunk order into out.  With dq != nullptr also
 // dq[t, g, d] = sum_f A[t, g, f] Wt[g, d, f] (Wt [G, DH, F]), rounded once.
@@ -186,9 +186,13 @@ struct Wgrad {
   int64_t T_q, tchunk, n_chunks;
   int G, F, DH;
 };
-bool wgrad16_supported(int F);
+bool wgrad16_supported(int F, bool dq);
+int wgrad16_slices(int F);  // column slices of A, each a workgroup of its own
 template <typename T> void launch_wgrad16(const Wgrad &, hipStream_t);
 template <typename T> void launch_rowgemm(const RowGemm &, hipStream_t);
+// RowGemm on fp32 operands and fp32 matrix cores, any widths; kj: W is
+// [g, k, j] (W[g*ws + k*ldw + j])
+void launch_rowgemm_f32(const RowGemm &, bool kj, hipStream_t);
 // dst [C, R] = src [R, C]^T
 template <typename T> void launch_transpose2d(const void *src, void *dst, int R, int C, hipStream_t);
 // absorb_bwd_mfma.hip: du/aX (query side) and dX (key side) on matrix cores
