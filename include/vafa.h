@@ -136,6 +136,13 @@ typedef struct vafa_plan_info {
 VAFA_API int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
                      int64_t D, int32_t *plan, int64_t plan_cap, vafa_plan_info *info);
 
+/* The same plan format with tiles and key splits that also fill the GPU on
+ * launches of few or short segments (vafa_plan_varlen keeps the fixed rules
+ * above at every size); the plan packed_varlen_attn runs. */
+VAFA_API int vafa_plan_varlen_balanced(const int64_t *cu_q, const int64_t *cu_k, int64_t n1,
+                                       int64_t H, int64_t D, int32_t *plan, int64_t plan_cap,
+                                       vafa_plan_info *info);
+
 /* Plan for packed_target_attn (ta/interface.py:191-216, 265-314). */
 VAFA_API int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
                      int64_t D_KV, int64_t D_H, int32_t *plan, int64_t plan_cap,

@@ -202,6 +202,48 @@ def test_varlen_wide_tiles(device, case, D, dtype, dist):
             assert_close(name, a, r)
 
 
+# Small launches run the balanced plan (128-row and 128-key tiles, finer key
+# chunks); these run the fixed-rule plan of the same cases, whose tiles are the
+# ones large launches take (256 rows, at D = 128 256 keys), and a balanced plan
+# of many splits.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32],
+                         ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("case", range(len(WIDE_CASES)))
+def test_varlen_fixed_rule_plan(device, monkeypatch, case, D, dtype):
+    from collections import OrderedDict
+    from varlenabsorbflashattn_amd import _lib
+    plan_varlen, used = _lib.plan_varlen, []
+
+    def fixed(*a, balanced=False):
+        used.append(plan_varlen(*a))
+        return used[-1]
+
+    monkeypatch.setattr(_lib, "plan_varlen", fixed)
+    monkeypatch.setattr(_lib, "_CACHE", OrderedDict())
+    q_lens, k_lens = WIDE_CASES[case]
+    print(f"[varlen fixed-rule plan] q={q_lens} k={k_lens} D={D} {dtype}", flush=True)
+    got, ref = run_case(q_lens, k_lens, 4, D, dtype, device)
+    assert used and used[0].info.q_tile == 256
+    for name, a, r in zip(("o", "dq", "dk", "dv"), got, ref):
+        assert_close(name, a, r)
+
+
+@pytest.mark.parametrize("q_lens,k_lens,D", [
+    ([500, 130, 1], [8611, 513, 1200], 64), ([129], [2387], 256), ([16, 2, 9], [24000, 1024, 40], 128),
+])
+def test_varlen_balanced_splits(device, q_lens, k_lens, D):
+    from varlenabsorbflashattn_amd import _lib
+    cq, ck = cu_from_lens(q_lens).numpy(), cu_from_lens(k_lens).numpy()
+    fixed, bal = (_lib.plan_varlen(cq, ck, 2, D, b).info for b in (False, True))
+    assert bal.max_split > fixed.max_split
+    for dtype in (torch.bfloat16, torch.float32):
+        print(f"[varlen balanced] q={q_lens} k={k_lens} D={D} {dtype}", flush=True)
+        got, ref = run_case(q_lens, k_lens, 2, D, dtype, device)
+        for name, a, r in zip(("o", "dq", "dk", "dv"), got, ref):
+            assert_close(name, a, r)
+
+
 @pytest.mark.parametrize("H,q_lens,k_lens,D", [
     (3, [300, 5, 140], [200, 3000, 150], 64),     # 256-row tiles, item-major grid
     (5, [3, 16, 1, 9], [3000, 1500, 1024, 40], 128),  # decode-shaped: an item's heads on one XCD

@@ -176,9 +176,9 @@ def test_chunk_indices_real_shapes():
 
 # ---- plan invariants ------------------------------------------------------------
 
-def check_varlen_plan(q_lens, k_lens, H=4, D=64):
+def check_varlen_plan(q_lens, k_lens, H=4, D=64, balanced=False):
     cq, ck = _cu(q_lens), _cu(k_lens)
-    p = _lib.plan_varlen(cq, ck, H, D)
+    p = _lib.plan_varlen(cq, ck, H, D, balanced)
     fwd, comb, kv = p.section("fwd"), p.section("comb"), p.section("kv")
     BM = p.info.q_tile
     # 1) every (query row, key) pair of a segment is covered by exactly one item
@@ -566,3 +566,31 @@ def test_absorb_small_launch_chunks():
     for n, bk in ((192, 128), (193, 256)):
         p = _lib.plan_absorb(_cu([1] * n), _cu([1024] * n), 8, 256, 32)
         assert p.info.k_tile == bk
+
+
+def test_varlen_balanced_plan():
+    """The balanced plan keeps every invariant of the fixed-rule one, equals it
+    on launches that fill the GPU, and on small ones takes 128-row tiles and
+    chunks of at least 512 keys within the partial-row bound."""
+    from varlenabsorbflashattn_amd import workloads as W
+    cases = [([7, 11], [19, 5]), ([300, 20], [9000, 70000]), ([500] * 3, [8611, 300, 60000]),
+             ([0, 5, 0], [3, 0, 9]), ([16, 3], [32768, 1024]), ([2387], [2387]), ([1], [1]),
+             ([500] * 4, [102400] * 4)]
+    for ql, kl in cases:
+        for D in (16, 32, 64, 128, 256):
+            p = check_varlen_plan(ql, kl, H=2, D=D, balanced=True)
+            if max(kl) < 50000:  # (longer ones fill the GPU with key tiles)
+                assert p.info.q_tile == 128 and p.info.k_tile == 128
+            f = p.section("fwd")
+            split = f[f[:, 7] > 1]
+            last = split[:, 6] == split[:, 7] - 1
+            assert np.all((split[:, 3] - split[:, 2])[~last] >= 448)
+            if p.info.max_split > 16 and max(kl) <= 16 * 4096:
+                assert p.info.n_part_rows * 2 * (D + 1) * 4 <= 32 << 20
+    for c in (W.config2(0), W.config3(0)):
+        a, b = (_lib.plan_varlen(_cu(c.q_lens), _cu(c.k_lens), c.H, c.D, bal) for bal in (0, 1))
+        assert np.array_equal(a.items, b.items)
+    # a wide tile is kept only where the longest walk is within a CU's share
+    for n, tile in ((127, 128), (128, 256)):
+        p = _lib.plan_varlen(_cu([256] * n), _cu([256] * n), 2, 128, True)
+        assert (p.info.q_tile, p.info.k_tile) == (tile, tile)

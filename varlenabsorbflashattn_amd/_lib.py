@@ -61,6 +61,7 @@ _SIGS = {
     "vafa_check_active_have_keys": (C.c_int, [_PI64, _PI64, _I64]),
     "vafa_chunk_indices": (C.c_int, [_PI64, _I64, _I32, _PI32, _I64, _PI64]),
     "vafa_plan_varlen": (C.c_int, [_PI64, _PI64, _I64, _I64, _I64, _PI32, _I64, _PINFO]),
+    "vafa_plan_varlen_balanced": (C.c_int, [_PI64, _PI64, _I64, _I64, _I64, _PI32, _I64, _PINFO]),
     "vafa_plan_absorb": (C.c_int, [_PI64, _PI64, _I64, _I64, _I64, _I64, _PI32, _I64, _PINFO]),
     "vafa_varlen_fwd_workspace": (C.c_int64, [_PINFO, _I64]),
     "vafa_varlen_bwd_workspace": (C.c_int64, [_PINFO, _I64]),
@@ -239,14 +240,18 @@ def _plan(fn, guess: int, *args) -> HostPlan:
         n = info.plan_ints
 
 
-def plan_varlen(cu_q: np.ndarray, cu_k: np.ndarray, H: int, D: int) -> HostPlan:
+def plan_varlen(cu_q: np.ndarray, cu_k: np.ndarray, H: int, D: int,
+                balanced: bool = False) -> HostPlan:
+    """A varlen plan on the fixed rules, or balanced over the GPU's CUs (the
+    plan the operator runs)."""
     a = np.ascontiguousarray(cu_q, dtype=np.int64)
     b = np.ascontiguousarray(cu_k, dtype=np.int64)
     if a.shape != b.shape:
         raise AssertionError(f"segment count mismatch: q has {a.size - 1}, k has {b.size - 1}")
     # forward, dQ and dK/dV items of 128 tokens, a few splits of short queries
     guess = 64 + 12 * a.size + int(max(a[-1], 0) + max(b[-1], 0)) // 32 if a.size else 64
-    return _plan(lib().vafa_plan_varlen, guess, _i64p(a), _i64p(b), a.size, H, D)
+    fn = lib().vafa_plan_varlen_balanced if balanced else lib().vafa_plan_varlen
+    return _plan(fn, guess, _i64p(a), _i64p(b), a.size, H, D)
 
 
 def plan_absorb(cu_q: np.ndarray, cu_k: np.ndarray, H: int, F: int, DH: int) -> HostPlan:
@@ -287,7 +292,7 @@ def device_plan(kind: str, cu_q: np.ndarray, cu_k: np.ndarray, dims: tuple, devi
         if dp is not None:
             _CACHE.move_to_end(key)
     if dp is None:
-        host = (plan_varlen(cu_q, cu_k, *dims) if kind == "varlen"
+        host = (plan_varlen(cu_q, cu_k, *dims, balanced=True) if kind == "varlen"
                 else plan_absorb(cu_q, cu_k, *dims))
         dp = DevicePlan(host, device)
         with _lock:

@@ -113,6 +113,61 @@ void varlen_tiles(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t 
   *xcd_heads = work > 0.0 && 2.0 * long_q < work ? 1 : 0;
 }
 
+// Tiles and key splits that fill the chip on a launch too small for the fixed
+// rules (kVarlenBalance in plan_params.h): narrow tiles where the longest item
+// would outlast the average work per CU, and key chunks that follow the
+// average work per workgroup slot.
+void varlen_balance(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H, int64_t D,
+                    int64_t *bm, int64_t *bk, SplitPolicy *pol) {
+  const VarlenBalance &vb = kVarlenBalance;
+  // keys (queries) walked by all items of wide query (key) tiles, and the
+  // longest single walk
+  int64_t wide_q = 0, wide_k = 0, max_k = 0, max_q = 0;
+  for (int64_t s = 0; s + 1 < n1; ++s) {
+    const int64_t lq = cu_q[s + 1] - cu_q[s], lk = cu_k[s + 1] - cu_k[s];
+    if (lq == 0 || lk == 0) continue;
+    wide_q += cdiv(lq, kVarlenWideTile) * lk;
+    wide_k += cdiv(lk, kVarlenWideTile) * lq;
+    max_k = std::max(max_k, std::min(lk, pol->long_threshold));
+    max_q = std::max(max_q, lq);
+  }
+  if (*bm == kVarlenWideTile && wide_q * H < max_k * vb.cus) *bm = kVarlenTile;
+  if (*bk == kVarlenWideTile && wide_k * H < max_q * vb.cus) *bk = kVarlenTile;
+  if (*bm == kVarlenWideTile) return;
+  // items and their keys under the fixed rules, partial rows under a policy
+  auto count = [&](const SplitPolicy &p, int64_t *items, int64_t *keys) {
+    int64_t rows = 0;
+    for (int64_t s = 0; s + 1 < n1; ++s) {
+      const int64_t lq = cu_q[s + 1] - cu_q[s], lk = cu_k[s + 1] - cu_k[s];
+      for (int64_t t = 0; t < lq; t += kVarlenTile) {
+        const int64_t r = std::min<int64_t>(kVarlenTile, lq - t);
+        int64_t ns, chunk;
+        key_split(r, lk, p, &ns, &chunk);
+        if (ns > 1) rows += ns * r;
+        *items += ns;
+        *keys += lk;
+      }
+    }
+    return rows;
+  };
+  int64_t items = 0, keys = 0;
+  count(*pol, &items, &keys);
+  items *= H;
+  const int64_t slots = (D > 128 ? 1 : 2) * vb.cus;  // resident workgroups
+  if (items >= 2 * slots) return;
+  const int64_t avg = cdiv(keys * H, slots);
+  auto chunk_of = [&](int64_t keys, int64_t most) {
+    return std::min(most, std::max(round_up(keys, pol->align), vb.min_chunk));
+  };
+  SplitPolicy p = *pol;
+  if (items * 5 < slots * (D > 128 ? 4 : 3))
+    p.long_chunk = p.long_threshold = chunk_of(avg * 3 / 2, p.long_threshold);
+  p.decode_chunk = chunk_of(avg / 2, p.decode_chunk);
+  if (p.decode_chunk * 2 <= pol->decode_chunk) p.decode_max_split *= 2;
+  const int64_t rows = count(p, &items, &keys);
+  if (rows * H * (D + 1) * 4 <= vb.max_part_bytes) *pol = p;
+}
+
 // Indices of `cost` in descending order, equal costs in index order: a
 // radix sort (a launch of thousands of samples sorts up to 100k items).
 std::vector<uint32_t> order_lpt(const std::vector<int64_t> &cost) {
@@ -337,13 +392,14 @@ int vafa_chunk_indices(const int64_t *cu, int64_t n1, int32_t BT, int32_t *out, 
 //   fcomb section : one item per fused segment, {q0, q1, pbase, nchunks, seg,
 //                   0, 0, 0}: chunk t of the segment owns rows
 //                   pbase + t*(q1-q0) + r (the comb layout), summed in order.
-int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H, int64_t D,
-                     int32_t *plan, int64_t plan_cap, vafa_plan_info *info) {
+static int plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H, int64_t D,
+                       bool balance, int32_t *plan, int64_t plan_cap, vafa_plan_info *info) {
   int rc = check_pair(cu_q, cu_k, n1);
   if (rc) return rc;
-  const SplitPolicy &pol = kVarlenPolicy;
+  SplitPolicy pol = kVarlenPolicy;
   int64_t BM = kVarlenTile, BK = kVarlenTile, xcd_heads = 0;
   varlen_tiles(cu_q, cu_k, n1, D, &BM, &BK, &xcd_heads);
+  if (balance) varlen_balance(cu_q, cu_k, n1, H, D, &BM, &BK, &pol);
   std::memset(info, 0, sizeof(*info));
   info->magic = VAFA_PLAN_MAGIC;
   info->kind = 1;
@@ -419,6 +475,16 @@ int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   info->n_fpart_rows = fprow;
   info->max_split = max_split;
   return emit(fwd, comb, kv, {}, dq, dqc, fkv, fcomb, plan, plan_cap, info);
+}
+
+int vafa_plan_varlen(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H, int64_t D,
+                     int32_t *plan, int64_t plan_cap, vafa_plan_info *info) {
+  return plan_varlen(cu_q, cu_k, n1, H, D, false, plan, plan_cap, info);
+}
+
+int vafa_plan_varlen_balanced(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
+                              int64_t D, int32_t *plan, int64_t plan_cap, vafa_plan_info *info) {
+  return plan_varlen(cu_q, cu_k, n1, H, D, true, plan, plan_cap, info);
 }
 
 // Absorb plan.  Query rows are (token, head) pairs; one item covers whole

@@ -36,6 +36,25 @@ struct SplitPolicy {
 };
 
 constexpr SplitPolicy kVarlenPolicy{16, 1024, 2048, 4, 16, 4096, 4096, 64, 64};
+// vafa_plan_varlen_balanced: launches whose items cannot fill `cus` CUs evenly.
+// 256-row (256-key) tiles become 128 where the longest walk exceeds a CU's
+// share of the work.  Below 3/5 item per resident 128-row workgroup (two per
+// CU; 4/5 at D = 256, one per CU) key ranges split beyond 3/2 of the average
+// keys per workgroup, below two items each decode tiles into chunks of half of
+// it (up to twice the splits); never below min_chunk keys, and only while the
+// fp32 partial rows stay within max_part_bytes.  GPU time, us, fixed rules ->
+// balanced (self-attention lengths log-uniform in [1, 4096] unless stated, H =
+// heads): 16 sequences D = 128 H = 4 forward + backward 262 -> 215, 8 sequences
+// H = 16 227 -> 206, 16 sequences D = 256 H = 2 402 -> 341, fp32 D = 64 32
+// sequences of <= 2048 H = 8 1148 -> 990 and H = 2 967 -> 505; 500 queries
+// against 3 histories of <= 8611 keys 157 -> 77; decode of 4 x 24k keys H = 4
+// 49 -> 33.  On launches that fill the chip the same splits lose: 64 sequences
+// D = 128 H = 16 2071 -> 2289 with 2048-key chunks, 8 sequences 215 -> 270 with
+// 1024.
+struct VarlenBalance {
+  int64_t cus, min_chunk, max_part_bytes;
+};
+constexpr VarlenBalance kVarlenBalance{256, 512, 32 << 20};
 // Absorb forward key splits.  A chunk holds kAbsorbSlack2 / 2 times the
 // average keys per resident forward workgroup (256 CUs x 3 on the MI355X), so
 // large launches stay whole (splitting C5's <= 8192-key samples into 1024-key
