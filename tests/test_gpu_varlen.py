@@ -523,3 +523,39 @@ def test_varlen_business_scale(device):
         e = _gpu_errors(a, r)
         report(name, e, torch.bfloat16)
         check(name, e, torch.bfloat16)
+
+
+def test_cached_plan_keeps_the_checks(device):
+    """A call whose plan is cached (by the content of cu_seqlens, int32 or int64,
+    device or host) still raises what a first call raises: another token count,
+    and in the absorb operator a segment with queries but no keys."""
+    from varlenabsorbflashattn_amd import target_attn_inner
+    cu = torch.tensor([0, 4, 10], dtype=torch.int32)
+    mk = lambda *s: torch.randn(*s, device=device, dtype=torch.bfloat16)
+    x, y = mk(10, 2, 64), mk(12, 2, 64)
+    outs = [packed_varlen_attn(x, x, x, cu_seqlens_q=c, cu_seqlens_k=c)
+            for c in (cu, cu.to(device), cu.long(), cu.long().to(device)) for _ in range(2)]
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    for c in (cu, cu.to(device)):
+        with pytest.raises(ValueError, match=r"cu_seqlens_q\[-1\] must equal total tokens 12"):
+            packed_varlen_attn(y, y, y, cu_seqlens_q=c, cu_seqlens_k=c)
+    cq, ck = (torch.tensor(c, dtype=torch.int32, device=device) for c in ([0, 2, 5], [0, 7, 7]))
+    args = (mk(5, 8, 64), mk(7, 64), mk(64, 8, 32), cq, ck)
+    for _ in range(2):
+        target_attn_inner(*args, validate=False)
+        with pytest.raises(ValueError, match="must have k_len > 0"):
+            target_attn_inner(*args)
+
+
+def test_host_module_maps_errors(device):
+    """Status codes of the C ABI reach Python as the reference's error types."""
+    import numpy as np
+    from varlenabsorbflashattn_amd import _lib
+    x = torch.zeros(300, 2, 64, device=device, dtype=torch.bfloat16)
+    wide = _lib.DevicePlan(_lib.plan_varlen(np.array([0, 300]), np.array([0, 300]), 2, 128), device)
+    with pytest.raises(ValueError, match="build the plan with this head_dim"):
+        _lib.ops().varlen_fwd(x, x, x, wide.native, 1.0)
+    with pytest.raises(AssertionError, match="head_dim 48"):
+        _lib.ops().varlen_fwd(*(x[:, :, :48].contiguous() for _ in range(3)), wide.native, 1.0)
+    with pytest.raises(AssertionError, match="dtype"):
+        _lib.ops().varlen_fwd(*(x.double() for _ in range(3)), wide.native, 1.0)

@@ -26,6 +26,8 @@ VAFA_ERR_WORKSPACE = -4
 VAFA_ERR_CAPACITY = -5
 
 DT_F32, DT_F16, DT_BF16 = 0, 1, 2
+# the host module that allocates and launches (csrc/torch_ops.cpp)
+TORCH_LIB_PATH = os.path.join(_HERE, "_vafa_torch.so")
 # bytes of the static per-GPU scratch of vafa_varlen_fwd_noalloc
 # (VAFA_NOALLOC_SCRATCH_BYTES in include/vafa.h)
 NOALLOC_SCRATCH_BYTES = 64 << 20
@@ -122,6 +124,30 @@ def lib():
                 fn.argtypes = args
             _lib = h
     return _lib
+
+
+_ops = None
+
+
+def ops():
+    """Load (once) and return the host module _vafa_torch.so, bound to LIB_PATH."""
+    global _ops
+    if _ops is not None:
+        return _ops
+    lib()
+    with _lock:
+        if _ops is None:
+            if not os.path.exists(TORCH_LIB_PATH):
+                raise RuntimeError(
+                    f"{TORCH_LIB_PATH} is missing: build it with "
+                    "`python -m varlenabsorbflashattn_amd.build`")
+            import importlib.util
+            spec = importlib.util.spec_from_file_location("_vafa_torch", TORCH_LIB_PATH)
+            m = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(m)
+            m.bind(LIB_PATH)
+            _ops = m
+    return _ops
 
 
 def last_error() -> str:
@@ -267,41 +293,88 @@ def plan_absorb(cu_q: np.ndarray, cu_k: np.ndarray, H: int, F: int, DH: int) -> 
 # ---- device plans (cached by cu_seqlens content) ------------------------------
 
 class DevicePlan:
+    """A plan on the device.  ``native`` is the handle the host module takes;
+    ``keys_ok`` remembers that every segment with queries has keys (a property
+    of the cu_seqlens the plan was built from)."""
+
     def __init__(self, host: HostPlan, device):
         import torch
         self.host = host
         self.info = host.info
+        self.T_q, self.T_k = int(host.info.T_q), int(host.info.T_k)
+        self.keys_ok = False
         t = torch.from_numpy(host.items)
         if host.items.size == 0:
             t = torch.zeros(ITEM_INTS, dtype=torch.int32)
         self.items = t.to(device, non_blocking=False)
+        self.native = ops().Plan(self.items, bytes(host.info)) if self.items.is_cuda else None
+
+    def use(self) -> "DevicePlan":
+        """Marks the plan as in use on the current stream: evicted from the cache
+        while a kernel on another stream still reads it, it keeps its memory
+        until that stream's work is done."""
+        if self.items.is_cuda:
+            import torch
+            self.items.record_stream(torch.cuda.current_stream(self.items.device))
+        return self
 
 
 _CACHE: "OrderedDict[tuple, DevicePlan]" = OrderedDict()
 _CACHE_MAX = 64
 
 
-def device_plan(kind: str, cu_q: np.ndarray, cu_k: np.ndarray, dims: tuple, device) -> DevicePlan:
-    """The cached device plan for these cu_seqlens, marked as in use on the
-    current stream: a plan evicted from the cache while a kernel on another
-    stream still reads it keeps its memory until that stream's work is done."""
+def host_cu_pair(a, b) -> Tuple[np.ndarray, np.ndarray]:
+    """Host copies of two cu_seqlens tensors in their own dtype, with one device
+    sync where as_host_i64_pair takes one."""
     import torch
-    key = (kind, cu_q.tobytes(), cu_k.tobytes(), dims, str(device))
+    if (a.is_floating_point() or a.is_complex() or b.is_floating_point() or b.is_complex()):
+        return as_host_i64_pair(a, b)
+    if a is b:
+        h = a.detach().cpu().numpy()
+        return h, h
+    if (a.is_cuda and b.is_cuda and a.device == b.device and a.dtype == b.dtype
+            and a.shape == b.shape and a.dim() == 1):
+        h = torch.stack((a.detach(), b.detach())).cpu().numpy()
+        return h[0], h[1]
+    return a.detach().cpu().numpy(), b.detach().cpu().numpy()
+
+
+def plan_key(kind: str, cu_q: np.ndarray, cu_k: np.ndarray, dims: tuple, device) -> tuple:
+    return (kind, cu_q.dtype.char, cu_k.dtype.char, cu_q.tobytes(), cu_k.tobytes(), dims, device)
+
+
+def cached_plan(key: tuple) -> Optional[DevicePlan]:
+    """The cached plan of these cu_seqlens (any integer dtype; by content), or
+    None.  A cached plan was built from them, so they start at 0, do not decrease
+    and end at its T_q / T_k."""
     with _lock:
         dp = _CACHE.get(key)
         if dp is not None:
             _CACHE.move_to_end(key)
-    if dp is None:
-        host = (plan_varlen(cu_q, cu_k, *dims, balanced=True) if kind == "varlen"
-                else plan_absorb(cu_q, cu_k, *dims))
-        dp = DevicePlan(host, device)
-        with _lock:
-            _CACHE[key] = dp
-            while len(_CACHE) > _CACHE_MAX:
-                _CACHE.popitem(last=False)
-    if dp.items.is_cuda:
-        dp.items.record_stream(torch.cuda.current_stream(dp.items.device))
     return dp
+
+
+def new_plan(key: tuple, cu_q: np.ndarray, cu_k: np.ndarray) -> DevicePlan:
+    """Builds and caches the plan of ``key``, from int64 cu_seqlens."""
+    kind, dims, device = key[0], key[5], key[6]
+    host = (plan_varlen(cu_q, cu_k, *dims, balanced=True) if kind == "varlen"
+            else plan_absorb(cu_q, cu_k, *dims))
+    dp = DevicePlan(host, device)
+    with _lock:
+        _CACHE[key] = dp
+        while len(_CACHE) > _CACHE_MAX:
+            _CACHE.popitem(last=False)
+    return dp
+
+
+def device_plan(kind: str, cu_q: np.ndarray, cu_k: np.ndarray, dims: tuple, device) -> DevicePlan:
+    """The cached device plan for these cu_seqlens, marked as in use on the
+    current stream."""
+    key = plan_key(kind, cu_q, cu_k, dims, device)
+    dp = cached_plan(key)
+    if dp is None:
+        dp = new_plan(key, as_host_i64(cu_q), as_host_i64(cu_k))
+    return dp.use()
 
 
 def dtype_code(dtype) -> int:

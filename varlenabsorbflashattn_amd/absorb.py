@@ -14,6 +14,7 @@ is deterministic (dW_V and dX are reduced in a fixed order).
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 import weakref
@@ -126,10 +127,6 @@ def prepare_target_attn_indices(cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.
     return q_idx, k_idx
 
 
-def _workspace(nbytes: int, device) -> torch.Tensor:
-    return torch.empty(max(int(nbytes), 0), dtype=torch.uint8, device=device)
-
-
 def _aligned(x: torch.Tensor) -> torch.Tensor:
     return x.clone() if x.data_ptr() % 16 != 0 else x
 
@@ -141,50 +138,36 @@ def _absorb_plan(T_q, T_k, H, D_KV, D_H, device, cu_seqlens_q, cu_seqlens_k,
     when they belong to these very tensors and validation is off."""
     known = _recall_host_cu(q_chunk_indices, cu_seqlens_q, cu_seqlens_k)
     if known is not None and not validate:
-        cu_q_h, cu_k_h = known
+        cu_q, cu_k = known
     else:
-        cu_q_h, cu_k_h = _lib.as_host_i64_pair(cu_seqlens_q, cu_seqlens_k)
-    if validate:
-        n_seg = cu_seqlens_q.numel() - 1
-        assert cu_seqlens_k.numel() - 1 == n_seg, "segment count mismatch q vs k"
-        _validate_cu_seqlens(cu_q_h, cu_seqlens_q.shape, T_q, "cu_seqlens_q")
-        _validate_cu_seqlens(cu_k_h, cu_seqlens_k.shape, T_k, "cu_seqlens_k")
-        _lib.check_active_have_keys(cu_q_h, cu_k_h)
-    B_DKV = _next_power_of_2(D_KV)
-    assert B_DKV <= 512, f"D_KV={D_KV} pads to {B_DKV}, which is too large for v1 tiles"
-    plan = _lib.device_plan("absorb", cu_q_h, cu_k_h, (H, D_KV, D_H), device)
-    if plan.info.T_q > T_q or plan.info.T_k > T_k:
+        cu_q, cu_k = _lib.host_cu_pair(cu_seqlens_q, cu_seqlens_k)
+    # the checks depend on the content and the token counts alone: a cached
+    # plan of the same content that covers exactly these tokens passed them
+    # (keys_ok: including the last one)
+    key = _lib.plan_key("absorb", cu_q, cu_k, (H, D_KV, D_H), device)
+    plan = _lib.cached_plan(key) if cu_q.ndim == 1 and cu_k.ndim == 1 else None
+    known_ok = (plan is not None and plan.T_q == T_q and plan.T_k == T_k
+                and (plan.keys_ok or not validate))
+    if not known_ok:
+        cu_q_h, cu_k_h = _lib.as_host_i64(cu_q), _lib.as_host_i64(cu_k)
+        if validate:
+            n_seg = cu_seqlens_q.numel() - 1
+            assert cu_seqlens_k.numel() - 1 == n_seg, "segment count mismatch q vs k"
+            _validate_cu_seqlens(cu_q_h, cu_seqlens_q.shape, T_q, "cu_seqlens_q")
+            _validate_cu_seqlens(cu_k_h, cu_seqlens_k.shape, T_k, "cu_seqlens_k")
+            _lib.check_active_have_keys(cu_q_h, cu_k_h)
+        B_DKV = _next_power_of_2(D_KV)
+        assert B_DKV <= 512, f"D_KV={D_KV} pads to {B_DKV}, which is too large for v1 tiles"
+        if plan is None:
+            plan = _lib.new_plan(key, cu_q_h, cu_k_h)
+        plan.keys_ok = plan.keys_ok or bool(validate)
+    if plan.T_q > T_q or plan.T_k > T_k:
         raise ValueError(
             f"cu_seqlens address {plan.info.T_q} query / {plan.info.T_k} key tokens but "
             f"the inputs hold {T_q} / {T_k}")
     if plan.info.n_fwd > 0:
         _select_fwd_mode()
-    return plan
-
-
-def _absorb_bwd(u, X, W_V, O, LSE, dO, plan, scale):
-    """du, dX, dW_V of the inner op through vafa_absorb_bwd."""
-    T_q, H, D_KV = u.shape
-    D_H = W_V.shape[2]
-    if dO.stride(-1) != 1 or not dO.is_contiguous():
-        dO = dO.contiguous()
-    if dO.dtype != u.dtype:
-        dO = dO.to(u.dtype)
-    dO = _aligned(dO)
-    if plan.info.n_kv > 0:
-        _select_dx_mode(int(plan.info.n_kv))
-    du = torch.empty_like(u)
-    dX = torch.empty_like(X)
-    dW_V = torch.empty_like(W_V)
-    L = _lib.lib()
-    ws = _workspace(L.vafa_absorb_bwd_workspace(plan.info, D_KV, D_H), u.device)
-    _lib.check(L.vafa_absorb_bwd(
-        u.data_ptr(), X.data_ptr(), W_V.data_ptr(), O.data_ptr(), dO.data_ptr(),
-        LSE.data_ptr(), du.data_ptr(), dX.data_ptr(), dW_V.data_ptr(),
-        plan.items.data_ptr(), plan.info, D_KV, D_H, _lib.dtype_code(u.dtype),
-        float(scale), ws.data_ptr() if ws.numel() else None, ws.numel(),
-        _lib.stream_ptr(u.device)))
-    return du, dX, dW_V
+    return plan.use()
 
 
 class _TargetAttnFunction(torch.autograd.Function):
@@ -204,18 +187,11 @@ class _TargetAttnFunction(torch.autograd.Function):
         assert u.is_cuda and X.is_cuda and W_V.is_cuda, "all inputs must be CUDA"
         assert u.device == X.device == W_V.device, "u/X/W_V must be on same device"
         assert D_H in (16, 32, 64, 128, 256), f"D_H {D_H} not supported"
-        dcode = _lib.dtype_code(u.dtype)
+        _lib.dtype_code(u.dtype)
         u, X, W_V = (_aligned(t.contiguous()) for t in (u, X, W_V))
         plan = _absorb_plan(T_q, T_k, H, D_KV, D_H, u.device, cu_seqlens_q, cu_seqlens_k,
                             q_chunk_indices, validate)
-        O = torch.empty((T_q, H, D_H), dtype=u.dtype, device=u.device)
-        LSE = torch.empty((T_q, H), dtype=torch.float32, device=u.device)
-        L = _lib.lib()
-        ws = _workspace(L.vafa_absorb_fwd_workspace(plan.info, D_KV, D_H), u.device)
-        _lib.check(L.vafa_absorb_fwd(
-            u.data_ptr(), X.data_ptr(), W_V.data_ptr(), O.data_ptr(), LSE.data_ptr(),
-            plan.items.data_ptr(), plan.info, D_KV, D_H, dcode, float(scale),
-            ws.data_ptr() if ws.numel() else None, ws.numel(), _lib.stream_ptr(u.device)))
+        O, LSE = _lib.ops().absorb_fwd(u, X, W_V, plan.native, scale)
         ctx.save_for_backward(u, X, W_V, O, LSE)
         ctx.plan = plan
         ctx.scale = scale
@@ -224,8 +200,10 @@ class _TargetAttnFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dO):
         u, X, W_V, O, LSE = ctx.saved_tensors
-        du, dX, dW_V = _absorb_bwd(u, X, W_V, O, LSE, dO, ctx.plan, ctx.scale)
-        return du, dX, dW_V, None, None, None, None, None, None
+        if ctx.plan.info.n_kv > 0:
+            _select_dx_mode(int(ctx.plan.info.n_kv))
+        return *_lib.ops().absorb_bwd(u, X, W_V, O, LSE, dO, ctx.plan.native, ctx.scale), \
+            None, None, None, None, None, None
 
 
 def target_attn_inner(
@@ -275,51 +253,19 @@ class _Project(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -> torch.Tensor:
-        T_q, d_q = q_raw.shape
-        _, H, D_H = W_Q.shape
-        d_kv = W_K.shape[0]
-        L = _lib.lib()
-        q_raw = _aligned(q_raw.contiguous())
-        W_Q = _aligned(W_Q.contiguous())
-        W_K = _aligned(W_K.contiguous())
-        q_proj = torch.empty((T_q, H * D_H), dtype=q_raw.dtype, device=q_raw.device)
-        u = torch.empty((T_q, H, d_kv), dtype=q_raw.dtype, device=q_raw.device)
-        args = (q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), u.data_ptr(),
-                T_q, H, d_q, d_kv, D_H)
-        st = _lib.stream_ptr(q_raw.device)
-        if q_raw.dtype == torch.float32:
-            _lib.check(L.vafa_absorb_project_f32_fwd(*args, st))
-        else:
-            ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 0),
-                            q_raw.device)
-            _lib.check(L.vafa_absorb_project_fwd(*args, _lib.dtype_code(q_raw.dtype),
-                                                 ws.data_ptr(), ws.numel(), st))
+        q_raw, W_Q, W_K = (_aligned(t.contiguous()) for t in (q_raw, W_Q, W_K))
+        q_proj, u = _lib.ops().project_fwd(q_raw, W_Q, W_K)
         ctx.save_for_backward(q_raw, W_Q, W_K, q_proj)
         return u
 
     @staticmethod
     def backward(ctx, du: torch.Tensor):
-        q_raw, W_Q, W_K, q_proj = ctx.saved_tensors
-        T_q, d_q = q_raw.shape
-        d_kv, H, D_H = W_K.shape
-        need_q, need_wq, need_wk = ctx.needs_input_grad[:3]
-        du = _aligned(du.contiguous())
-        dq = torch.empty_like(q_raw) if need_q else None
-        dwq = torch.empty_like(W_Q) if need_wq else None
-        dwk = torch.empty_like(W_K) if need_wk else None
-        L = _lib.lib()
-        args = (q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(), du.data_ptr(),
-                _lib.ptr(dq), _lib.ptr(dwq), _lib.ptr(dwk), T_q, H, d_q, d_kv, D_H)
-        st = _lib.stream_ptr(du.device)
-        if du.dtype == torch.float32:
-            ws = _workspace(L.vafa_absorb_project_f32_workspace(T_q, H, d_q, d_kv, D_H),
-                            du.device)
-            _lib.check(L.vafa_absorb_project_f32_bwd(*args, ws.data_ptr(), ws.numel(), st))
-        else:
-            ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 1), du.device)
-            _lib.check(L.vafa_absorb_project_bwd(*args, _lib.dtype_code(du.dtype), ws.data_ptr(),
-                                                 ws.numel(), st))
-        return dq, dwq, dwk
+        return _lib.ops().project_bwd(*ctx.saved_tensors, du, *ctx.needs_input_grad[:3])
+
+
+@functools.lru_cache(maxsize=256)
+def _fold_shape(H: int, d_kv: int, D_H: int, dtype: torch.dtype) -> bool:
+    return bool(_lib.lib().vafa_absorb_fold_supported(H, d_kv, D_H, _lib.dtype_code(dtype)))
 
 
 def _fold_native(q_raw, X, W_Q, W_K, W_V) -> bool:
@@ -334,8 +280,7 @@ def _fold_native(q_raw, X, W_Q, W_K, W_V) -> bool:
     if not (q_raw.device == X.device == W_Q.device == W_K.device == W_V.device):
         return False
     d_kv, H, D_H = W_K.shape
-    return bool(_lib.lib().vafa_absorb_fold_supported(H, d_kv, D_H,
-                                                      _lib.dtype_code(q_raw.dtype)))
+    return _fold_shape(H, d_kv, D_H, q_raw.dtype)
 
 
 class _FoldedTargetAttn(torch.autograd.Function):
@@ -353,23 +298,12 @@ class _FoldedTargetAttn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q_raw, X, W_Q, W_K, W_V, cu_seqlens_q, cu_seqlens_k, scale,
                 q_chunk_indices, k_chunk_indices, validate):
-        T_q, d_q = q_raw.shape
         T_k, d_kv = X.shape
         _, H, D_H = W_Q.shape
-        dcode = _lib.dtype_code(q_raw.dtype)
         q_raw, X, W_Q, W_K, W_V = (_aligned(t.contiguous()) for t in (q_raw, X, W_Q, W_K, W_V))
-        plan = _absorb_plan(T_q, T_k, H, d_kv, D_H, X.device, cu_seqlens_q, cu_seqlens_k,
-                            q_chunk_indices, validate)
-        L = _lib.lib()
-        st = _lib.stream_ptr(X.device)
-        q_proj = torch.empty((T_q, H * D_H), dtype=q_raw.dtype, device=q_raw.device)
-        O = torch.empty((T_q, H, D_H), dtype=q_raw.dtype, device=X.device)
-        LSE = torch.empty((T_q, H), dtype=torch.float32, device=X.device)
-        ws = _workspace(L.vafa_absorb_fwd_full_workspace(plan.info, d_q, d_kv, D_H), X.device)
-        _lib.check(L.vafa_absorb_fwd_full(
-            q_raw.data_ptr(), X.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), W_V.data_ptr(),
-            q_proj.data_ptr(), O.data_ptr(), LSE.data_ptr(), T_q, plan.items.data_ptr(),
-            plan.info, d_q, d_kv, D_H, dcode, float(scale), ws.data_ptr(), ws.numel(), st))
+        plan = _absorb_plan(q_raw.shape[0], T_k, H, d_kv, D_H, X.device, cu_seqlens_q,
+                            cu_seqlens_k, q_chunk_indices, validate)
+        q_proj, O, LSE = _lib.ops().absorb_full_fwd(q_raw, X, W_Q, W_K, W_V, plan.native, scale)
         ctx.save_for_backward(q_raw, W_Q, W_K, q_proj, X, W_V, O, LSE)
         ctx.plan = plan
         ctx.scale = scale
@@ -377,26 +311,12 @@ class _FoldedTargetAttn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dO):
-        q_raw, W_Q, W_K, q_proj, X, W_V, O, LSE = ctx.saved_tensors
-        T_q, d_q = q_raw.shape
-        d_kv, H, D_H = W_K.shape
-        L = _lib.lib()
-        st = _lib.stream_ptr(X.device)
-        u = torch.empty((T_q, H, d_kv), dtype=q_raw.dtype, device=X.device)
-        _lib.check(L.vafa_absorb_project_u(q_proj.data_ptr(), W_K.data_ptr(), u.data_ptr(), T_q,
-                                           H, d_kv, D_H, _lib.dtype_code(u.dtype), st))
-        du, dX, dW_V = _absorb_bwd(u, X, W_V, O, LSE, dO, ctx.plan, ctx.scale)
+        if ctx.plan.info.n_kv > 0:
+            _select_dx_mode(int(ctx.plan.info.n_kv))
         need_q, _, need_wq, need_wk = ctx.needs_input_grad[:4]
-        dq = torch.empty_like(q_raw) if need_q else None
-        dwq = torch.empty_like(W_Q) if need_wq else None
-        dwk = torch.empty_like(W_K) if need_wk else None
-        if need_q or need_wq or need_wk:
-            ws = _workspace(L.vafa_absorb_project_workspace(T_q, H, d_q, d_kv, D_H, 1), X.device)
-            _lib.check(L.vafa_absorb_project_bwd(
-                q_raw.data_ptr(), W_Q.data_ptr(), W_K.data_ptr(), q_proj.data_ptr(),
-                du.data_ptr(), _lib.ptr(dq), _lib.ptr(dwq), _lib.ptr(dwk), T_q, H, d_q, d_kv,
-                D_H, _lib.dtype_code(du.dtype), ws.data_ptr(), ws.numel(), st))
-        return dq, dX, dwq, dwk, dW_V, None, None, None, None, None, None
+        return *_lib.ops().absorb_full_bwd(*ctx.saved_tensors, dO, ctx.plan.native, ctx.scale,
+                                           need_q, need_wq, need_wk), \
+            None, None, None, None, None, None
 
 
 def _project_u(q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -> torch.Tensor:

@@ -82,6 +82,29 @@ def _check_tokens(info, T_q: int, T_k: int) -> None:
             f"hold {T_q} / {T_k}")
 
 
+def _plan_of(q, k, cu_seqlens_q, cu_seqlens_k):
+    """Validation (fa/interface.py:96-118, 158-175) and the device plan.  The
+    checks of cu_seqlens depend on their content and the token counts alone:
+    a cached plan of the same content that covers exactly these tokens passed
+    them when it was built."""
+    T_q, H, D = q.shape
+    T_k = k.shape[0]
+    cu_q, cu_k = _lib.host_cu_pair(cu_seqlens_q, cu_seqlens_k)
+    key = _lib.plan_key("varlen", cu_q, cu_k, (H, D), q.device)
+    plan = _lib.cached_plan(key) if cu_q.ndim == 1 and cu_k.ndim == 1 else None
+    if plan is not None and plan.T_q == T_q and plan.T_k == T_k:
+        return plan.use()
+    cu_q_h, cu_k_h = _lib.as_host_i64(cu_q), _lib.as_host_i64(cu_k)
+    _validate_cu_seqlens(cu_q_h, cu_seqlens_q.shape, T_q, "cu_seqlens_q")
+    _validate_cu_seqlens(cu_k_h, cu_seqlens_k.shape, T_k, "cu_seqlens_k")
+    if cu_q_h.ndim != 1 or cu_q_h.size < 2:
+        raise ValueError("cu_seqlens_q: must be 1-D with at least 2 elements")
+    if plan is None:
+        plan = _lib.new_plan(key, cu_q_h, cu_k_h)
+    _check_tokens(plan.info, T_q, T_k)
+    return plan.use()
+
+
 class _PackedVarlenAttnFunction(torch.autograd.Function):
     """Autograd wrapper (fa/interface.py:153-341)."""
 
@@ -96,7 +119,7 @@ class _PackedVarlenAttnFunction(torch.autograd.Function):
         assert q.is_cuda, "packed_varlen_attn requires GPU tensors"
         assert k.device == q.device and v.device == q.device, "q/k/v must be on the same device"
         assert D in (16, 32, 64, 128, 256), f"head_dim {D} not supported (try 64/128/256)"
-        dcode = _lib.dtype_code(q.dtype)
+        _lib.dtype_code(q.dtype)
 
         n_seg = cu_seqlens_q.numel() - 1
         assert cu_seqlens_k.numel() - 1 == n_seg, \
@@ -105,22 +128,9 @@ class _PackedVarlenAttnFunction(torch.autograd.Function):
         # copy waits for the GPU work already queued, and what follows it runs
         # while the GPU is idle
         q, k, v = _aligned(q), _aligned(k), _aligned(v)
-        o = torch.empty_like(q)
-        lse = torch.empty((T_q, H), dtype=torch.float32, device=q.device)
-        L = _lib.lib()
-        cu_q_h, cu_k_h = _lib.as_host_i64_pair(cu_seqlens_q, cu_seqlens_k)
-        _validate_cu_seqlens(cu_q_h, cu_seqlens_q.shape, T_q, "cu_seqlens_q")
-        _validate_cu_seqlens(cu_k_h, cu_seqlens_k.shape, T_k, "cu_seqlens_k")
-        if cu_q_h.ndim != 1 or cu_q_h.size < 2:
-            raise ValueError("cu_seqlens_q: must be 1-D with at least 2 elements")
-
-        plan = _lib.device_plan("varlen", cu_q_h, cu_k_h, (H, D), q.device)
-        _check_tokens(plan.info, T_q, T_k)
-        ws = _workspace(L.vafa_varlen_fwd_workspace(plan.info, D), q.device)
-        _lib.check(L.vafa_varlen_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-            plan.items.data_ptr(), plan.info, D, dcode, float(scale),
-            ws.data_ptr() if ws.numel() else None, ws.numel(), _lib.stream_ptr(q.device)))
+        ops = _lib.ops()
+        plan = _plan_of(q, k, cu_seqlens_q, cu_seqlens_k)
+        o, lse = ops.varlen_fwd(q, k, v, plan.native, scale)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.plan = plan
         ctx.scale = scale
@@ -129,24 +139,8 @@ class _PackedVarlenAttnFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        plan = ctx.plan
-        T_q, H, D = q.shape
-        if do.stride(-1) != 1 or not do.is_contiguous():
-            do = do.contiguous()
-        if do.dtype != q.dtype:
-            do = do.to(q.dtype)
-        do = _aligned(do)
-        dq = torch.empty_like(q)
-        dk = torch.empty_like(k)
-        dv = torch.empty_like(v)
-        L = _lib.lib()
-        ws = _workspace(L.vafa_varlen_bwd_workspace(plan.info, D), q.device)
-        _lib.check(L.vafa_varlen_bwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
-            lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            plan.items.data_ptr(), plan.info, D, _lib.dtype_code(q.dtype), float(ctx.scale),
-            ws.data_ptr() if ws.numel() else None, ws.numel(), _lib.stream_ptr(q.device)))
-        return dq, dk, dv, None, None, None
+        return *_lib.ops().varlen_bwd(q, k, v, o, lse, do, ctx.plan.native, ctx.scale), \
+            None, None, None
 
 
 def packed_varlen_attn(
