@@ -165,6 +165,51 @@ def test_absorb_du_split(device, H, d_kv, dtype):
         assert_close(n, a, r)
 
 
+# du, aX and dX in one kernel (segments of at most 64 rows, 65 to 256 features):
+# row counts at the edges of its 16-row groups, key counts at those of its 32-key
+# tiles and 4-deep ring, split and whole ranges, segments without queries or keys.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("H,d_kv", [(1, 72), (1, 128), (2, 192), (4, 216), (8, 256), (1, 250)])
+def test_absorb_merged_backward(device, H, d_kv, dtype):
+    rows = [1, 15, 16, 17, 32, 33, 48, 49, 63, 64, 0, 2, 64, 5, 64]
+    k_lens = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 40, 300, 513, 7, 257]
+    q_lens = [-(-r // H) for r in rows]
+    print(f"[absorb merged {dtype}] H={H} d_kv={d_kv}", flush=True)
+    plan = _lib.plan_absorb(cu_from_lens(q_lens).numpy(), cu_from_lens(k_lens).numpy(), H,
+                            d_kv, 32)
+    assert plan.info.n_fkv == plan.info.n_dq > 0 and plan.info.n_dqc > 0
+    got, ref = run_case(q_lens, k_lens, dtype, device, d_q=64, d_kv=d_kv, H=H, D_H=32)
+    for n, a, r in zip(NAMES, got, ref):
+        assert_close(n, a, r)
+
+
+def test_absorb_merged_beside_streamed(device):
+    """A launch of more than 384k keys whose segments lie on both sides of 64
+    rows: merged items, and the du and dX kernels for the rest.  The keys of
+    two long segments carry the launch over the line; the others' gradients
+    are compared with a launch without them."""
+    H, d_kv = 8, 128
+    q_lens, k_lens = [3, 9, 8, 20, 0, 1], [70, 300, 33, 129, 20, 5]
+    g = torch.Generator().manual_seed(3)
+    mk = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(torch.bfloat16)
+
+    def grads(big):
+        ql, kl = q_lens + ([1, 9] if big else []), k_lens + ([200000] * 2 if big else [])
+        Tq, Tk = sum(ql), sum(kl)
+        u, X, W, dO = ins
+        dev = [t.to(device).requires_grad_(True) for t in (u[:Tq], X[:Tk], W)]
+        O = target_attn_inner(*dev, cu_from_lens(ql).to(device), cu_from_lens(kl).to(device))
+        return torch.autograd.grad(O, dev[:2], dO[:Tq].to(device))
+
+    n_q, n_k = sum(q_lens), sum(k_lens)
+    ins = (mk(n_q + 10, H, d_kv), mk(n_k + 400000, d_kv), mk(d_kv, H, 32), mk(n_q + 10, H, 32))
+    for a, b in zip(grads(False), grads(True)):
+        n = a.shape[0]
+        err = (a.float() - b[:n].float()).abs().max().item()
+        # the same products in another order, rounded once to bf16
+        assert torch.isfinite(b).all() and err <= 2.0 ** -7 * a.float().abs().max().item()
+
+
 def test_absorb_bf16_config4_dims(device):
     """C4 dims (D_in=256, N(0,1) inputs, Xavier weights) on a small sample."""
     from varlenabsorbflashattn_amd import workloads as W

@@ -527,19 +527,35 @@ def test_varlen_bwd_rejects_fused_items_at_wider_head_dim(D):
 def test_absorb_du_split_sections(q_lens, k_lens, H):
     """The dU pass's items (dq) cover every token tile's key range once, in
     equal chunks of at least 128 keys (but the last), with partial rows that tile
-    [0, n_fpart_rows); without a split both sections are empty."""
+    [0, n_fpart_rows).  The first n_fkv items are those of the segments of at most
+    64 rows (one tile each; a segment without queries is an item without
+    tokens), and the kv items beyond n_kv_res those of the others.  H > 64 has
+    neither section."""
     cq, ck = _cu(q_lens), _cu(k_lens)
     p = _lib.plan_absorb(cq, ck, H, 256, 32)
     dq, dqc = p.section("dq").tolist(), p.section("dqc").tolist()
     split = H <= 64 and any(q > 0 and k > 256 for q, k in zip(q_lens, k_lens))
-    assert bool(dq) == bool(dqc) == split
+    assert bool(dq) == (H <= 64) and bool(dqc) == split
+    assert p.info.off_fkv == p.info.off_dq
+    small = [q * H <= 64 for q in q_lens]
+    assert [small[r[5]] for r in dq] == sorted((small[r[5]] for r in dq), reverse=True)
+    assert p.info.n_fkv == sum(small[r[5]] for r in dq)
+    if H <= 64:
+        kv = p.section("kv").tolist()
+        assert [small[r[4]] for r in kv] == [True] * p.info.n_kv_res + [False] * (
+            len(kv) - p.info.n_kv_res)
+        empty = [r for r in dq if r[0] == r[1]]
+        assert sorted(r[5] for r in empty) == [s for s, (q, k) in enumerate(zip(q_lens, k_lens))
+                                               if q == 0 and k > 0]
+        assert all((r[2], r[3]) == (ck[r[5]], ck[r[5] + 1]) for r in empty)
+    dq = [r for r in dq if r[0] < r[1]]
     assert p.info.max_dqc_rows == max([r[1] - r[0] for r in dqc], default=0)
     rows = np.zeros(p.info.n_fpart_rows, dtype=np.int64)
     comb = {(r[0], r[1]): r for r in dqc}
     tiles = {}
     for t0, t1, k0, k1, pb, seg, j, ns in dq:
         tiles.setdefault((t0, t1), []).append((j, k0, k1, pb, ns))
-    if split:
+    if H <= 64:
         assert set(tiles) == {(r[0], r[1]) for r in p.section("qt").tolist()}
     for (t0, t1), its in tiles.items():
         its.sort()

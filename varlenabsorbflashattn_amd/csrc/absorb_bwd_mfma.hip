@@ -20,6 +20,8 @@
 //     summed over heads in registers (no partial buffers, no atomics).
 // dAX = dO W_V^T arrives in the input dtype: the reference rounds it to that
 // dtype before every product it feeds (ta/kernels.py:480, 617-626).
+#include <type_traits>
+
 #include "absorb_tiles.h"
 
 namespace vafa {
@@ -576,6 +578,305 @@ __global__ __launch_bounds__(64 * kDxWaves, FP > kMaxF ? 1 : 2) void absorb_dx_k
   wait_vmcnt<0>();
 }
 
+// ---------------------------------------------------------------------------
+// Both sides in one pass over X, for samples of at most 64 (token, head) rows:
+// du, aX and dX from one read of X and one S / dP / exp2 per (row, key).
+// ---------------------------------------------------------------------------
+// The two kernels above read X twice and form S and dP twice; each moves its
+// bytes at 4.3-4.6 TB/s, near a device copy's rate, so only a pass less makes
+// them faster.  One workgroup of 8 waves per CU (two per SIMD) holds a sample's
+// u and dAX rows in LDS, a 4-deep LDS-DMA ring of 32-key X tiles and two slots
+// of P and scale*dS, which the waves exchange so that each phase splits the way
+// it reads least:
+//   A  wave (16 rows, 16 keys): S^T = X U^T, dP^T = X dAX^T (U^T / dAX^T
+//      fragments in registers), P and scale*dS rounded to T into the slot;
+//   B  wave (32 features): du^T += X^T dS^T, aX^T += X^T P^T over all rows;
+//   C  wave (32 features): dX^T = dAX^T P + U^T (scale dS) over all rows, stored.
+// Between two barriers a wave runs A of tile j+1, then B and C of tile j, so one
+// barrier per tile suffices.  Per 32-key tile and 64 rows 1536 cycles of
+// products per SIMD and 270 KB of LDS reads.  C4 (2048 samples, 648k keys, 853
+// MB): 273 us in the two kernels, 202 here (4.2 TB/s); 1127 samples of <= 2048
+// keys, D_KV 216 (those of at most 64 rows): 326 -> 245.  Measured on the way: dX
+// stored as 2-byte elements (16 stores a wave and tile instead of 2) 280 -> 226;
+// waves of one SIMD in opposite phase order (twice the code, 10 spills) 226
+// against 202; B and C before A 207.
+constexpr int kMgWaves = 8;
+
+template <int FP>
+struct MgSmem {
+  static constexpr int XS = FP + kXPad16;
+  static constexpr int kTile = kBK * XS;           // elements of one X tile
+  static constexpr int kRing = 4;
+  static constexpr int kRows = kDxResidentRows * XS;  // u or dAX rows
+  static constexpr int PS = kBK + 16;              // row stride of P / dS
+  static constexpr int kP = kDxResidentRows * PS;  // P or dS of one tile
+  static constexpr int kBytes = (kRing * kTile + 2 * kRows + 4 * kP) * 2;
+};
+
+template <typename T, int FP>
+__global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
+    const T *__restrict__ u, const T *__restrict__ X, const T *__restrict__ dax,
+    const float *__restrict__ lse, const float *__restrict__ delta, T *__restrict__ du,
+    float *__restrict__ ax, float *__restrict__ part_du, float *__restrict__ part_ax,
+    T *__restrict__ dX, const int32_t *__restrict__ items, int H, int F, float c, float scale) {
+  using M16 = Mfma16<T>;
+  using M = Mfma<T>;
+  using v8 = typename M::v8;
+  using S = MgSmem<FP>;
+  constexpr int XS = S::XS, PS = S::PS;
+  constexpr int NK = FP / 32;                  // 32-wide reduction chunks of S^T / dP^T
+  constexpr int kPerWave = kBK / kMgWaves;     // DMA instructions per wave per tile
+  constexpr int kStores = 2;                   // dX stores per wave per tile
+  constexpr int kPre = 4;
+  typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *xbuf = reinterpret_cast<T *>(smem_raw);
+  T *us = xbuf + S::kRing * S::kTile, *gs = us + S::kRows, *ps = gs + S::kRows;
+
+  const PlanItem it = load_item(items, blockIdx.x);
+  const int t0 = it.v[0], t1 = it.v[1], k0 = it.v[2], k1 = it.v[3], pbase = it.v[4];
+  const int nrows = (t1 - t0) * H;
+  if (nrows > kDxResidentRows) return;
+  const int tid = threadIdx.x;
+  if (nrows == 0) {  // a sample without queries: its keys get zero gradient
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    // (a uniform trip count: a divergent loop exit on the way to the return
+    // would make the compiler pass every scalar of the kernel through VGPRs)
+    for (int k = k0; k < k1; ++k)
+      if (tid < F / 8) *reinterpret_cast<u32x4 *>(dX + (int64_t)k * F + tid * 8) = z;
+    return;
+  }
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lq = lane >> 4, l32 = lane & 31, lh = lane >> 5;
+  const int rg = wave & 3, kh = wave >> 2;     // phase A: 16 rows, 16 keys
+  const int nrg = (nrows + 15) / 16;
+  const bool has_f = wave * 32 < FP;           // phases B and C: 32 features
+  const int nt = (k1 - k0 + kBK - 1) / kBK;
+
+  // (width and wave are opaque to each DMA block: values shared between the
+  // blocks' lane conditions would be merged at their joins, in VGPRs)
+  auto dma = [&](const T *src, int rows, T *dst) {
+    int w = wave, f = F;
+    asm volatile("" : "+s"(w), "+s"(f));
+    dma_block<FP, kMgWaves, XS>(src, (uint32_t)(rows * f * 2), f, lds_addr(dst), w, lane);
+  };
+  auto rows_dma = [&](const T *src, T *dst) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)  // a block without rows reads as zeros
+      dma(src + ((int64_t)t0 * H + 32 * b) * F, uniform_clamp(nrows - 32 * b, 32),
+          dst + 32 * b * XS);
+  };
+  auto issue = [&](int j) {
+    const int kb = k0 + j * kBK;
+    dma(X + (int64_t)kb * F, uniform_clamp(k1 - kb, kBK),
+        xbuf + (j & (S::kRing - 1)) * S::kTile);
+  };
+  rows_dma(u, us);
+  rows_dma(dax, gs);
+#pragma unroll
+  for (int j = 0; j < S::kRing - 1; ++j)
+    if (j < nt) issue(j);
+  const int row = rg * 16 + l16;
+  const bool row_ok = row < nrows;
+  float L = row_ok ? lse[(int64_t)t0 * H + row] : __builtin_inff();
+  float dl = row_ok ? delta[(int64_t)t0 * H + row] : 0.f;
+  asm volatile("" : "+v"(L), "+v"(dl));  // waited for here, before the loop
+  wait_vmcnt<0>();
+  __syncthreads();
+  v8 uf[NK], gf[NK];
+#pragma unroll
+  for (int kc = 0; kc < NK; ++kc) {
+    uf[kc] = as_v8<T>(lds_ld16<T>(as_lds(us + row * XS + kc * 32 + lq * 8)));
+    gf[kc] = as_v8<T>(lds_ld16<T>(as_lds(gs + row * XS + kc * 32 + lq * 8)));
+  }
+  f32x4 adu[2][4], aax[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) adu[i][g] = aax[i][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int a_off = (kh * 16 + l16) * XS + lq * 8;
+  const int t_off = (4 * lq + (l16 >> 2)) * XS + 4 * (l16 & 3) + wave * 32;
+  // transposed 32x32 operands (layout of tr_operand): P / dS slots and u / dAX
+  const int tr = 4 * (lane >> 5) + ((lane & 15) >> 2), tc = ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
+  // dX: lane holds the key of slot position l32, 8 features from f_out (and 16
+  // further); features past F fall outside the store's range
+  const int key_out = (l32 & 7) < 4 ? 4 * (l32 >> 3) + (l32 & 3) : 16 + 4 * (l32 >> 3) + (l32 & 3);
+  const int f_out = wave * 32 + 8 * lh;
+  const int st_off = f_out < F ? (key_out * F + f_out) * 2 : 0x7fff0000;
+  const int st_off16 = f_out + 16 < F ? st_off + 32 : 0x7fff0000;
+
+  // A: lane holds keys 16 kh + 4 lq + r of its row; in the slot the 32 keys of a
+  // tile lie in the order 8a + b <-> 4a + b (b < 4), 16 + 4a + b - 4, which the
+  // transposed X reads of phase B give their reduction
+  auto phase_a = [&](int j) {
+    if (rg >= nrg) return;
+    const lds_cptr<T> xa = as_lds(xbuf + (j & (S::kRing - 1)) * S::kTile + a_off);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+    u32x4 ring[kPre];
+    constexpr int kP0 = kPre < NK ? kPre : NK;
+#pragma unroll
+    for (int i = 0; i < kP0; ++i) ring[i] = lds_ld16<T>(xa + i * 32);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kc = 0; kc < NK; ++kc) {
+      const v8 a = as_v8<T>(ring[kc % kPre]);
+      s = M16::mma(a, uf[kc], s);
+      dp = M16::mma(a, gf[kc], dp);
+      if (kc + kPre < NK) ring[kc % kPre] = lds_ld16<T>(xa + (kc + kPre) * 32);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int kb = k0 + j * kBK + kh * 16 + lq * 4;
+    T4 pv, sv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float p = fast_exp2(__builtin_fmaf(s[r], c, -L));
+      if (kb + r >= k1) p = 0.f;
+      pv[r] = static_cast<T>(p);
+      sv[r] = static_cast<T>(p * (dp[r] - dl) * scale);
+    }
+    T *slot = ps + (j & 1) * 2 * S::kP + row * PS + lq * 8 + kh * 4;
+    *reinterpret_cast<T4 *>(slot) = pv;
+    *reinterpret_cast<T4 *>(slot + S::kP) = sv;
+  };
+  // B and C over the NG 16-row groups in use, each operand of the next group
+  // read as soon as the current product has taken it
+  auto phase_bc = [&](int j, auto ng) {
+    constexpr int NG = decltype(ng)::value;
+    const lds_cptr<T> xt = as_lds(xbuf + (j & (S::kRing - 1)) * S::kTile + t_off);
+    const lds_cptr<T> pp = as_lds(ps + (j & 1) * 2 * S::kP);
+    const lds_cptr<T> pr = pp + l16 * PS + lq * 8, pt = pp + tr * PS + tc;
+    const lds_cptr<T> ut = as_lds(us) + tr * XS + tc + wave * 32, gt = ut + S::kRows;
+    auto trop = [&](lds_cptr<T> q, int stride) {
+      return as_v8<T>(join(lds_tr8<T>(q), lds_tr8<T>(q + 8 * stride)));
+    };
+    v8 xa[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      xa[i] = as_v8<T>(join(lds_tr8<T>(xt + 16 * i), lds_tr8<T>(xt + 16 * XS + 16 * i)));
+    v8 og, op, ob, os, ou, od;
+    auto load_c1 = [&](int g) {
+      op = trop(pt + 16 * g * PS, PS);
+      og = trop(gt + 16 * g * XS, XS);
+    };
+    auto load_b = [&](int g) {
+      ob = as_v8<T>(lds_ld16<T>(pr + 16 * g * PS));
+      os = as_v8<T>(lds_ld16<T>(pr + S::kP + 16 * g * PS));
+    };
+    auto load_c2 = [&](int g) {
+      od = trop(pt + S::kP + 16 * g * PS, PS);
+      ou = trop(ut + 16 * g * XS, XS);
+    };
+    load_c1(0);
+    load_b(0);
+    load_c2(0);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      acc = M::mma(og, op, acc);
+      if (g + 1 < NG) load_c1(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        aax[i][g] = M16::mma(xa[i], ob, aax[i][g]);
+        adu[i][g] = M16::mma(xa[i], os, adu[i][g]);
+      }
+      if (g + 1 < NG) load_b(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      acc = M::mma(ou, od, acc);
+      if (g + 1 < NG) load_c2(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // dX^T: element 4 g + e is feature 8 g + 4 lh + e of this lane's key; the
+    // halves of a pair of g are swapped between lanes l and l + 32, so a lane
+    // stores 8 features (16 bytes) of g = 2 i + lh and a row leaves as 2 x 32 bytes
+    const int kb = k0 + j * kBK;
+    const rsrc_t rs = make_rsrc32(dX + (int64_t)kb * F,
+                                  (uint32_t)(uniform_clamp(k1 - kb, kBK) * F * 2));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      u32x4 w;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        typedef __attribute__((__vector_size__(2 * sizeof(T)))) T T2;
+        const T2 x = {static_cast<T>(acc[8 * i + 2 * h]), static_cast<T>(acc[8 * i + 2 * h + 1])};
+        const T2 y = {static_cast<T>(acc[8 * i + 4 + 2 * h]),
+                      static_cast<T>(acc[8 * i + 4 + 2 * h + 1])};
+        uint32_t lo = __builtin_bit_cast(uint32_t, x), hi = __builtin_bit_cast(uint32_t, y);
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
+        w[h] = lo;
+        w[2 + h] = hi;
+      }
+      __builtin_amdgcn_raw_buffer_store_b128(w, rs, i == 0 ? st_off : st_off16, 0, 0);
+    }
+  };
+
+  // one instance per number of 16-row groups
+  auto run = [&](auto ng) {
+    phase_a(0);
+    for (int j = 0; j < nt; ++j) {
+      // tile j+1 landed (the first three did before the loop): behind its DMA lie
+      // at most tile j+2's and the stores of two intervals
+      if (j >= 2 && j + 1 < nt) {
+        if (j + 2 < nt) {
+          if (has_f)
+            wait_vmcnt<kPerWave + 2 * kStores>();
+          else
+            wait_vmcnt<kPerWave>();
+        } else {
+          if (has_f)
+            wait_vmcnt<2 * kStores>();
+          else
+            wait_vmcnt<0>();
+        }
+      }
+      // tile j+1 and the slot of tile j are visible; tile j-1's ring slot and
+      // the other P slot are free
+      __syncthreads();
+      if (j + S::kRing - 1 < nt) issue(j + S::kRing - 1);
+      if (j + 1 < nt) phase_a(j + 1);
+      if (has_f) phase_bc(j, ng);
+    }
+  };
+  if (nt > 0) {
+    switch (nrg) {
+      case 1: run(std::integral_constant<int, 1>{}); break;
+      case 2: run(std::integral_constant<int, 2>{}); break;
+      case 3: run(std::integral_constant<int, 3>{}); break;
+      default: run(std::integral_constant<int, 4>{}); break;
+    }
+  }
+  wait_vmcnt<0>();
+
+  if (!has_f) return;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int r = 16 * g + l16;
+    if (r >= nrows) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int f = wave * 32 + 16 * i + lq * 4;
+      if (f >= F) continue;
+      if (pbase < 0) {
+        const int64_t o = ((int64_t)t0 * H + r) * F + f;
+        T4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(adu[i][g][e]);
+        *reinterpret_cast<T4 *>(du + o) = w;
+        *reinterpret_cast<f32x4 *>(ax + o) = aax[i][g];
+      } else {
+        const int64_t o = ((int64_t)pbase * H + r) * F + f;
+        *reinterpret_cast<f32x4 *>(part_du + o) = adu[i][g];
+        *reinterpret_cast<f32x4 *>(part_ax + o) = aax[i][g];
+      }
+    }
+  }
+}
+
 // dAX[t,h,f] = sum_d dO[t,h,d] W_V[f,h,d] (ta/kernels.py:474-476), rounded to
 // the input dtype.  One wave per (32 tokens, head, kDaxTiles f tiles): dAX =
 // dO W_V^T with dO rows as A (32 tokens x 16 d) and W_V rows as B (16 d x 32 f).
@@ -665,6 +966,16 @@ void launch_du_fp(const AbsorbArgs &a, hipStream_t st) {
 }
 
 template <typename T, int FP>
+void launch_merged_fp(const AbsorbArgs &a, hipStream_t st) {
+  const int smem = MgSmem<FP>::kBytes;
+  allow_dynamic_lds(reinterpret_cast<const void *>(&absorb_bwd_kernel<T, FP>), smem);
+  hipLaunchKernelGGL((absorb_bwd_kernel<T, FP>), dim3((unsigned)a.n_merged), dim3(64 * kMgWaves),
+                     smem, st, (const T *)a.u, (const T *)a.X, (const T *)a.dax, a.lse_in, a.delta,
+                     (T *)a.du, a.ax, a.part_du, a.part_ax, (T *)a.dX, a.merged_items, a.H, a.F,
+                     a.scale * kLog2e, a.scale);
+}
+
+template <typename T, int FP>
 void launch_dx_fp(const AbsorbArgs &a, hipStream_t st) {
   const int smem = DxSmem<FP>::kBytes;
   // the plan puts the resident-row items first (items are 8 int32 each): each
@@ -689,17 +1000,35 @@ void launch_dx_fp(const AbsorbArgs &a, hipStream_t st) {
 
 }  // namespace
 
+// Widths of the merged kernel.  At 64 features two of its eight waves have a
+// slice in B and C: C4's forward + backward 245 us against 214 on the two
+// kernels (128: 320 both, 192: 388 against 429, 256: 448 against 543).
+bool mfma_absorb_merged(int F) { return padded_f(F) >= 128 && padded_f(F) <= kMaxF; }
+
+template <typename T>
+void launch_mfma_absorb_bwd_merged(const AbsorbArgs &a, hipStream_t st) {
+  if (a.n_merged == 0) return;
+  switch (padded_f(a.F)) {
+    case 128: launch_merged_fp<T, 128>(a, st); break;
+    case 192: launch_merged_fp<T, 192>(a, st); break;
+    case 224: launch_merged_fp<T, 224>(a, st); break;
+    case 256: launch_merged_fp<T, 256>(a, st); break;
+    default: break;
+  }
+}
+
 template <typename T>
 void launch_mfma_absorb_du(const AbsorbArgs &a, hipStream_t st) {
-  if (a.n_qseg == 0) return;
-  switch (padded_f(a.F)) {
-    case 64: launch_du_fp<T, 64>(a, st); break;
-    case 128: launch_du_fp<T, 128>(a, st); break;
-    case 192: launch_du_fp<T, 192>(a, st); break;
-    case 224: launch_du_fp<T, 224>(a, st); break;
-    case 256: launch_du_fp<T, 256>(a, st); break;
-    case 512: launch_du_fp<T, 512>(a, st); break;
-    default: break;
+  if (a.n_qseg > 0) {
+    switch (padded_f(a.F)) {
+      case 64: launch_du_fp<T, 64>(a, st); break;
+      case 128: launch_du_fp<T, 128>(a, st); break;
+      case 192: launch_du_fp<T, 192>(a, st); break;
+      case 224: launch_du_fp<T, 224>(a, st); break;
+      case 256: launch_du_fp<T, 256>(a, st); break;
+      case 512: launch_du_fp<T, 512>(a, st); break;
+      default: break;
+    }
   }
   launch_du_combine<T>(a, st);
 }
@@ -735,6 +1064,8 @@ bool launch_mfma_absorb_dax(const AbsorbArgs &a, hipStream_t st) {
 
 template bool launch_mfma_absorb_dax<bf16>(const AbsorbArgs &, hipStream_t);
 template bool launch_mfma_absorb_dax<f16>(const AbsorbArgs &, hipStream_t);
+template void launch_mfma_absorb_bwd_merged<bf16>(const AbsorbArgs &, hipStream_t);
+template void launch_mfma_absorb_bwd_merged<f16>(const AbsorbArgs &, hipStream_t);
 template void launch_mfma_absorb_du<bf16>(const AbsorbArgs &, hipStream_t);
 template void launch_mfma_absorb_du<f16>(const AbsorbArgs &, hipStream_t);
 template void launch_mfma_absorb_dx<bf16>(const AbsorbArgs &, hipStream_t);

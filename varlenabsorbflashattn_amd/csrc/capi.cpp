@@ -373,8 +373,18 @@ void absorb_bwd_all(const AbsorbArgs &a, hipStream_t st) {
   }
   if (mfma) {
     if constexpr (sizeof(T) == 2) {
-      launch_mfma_absorb_du<T>(a, st);
-      launch_mfma_absorb_dx<T>(a, st);
+      AbsorbArgs r = a;  // what the merged kernel leaves to the du and dX kernels
+      const bool all = a.n_merged == a.n_qseg;
+      if (a.n_merged > 0 && mfma_absorb_merged(a.F) && (all || a.T_k > kAbsorbMergedKeys)) {
+        launch_mfma_absorb_bwd_merged<T>(a, st);
+        r.qseg_items = a.qseg_items + a.n_merged * VAFA_ITEM_INTS;
+        r.n_qseg = a.n_qseg - a.n_merged;
+        r.kv_items = a.kv_items + a.n_kv_res * VAFA_ITEM_INTS;
+        r.n_kv = a.n_kv - a.n_kv_res;
+        r.n_kv_res = 0;
+      }
+      launch_mfma_absorb_du<T>(r, st);
+      launch_mfma_absorb_dx<T>(r, st);
     }
   } else if (sizeof(T) == 4 && f32_absorb_supported(a.H, a.F, a.DH)) {
     launch_f32_absorb_du_dx(a, st);
@@ -1016,7 +1026,9 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
                     int64_t workspace_bytes, void *stream) {
   if (int rc = check_info(info, 2)) return rc;
   if (int rc = check_absorb_dims(D_KV, D_H)) return rc;
-  if (info->n_dqc > 0 && info->H > kAbsorbRows)
+  if (info->n_fkv < 0 || info->n_fkv > info->n_dq)
+    return fail(VAFA_ERR_VALUE, "plan info is inconsistent (n_fkv)");
+  if (info->n_dq > 0 && info->H > kAbsorbRows)
     return fail(VAFA_ERR_VALUE, "plan splits token tiles, which H=%lld does not run",
                 (long long)info->H);
   AbsorbWs w = carve_absorb(workspace, info, D_KV, D_H, true);
@@ -1047,8 +1059,9 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
   a.comb_rows = (int)info->max_comb_rows;
   a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
   a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
-  if (info->n_dq > 0) {  // the du pass splits key ranges
+  if (info->n_dq > 0) {  // the du pass's own items (split key ranges, merged tiles first)
     a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
+    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv;
   }
   a.T_q = info->T_q; a.T_k = info->T_k;
   a.H = (int)info->H; a.F = (int)F; a.DH = (int)D_H; a.scale = scale;

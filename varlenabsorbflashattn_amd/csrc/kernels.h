@@ -75,6 +75,8 @@ struct AbsorbArgs {
   int64_t n_items, n_comb, n_kv, n_qseg;
   int64_t n_kv_res;           // leading kv items for absorb_dx_res_kernel
   int comb_rows;              // most tokens of one combine item
+  const int32_t *merged_items;  // token tiles whose du, aX and dX one kernel forms
+  int64_t n_merged;
   const int32_t *qtc_items;   // split token tiles of the du pass
   int64_t n_qtc;
   int qtc_rows;               // most tokens of one of them
@@ -196,6 +198,9 @@ void launch_rowgemm_f32(const RowGemm &, bool kj, hipStream_t);
 // dst [C, R] = src [R, C]^T
 template <typename T> void launch_transpose2d(const void *src, void *dst, int R, int C, hipStream_t);
 // absorb_bwd_mfma.hip: du/aX (query side) and dX (key side) on matrix cores
+// du / aX and dX of the merged items in one pass over X (at most 64 rows each)
+bool mfma_absorb_merged(int F);
+template <typename T> void launch_mfma_absorb_bwd_merged(const AbsorbArgs &, hipStream_t);
 template <typename T> void launch_mfma_absorb_du(const AbsorbArgs &, hipStream_t);
 // dAX = dO W_V^T; false (nothing launched) for a D_H it does not cover
 template <typename T> bool launch_mfma_absorb_dax(const AbsorbArgs &, hipStream_t);

@@ -500,11 +500,15 @@ int vafa_plan_varlen_balanced(const int64_t *cu_q, const int64_t *cu_k, int64_t 
 //                 segment's whole token range [t0, t1).
 //   qt section  : {t0, t1, k0, k1, -1, seg, 0, 1} unsplit token tiles with the
 //                 segment's whole key range (backward dU pass).
-//   dq, dqc     : where the dU pass splits key ranges (its own policy), the
-//                 items it runs instead of qt, {t0, t1, k0, k1, pbase, seg,
-//                 split, nsplit} with fp32 du / aX partials in rows pbase + r
-//                 (n_fpart_rows in all), and one item per split tile, laid out
-//                 as the comb items.
+//   dq, dqc     : (H <= kAbsorbRows) the items the backward runs instead of
+//                 qt, {t0, t1, k0, k1, pbase, seg, split, nsplit}, key ranges
+//                 split by a policy of their own with fp32 du / aX partials in
+//                 rows pbase + r (n_fpart_rows in all), and one item per split
+//                 tile, laid out as the comb items.  The first n_fkv items (off_fkv
+//                 = off_dq) belong to segments of at most kDxResidentRows rows,
+//                 whose dX the merged kernel forms too (t0 == t1: a segment
+//                 without queries, whose dX is cleared); the kv items beyond
+//                 n_kv_res belong to the others.
 int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
                      int64_t D_KV, int64_t D_H, int32_t *plan, int64_t plan_cap,
                      vafa_plan_info *info) {
@@ -533,9 +537,7 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   };
   raise_chunk(pol, kAbsorbSlack2, 2 * kAbsorbSlots);
   raise_chunk(du_pol, kAbsorbDuSlack, kAbsorbDuSlots);
-  bool du_split = false;  // some token tile's range is split
-  for (int64_t s = 0; s + 1 < n1 && H <= kAbsorbRows && !du_split; ++s)
-    du_split = cu_q[s + 1] > cu_q[s] && cu_k[s + 1] - cu_k[s] > du_pol.long_threshold;
+  const bool du_items = H <= kAbsorbRows;  // the wave-per-row kernels run qt and kv
   std::memset(info, 0, sizeof(*info));
   info->magic = VAFA_PLAN_MAGIC;
   info->kind = 2;
@@ -565,17 +567,20 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
       key_split(std::min<int64_t>(lq, TT) * H, lk, p, &ns, &chunk);
     }
     max_split = std::max(max_split, ns);
-    // the du pass's own split; the wave-per-row kernels (H > kAbsorbRows) walk
-    // whole key ranges
+    // the du pass's own split; a segment without queries is one item of the
+    // merged kernel, which clears its dX
     int64_t du_ns = 1, du_chunk = lk;
-    if (du_split && lq > 0) key_split(kAbsorbRows, lk, du_pol, &du_ns, &du_chunk);
+    if (du_items && lq > 0) key_split(kAbsorbRows, lk, du_pol, &du_ns, &du_chunk);
+    if (du_items && lq == 0 && lk > 0)
+      qs.push_back(Item{{(int32_t)q0, (int32_t)q0, (int32_t)k0, (int32_t)k1, -1, (int32_t)s, 0, 1},
+                        0});
     const int64_t seg_prow = prow;
     for (int64_t t = q0; t < q1; t += TT) {
       const int64_t te = std::min(t + TT, q1), ntok = te - t;
       const int64_t row_cost = round_up(ntok * H, 32);
       qt.push_back(Item{{(int32_t)t, (int32_t)te, (int32_t)k0, (int32_t)k1, -1, (int32_t)s, 0, 1},
                         (lk + pol.item_overhead) * row_cost});
-      for (int64_t j = 0; du_split && j < du_ns; ++j) {
+      for (int64_t j = 0; du_items && j < du_ns; ++j) {
         const int64_t a = k0 + j * du_chunk, b = du_ns > 1 ? std::min(k1, a + du_chunk) : k1;
         const int32_t pb = du_ns > 1 ? (int32_t)(qprow + j * ntok) : -1;
         qs.push_back(Item{{(int32_t)t, (int32_t)te, (int32_t)a, (int32_t)b, pb, (int32_t)s,
@@ -625,12 +630,22 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   info->n_kv_res = (int64_t)(res_end - kv.order.begin());
   sort_lpt(qt);
   sort_lpt(qs);
+  // tiles that hold a whole segment of at most kDxResidentRows rows first: the
+  // merged kernel's items, n_fkv of them (off_fkv = off_dq)
+  const auto mg_end = std::stable_partition(qs.order.begin(), qs.order.end(), [&](uint32_t i) {
+    const Item &it = qs.items[i];
+    const int64_t lq = cu_q[it.v[5] + 1] - cu_q[it.v[5]];
+    return lq * H <= kDxResidentRows;
+  });
   comb.keep_order();
   qsc.keep_order();
   info->n_part_rows = prow;
   info->n_fpart_rows = qprow;
   info->max_split = max_split;
-  return emit(fwd, comb, kv, qt, qs, qsc, {}, {}, plan, plan_cap, info);
+  rc = emit(fwd, comb, kv, qt, qs, qsc, {}, {}, plan, plan_cap, info);
+  info->off_fkv = info->off_dq;
+  info->n_fkv = (int64_t)(mg_end - qs.order.begin());
+  return rc;
 }
 
 }  // extern "C"

@@ -114,5 +114,11 @@ constexpr int kXcds = 8;
 // them resident in one workgroup (absorb_dx_res_kernel); longer segments are
 // streamed in 32-row blocks (absorb_dx_kernel).
 constexpr int kDxResidentRows = 64;
+// 16-bit backward: the segments of at most kDxResidentRows rows run on the
+// merged kernel when they are all of the launch or it holds more keys than this;
+// in a smaller mixed launch a third kernel costs more than the pass saved (100
+// samples of <= 2048 keys, a quarter above 64 rows, forward + backward: 187 us
+// merged, 179 not; 500 samples 437 and 470).
+constexpr int64_t kAbsorbMergedKeys = 384 * 1024;
 
 }  // namespace vafa
