@@ -329,6 +329,21 @@ VAFA_API int vafa_absorb_project_bwd(const void *q_raw, const void *W_Q, const v
                                      int64_t D_KV, int64_t D_H, int32_t dtype, void *workspace,
                                      int64_t workspace_bytes, void *stream);
 
+/* The whole packed_target_attn backward of vafa_absorb_fwd_full in one call
+ * (vafa_absorb_project_u, vafa_absorb_bwd and vafa_absorb_project_bwd, in fewer
+ * launches): from dO and what the forward saved to dq_raw, dX, dW_Q, dW_K, dW_V.
+ * Any of dq_raw, dW_Q, dW_K may be NULL. */
+VAFA_API int64_t vafa_absorb_bwd_full_workspace(const vafa_plan_info *info, int64_t T_q,
+                                                int64_t D_Q, int64_t D_KV, int64_t D_H);
+VAFA_API int vafa_absorb_bwd_full(const void *q_raw, const void *X, const void *W_Q,
+                                  const void *W_K, const void *W_V, const void *q_proj,
+                                  const void *O, const void *dO, const float *lse, void *dq_raw,
+                                  void *dX, void *dW_Q, void *dW_K, void *dW_V, int64_t T_q,
+                                  const int32_t *plan_dev, const vafa_plan_info *info,
+                                  int64_t D_Q, int64_t D_KV, int64_t D_H, int32_t dtype,
+                                  float scale, void *workspace, int64_t workspace_bytes,
+                                  void *stream);
+
 /* The projections and their backward on fp32 operands (fp32 matrix cores,
  * IEEE products; the reference's documented fp32 call): any D_Q and D_KV, D_H a
  * multiple of 8, 16-byte aligned operands.  u may be NULL in the forward, any

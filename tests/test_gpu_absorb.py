@@ -587,6 +587,31 @@ def test_absorb_fold_matches_unfused_and_oracle(device, H, D_H, d_kv, dtype):
         assert_close(n + " vs unfused", a, b.detach().float().cpu().numpy())
 
 
+# The folded shapes' backward forms u, dAX, delta and W_K^T in one launch and
+# sums the weight gradients' chunks in one: token counts at its 32-token tiles
+# (one and several chunks), column blocks past D_KV, 2..16 lanes a delta row,
+# a D_Q in slices, and any subset of the query-side gradients.
+@pytest.mark.parametrize("T", [1, 32, 33, 600])
+@pytest.mark.parametrize("H,D_H,d_kv,d_q", [(8, 32, 216, 64), (4, 16, 256, 520), (4, 128, 72, 8),
+                                            (1, 64, 8, 64)])
+def test_absorb_full_backward(device, T, H, D_H, d_kv, d_q):
+    q_lens, k_lens = [T - T // 2, T // 2], [70, 300]
+    print(f"[absorb full bwd] T={T} H={H} D_H={D_H} d_kv={d_kv} d_q={d_q}", flush=True)
+    got, ref = run_case(q_lens, k_lens, torch.bfloat16, device, d_q=d_q, d_kv=d_kv, H=H, D_H=D_H)
+    for n, a, r in zip(NAMES, got, ref):
+        assert_close(n, a, r)
+    ins = [t.to(torch.bfloat16) for t in make_inputs(q_lens, k_lens, d_q, d_kv, H, D_H)]
+    cq, ck = cu_from_lens(q_lens).to(device), cu_from_lens(k_lens).to(device)
+    dO = (torch.randn(got[0].shape, generator=torch.Generator().manual_seed(7)) * 0.1)
+    for need in [(1,), (0, 4), (3,), (2, 3)]:  # positions of the inputs with a gradient
+        dev = [t.to(device).requires_grad_(i in need) for i, t in enumerate(ins)]
+        O = packed_target_attn(*dev, cu_seqlens_q=cq, cu_seqlens_k=ck)
+        O.backward(dO.to(torch.bfloat16).to(device))
+        for i, t in enumerate(dev):
+            assert (t.grad is not None) == (i in need)
+            assert i not in need or torch.equal(t.grad, got[1 + i].to(t.device))
+
+
 def test_absorb_fold_negative_scale(device):
     """A negative scale is folded into u as an exact sign flip (before the
     rounding) by the folded kernel, as by the u-reading one."""

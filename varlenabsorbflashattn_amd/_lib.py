@@ -96,6 +96,9 @@ _SIGS = {
                                               _P]),
     "vafa_absorb_project_f32_bwd": (C.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64,
                                               _I64, _I64, _P, _I64, _P]),
+    "vafa_absorb_bwd_full_workspace": (C.c_int64, [_PINFO, _I64, _I64, _I64, _I64]),
+    "vafa_absorb_bwd_full": (C.c_int, [_P] * 14 + [_I64, _P, _PINFO, _I64, _I64, _I64, _I32,
+                                                   C.c_float, _P, _I64, _P]),
     "vafa_absorb_fwd_full_workspace": (C.c_int64, [_PINFO, _I64, _I64, _I64]),
     "vafa_absorb_fwd_full": (C.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _PINFO, _I64,
                                        _I64, _I64, _I32, C.c_float, _P, _I64, _P]),

@@ -134,18 +134,25 @@ __global__ __launch_bounds__(256) void rowgemm_nt_kernel(
 // X tiles go through a double-buffered LDS ring (the next tile's 16-byte
 // loads held in registers under the current tile's products), and each
 // tile's Y block is staged in LDS and stored while the next X tile lands.
+template <int NJ, int KS>
+struct RgTiles {
+  static constexpr int kXS = 32 * KS + 16;     // padded LDS row stride of an X tile
+  static constexpr int kYS = 64 * NJ + 8;      // and of the Y block
+  static constexpr int kXElems = kRgTok * kXS;
+  static constexpr int kElems = 2 * kXElems + kRgTok * kYS;
+};
+
 template <typename T, int NJ, int KS>
-__global__ __launch_bounds__(256) void rowgemm_tiles_kernel(
-    const T *__restrict__ X, const T *__restrict__ W, T *__restrict__ Y, int64_t T_q, int G,
-    int J, int K, int64_t ldx, int64_t xs, int64_t ws, int64_t ldw, int64_t ldy, int64_t ys,
-    int n_jb, int tiles_per_wg, int64_t n_tt) {
+__device__ __forceinline__ void rowgemm_tiles(
+    T *smem, const T *__restrict__ X, const T *__restrict__ W, T *__restrict__ Y, int64_t T_q,
+    int G, int J, int K, int64_t ldx, int64_t xs, int64_t ws, int64_t ldw, int64_t ldy,
+    int64_t ys, int n_jb, int tiles_per_wg, int64_t n_tt) {
   using M16 = Mfma16<T>;
   constexpr int kKBlk = 32 * KS;
-  constexpr int kXS = kKBlk + 16;
+  constexpr int kXS = RgTiles<NJ, KS>::kXS;
   constexpr int kJB = 64 * NJ;
-  constexpr int kYS = kJB + 8;
-  constexpr int kXElems = kRgTok * kXS;
-  __shared__ __align__(16) T smem[2 * kXElems + kRgTok * kYS];
+  constexpr int kYS = RgTiles<NJ, KS>::kYS;
+  constexpr int kXElems = RgTiles<NJ, KS>::kXElems;
   T *ystage = smem + 2 * kXElems;
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
   const int wave = tid >> 6;
@@ -245,6 +252,60 @@ __global__ __launch_bounds__(256) void rowgemm_tiles_kernel(
     if (tt + 1 < tt1) store_x(buf ^ 1);
     __syncthreads();  // next X tile visible; the Y block is read out
   }
+}
+
+template <typename T, int NJ, int KS>
+__global__ __launch_bounds__(256) void rowgemm_tiles_kernel(
+    const T *__restrict__ X, const T *__restrict__ W, T *__restrict__ Y, int64_t T_q, int G,
+    int J, int K, int64_t ldx, int64_t xs, int64_t ws, int64_t ldw, int64_t ldy, int64_t ys,
+    int n_jb, int tiles_per_wg, int64_t n_tt) {
+  __shared__ __align__(16) T smem[RgTiles<NJ, KS>::kElems];
+  rowgemm_tiles<T, NJ, KS>(smem, X, W, Y, T_q, G, J, K, ldx, xs, ws, ldw, ldy, ys, n_jb,
+                           tiles_per_wg, n_tt);
+}
+
+// What the whole op's backward needs before the attention pass, in one launch
+// (blockIdx.y): 0 u = q_proj W_K,h^T, 1 dAX = dO W_V,h^T -- the same row GEMM --
+// with delta = sum_d dO O by the blocks of its first columns, 2 W_K^T [H*DH, F].
+// Bound by the writes of u and dAX (77 MB on 9424 tokens of 8 heads, 256
+// columns): 29 us there, 40 in the three launches this replaces.
+template <typename T, int NJ, int KS>
+__global__ __launch_bounds__(256) void absorb_prep_kernel(
+    const T *__restrict__ q_proj, const T *__restrict__ wk, T *__restrict__ u,
+    const T *__restrict__ dO, const T *__restrict__ wv, T *__restrict__ dax,
+    const T *__restrict__ O, float *__restrict__ delta, int64_t T_q, T *__restrict__ wkt, int H,
+    int F, int DH, int n_jb, int tiles_per_wg, int64_t n_tt) {
+  __shared__ __align__(16) T smem[RgTiles<NJ, KS>::kElems];
+  const int64_t HD = (int64_t)H * DH;
+  const int tid = threadIdx.x;
+  if (blockIdx.y == 2) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < HD * F; i += (int64_t)gridDim.x * 256)
+      wkt[i] = wk[(i % F) * HD + i / F];
+    return;
+  }
+  if (blockIdx.y == 1) {
+    const int jb = (int)(blockIdx.x % n_jb), h = (int)(blockIdx.x / n_jb % H);
+    if (jb == 0) {
+      const int64_t t0 = (int64_t)(blockIdx.x / n_jb / H) * tiles_per_wg * kRgTok;
+      const int64_t t1 = t0 + (int64_t)tiles_per_wg * kRgTok;
+      const int part = tid & 7;  // 8 lanes a row, 8 elements each at a time
+      for (int64_t t = t0 + (tid >> 3); t < t1; t += 32) {
+        float s = 0.f;
+        for (int d = part * 8; d < DH && t < T_q; d += 64) {
+          const int64_t o = t * HD + (int64_t)h * DH + d;
+          const auto x = as_v8<T>(*reinterpret_cast<const u32x4 *>(dO + o));
+          const auto y = as_v8<T>(*reinterpret_cast<const u32x4 *>(O + o));
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s = __builtin_fmaf(to_f(x[e]), to_f(y[e]), s);
+        }
+        for (int x = 1; x < 8; x <<= 1) s += __shfl_xor(s, x, 64);
+        if (t < T_q && part == 0) delta[t * H + h] = s;
+      }
+    }
+  }
+  const bool g = blockIdx.y == 1;
+  rowgemm_tiles<T, NJ, KS>(smem, g ? dO : q_proj, g ? wv : wk, g ? dax : u, T_q, H, F, DH,
+                           HD, DH, DH, HD, (int64_t)H * F, F, n_jb, tiles_per_wg, n_tt);
 }
 
 // Weight gradient of a projection on 16-bit matrix cores, one workgroup per
@@ -539,6 +600,27 @@ void rowgemm_nj(const RowGemm &p, hipStream_t st) {
                      p.ws, p.ldw, p.ldy, p.ys, n_jb);
 }
 
+template <typename T, int NJ, int KS>
+void prep_nj(const AbsorbArgs &a, const void *q_proj, void *wkt, hipStream_t st) {
+  const int n_jb = (a.F + 64 * NJ - 1) / (64 * NJ);
+  const int64_t n_tt = (a.T_q + kRgTok - 1) / kRgTok;
+  const int64_t units = n_tt * a.H * n_jb;
+  int64_t tpw = 2 * units / kRgTargetWgs;  // two products share the launch
+  tpw = tpw < 1 ? 1 : (tpw > 16 ? 16 : tpw);
+  const int64_t wgs = (n_tt + tpw - 1) / tpw * a.H * n_jb;
+  hipLaunchKernelGGL((absorb_prep_kernel<T, NJ, KS>), dim3((unsigned)wgs, wkt != nullptr ? 3 : 2),
+                     dim3(256), 0, st, (const T *)q_proj, (const T *)a.wk, (T *)a.u_out,
+                     (const T *)a.dO, (const T *)a.wv, (T *)a.dax, (const T *)a.O_in, a.delta,
+                     a.T_q, (T *)wkt, a.H, a.F, a.DH, n_jb, (int)tpw, n_tt);
+}
+
+template <typename T, int NJ>
+void prep_ks(const AbsorbArgs &a, const void *q_proj, void *wkt, hipStream_t st) {
+  if (a.DH <= 32) prep_nj<T, NJ, 1>(a, q_proj, wkt, st);
+  else if (a.DH <= 64) prep_nj<T, NJ, 2>(a, q_proj, wkt, st);
+  else prep_nj<T, NJ, 4>(a, q_proj, wkt, st);
+}
+
 template <typename T, int NJ>
 void rowgemm_ks(const RowGemm &p, hipStream_t st) {
   if (p.K <= 32) rowgemm_nj<T, NJ, 1>(p, st);
@@ -609,13 +691,27 @@ void launch_rowgemm(const RowGemm &p, hipStream_t st) {
 bool wgrad16_supported(int F, bool dq) { return F >= 8 && F % 8 == 0 && (F <= 512 || !dq); }
 int wgrad16_slices(int F) { return F <= 512 ? 1 : (F + 255) / 256; }
 
+// D_H <= 128 (the folded shapes); at least one token.
+template <typename T>
+void launch_absorb_prep(const AbsorbArgs &a, const void *q_proj, void *wkt, hipStream_t st) {
+  const int64_t tiles = (a.T_q + kRgTok - 1) / kRgTok * a.H;
+  auto wgs = [&](int jb) { return 2 * tiles * ((a.F + jb - 1) / jb); };
+  if (wgs(256) >= 1024) prep_ks<T, 4>(a, q_proj, wkt, st);
+  else if (wgs(128) >= 1024) prep_ks<T, 2>(a, q_proj, wkt, st);
+  else prep_ks<T, 1>(a, q_proj, wkt, st);
+}
+
 template <typename T>
 void launch_wgrad16(const Wgrad &p, hipStream_t st) {
   if (p.F <= 64) wgrad_fp<T, 64>(p, st);
   else if (p.F <= 128) wgrad_fp<T, 128>(p, st);
   else if (p.F > 256 && p.F <= 512) wgrad_fp<T, 512>(p, st);
   else wgrad_fp<T, 256>(p, st);
-  launch_chunk_sum<T>(p.part, p.out, (int64_t)p.F * p.G * p.DH, p.n_chunks, st);
+  const ChunkSum sum{p.part, p.out, (int64_t)p.F * p.G * p.DH, p.n_chunks};
+  if (p.sums != nullptr)
+    p.sums->add(sum);
+  else
+    launch_chunk_sum<T>(sum.part, sum.out, sum.n_out, sum.n_chunks, st);
 }
 
 template <typename T>
@@ -628,6 +724,8 @@ void launch_transpose2d(const void *src, void *dst, int R, int C, hipStream_t st
 
 template void launch_rowgemm<bf16>(const RowGemm &, hipStream_t);
 template void launch_rowgemm<f16>(const RowGemm &, hipStream_t);
+template void launch_absorb_prep<bf16>(const AbsorbArgs &, const void *, void *, hipStream_t);
+template void launch_absorb_prep<f16>(const AbsorbArgs &, const void *, void *, hipStream_t);
 template void launch_wgrad16<bf16>(const Wgrad &, hipStream_t);
 template void launch_wgrad16<f16>(const Wgrad &, hipStream_t);
 template void launch_transpose2d<bf16>(const void *, void *, int, int, hipStream_t);

@@ -357,6 +357,23 @@ void absorb_fwd_all(const AbsorbArgs &a, hipStream_t st) {
                         a.comb_rows, st);
 }
 
+// du, aX and dX on the 16-bit matrix cores, from u, dAX and delta.
+template <typename T>
+void mfma_absorb_du_dx(const AbsorbArgs &a, hipStream_t st) {
+  AbsorbArgs r = a;  // what the merged kernel leaves to the du and dX kernels
+  const bool all = a.n_merged == a.n_qseg;
+  if (a.n_merged > 0 && mfma_absorb_merged(a.F) && (all || a.T_k > kAbsorbMergedKeys)) {
+    launch_mfma_absorb_bwd_merged<T>(a, st);
+    r.qseg_items = a.qseg_items + a.n_merged * VAFA_ITEM_INTS;
+    r.n_qseg = a.n_qseg - a.n_merged;
+    r.kv_items = a.kv_items + a.n_kv_res * VAFA_ITEM_INTS;
+    r.n_kv = a.n_kv - a.n_kv_res;
+    r.n_kv_res = 0;
+  }
+  launch_mfma_absorb_du<T>(r, st);
+  launch_mfma_absorb_dx<T>(r, st);
+}
+
 template <typename T>
 void absorb_bwd_all(const AbsorbArgs &a, hipStream_t st) {
   bool mfma = false;
@@ -372,20 +389,7 @@ void absorb_bwd_all(const AbsorbArgs &a, hipStream_t st) {
       launch_absorb_dax<T>(a, st);
   }
   if (mfma) {
-    if constexpr (sizeof(T) == 2) {
-      AbsorbArgs r = a;  // what the merged kernel leaves to the du and dX kernels
-      const bool all = a.n_merged == a.n_qseg;
-      if (a.n_merged > 0 && mfma_absorb_merged(a.F) && (all || a.T_k > kAbsorbMergedKeys)) {
-        launch_mfma_absorb_bwd_merged<T>(a, st);
-        r.qseg_items = a.qseg_items + a.n_merged * VAFA_ITEM_INTS;
-        r.n_qseg = a.n_qseg - a.n_merged;
-        r.kv_items = a.kv_items + a.n_kv_res * VAFA_ITEM_INTS;
-        r.n_kv = a.n_kv - a.n_kv_res;
-        r.n_kv_res = 0;
-      }
-      launch_mfma_absorb_du<T>(r, st);
-      launch_mfma_absorb_dx<T>(r, st);
-    }
+    if constexpr (sizeof(T) == 2) mfma_absorb_du_dx<T>(a, st);
   } else if (sizeof(T) == 4 && f32_absorb_supported(a.H, a.F, a.DH)) {
     launch_f32_absorb_du_dx(a, st);
   } else {
@@ -503,12 +507,13 @@ struct ProjectWs {
   void *wt = nullptr;      // W_Q^T [HD, D_Q] (forward) or W_K^T [HD, D_KV] (backward)
   void *dq_proj = nullptr; // [T_q, HD]
   float *part = nullptr;   // weight-gradient chunk partials
+  float *part_q = nullptr; // dW_Q's own, where both are summed in one launch
   Chunks ck, cq;           // chunks of dW_K and dW_Q
   int64_t bytes = 0;
 };
 
 ProjectWs carve_project(void *ws, int64_t T_q, int64_t H, int64_t D_Q, int64_t D_KV, int64_t D_H,
-                        bool bwd, bool f32) {
+                        bool bwd, bool f32, bool both = false) {
   Carver c(ws);
   ProjectWs w;
   const int64_t HD = H * D_H;
@@ -518,7 +523,8 @@ ProjectWs carve_project(void *ws, int64_t T_q, int64_t H, int64_t D_Q, int64_t D
     w.ck = wgrad_chunks(T_q, D_KV, H * ((D_H + 31) / 32), true, f32);
     w.cq = wgrad_chunks(T_q, D_Q, (HD + 31) / 32 * wgrad16_slices((int)D_Q), false, f32);
     const int64_t pk = w.ck.n * D_KV * HD, pq = w.cq.n * D_Q * HD;
-    w.part = c.take<float>((pk > pq ? pk : pq) * 4 + 4);
+    w.part = c.take<float>((both || pk > pq ? pk : pq) * 4 + 4);
+    if (both) w.part_q = c.take<float>(pq * 4 + 4);
   }
   w.bytes = c.used;
   return w;
@@ -537,17 +543,17 @@ void project_fwd(const void *q_raw, const void *W_Q, const void *W_K, void *q_pr
 template <typename T>
 void project_bwd(const void *q_raw, const void *W_Q, const void *W_K, const void *q_proj,
                  const void *du, void *dq_raw, void *dW_Q, void *dW_K, int64_t T_q, int H, int DQ,
-                 int F, int DH, const ProjectWs &w, hipStream_t st) {
+                 int F, int DH, const ProjectWs &w, ChunkSums *sums, hipStream_t st) {
   const int HD = H * DH;
   const bool need_dq = dq_raw != nullptr || dW_Q != nullptr;
-  // W_K^T [HD, F]: the dq_proj product's weight rows
-  if (need_dq) launch_transpose2d<T>(W_K, w.wt, F, HD, st);
+  // W_K^T [HD, F]: the dq_proj product's weight rows (with `sums`, already there)
+  if (need_dq && sums == nullptr) launch_transpose2d<T>(W_K, w.wt, F, HD, st);
   // dW_K[f, h, d] = sum_t du[t, h, f] q_proj[t, h, d], and on the 16-bit
   // kernel dq_proj[t, h, d] = sum_f du[t, h, f] W_K[f, h, d] from the same du reads
   const bool fused = wgrad16_supported(F, true) && dW_K != nullptr;
   if (fused) {
     launch_wgrad16<T>(Wgrad{du, q_proj, w.wt, need_dq ? w.dq_proj : nullptr, dW_K, w.part, T_q,
-                            w.ck.tchunk, w.ck.n, H, F, DH}, st);
+                            w.ck.tchunk, w.ck.n, H, F, DH, sums}, st);
   } else if (dW_K != nullptr) {
     launch_wgrad<T, T>(du, q_proj, w.part, dW_K, T_q, w.ck.tchunk, w.ck.n, H, F, DH, st);
   }
@@ -558,12 +564,38 @@ void project_bwd(const void *q_raw, const void *W_Q, const void *W_K, const void
   if (dq_raw != nullptr)  // dq_raw [T, DQ] = dq_proj [T, HD] . W_Q [DQ, HD]^T
     launch_rowgemm<T>(RowGemm{w.dq_proj, W_Q, dq_raw, T_q, 1, DQ, HD, HD, 0, 0, HD, DQ, 0}, st);
   if (dW_Q != nullptr) {  // dW_Q[c, hd] = sum_t q_raw[t, c] dq_proj[t, hd]
+    float *part = sums != nullptr ? w.part_q : w.part;
     if (wgrad16_supported(DQ, false))
-      launch_wgrad16<T>(Wgrad{q_raw, w.dq_proj, nullptr, nullptr, dW_Q, w.part, T_q, w.cq.tchunk,
-                              w.cq.n, 1, DQ, HD}, st);
+      launch_wgrad16<T>(Wgrad{q_raw, w.dq_proj, nullptr, nullptr, dW_Q, part, T_q, w.cq.tchunk,
+                              w.cq.n, 1, DQ, HD, sums}, st);
     else
-      launch_wgrad<T, T>(q_raw, w.dq_proj, w.part, dW_Q, T_q, w.cq.tchunk, w.cq.n, 1, DQ, HD, st);
+      launch_wgrad<T, T>(q_raw, w.dq_proj, part, dW_Q, T_q, w.cq.tchunk, w.cq.n, 1, DQ, HD, st);
   }
+}
+
+// Backward of the whole op on a folded shape (16-bit, D_KV <= 256): u, dAX,
+// delta and W_K^T in one launch, the three weight gradients' chunk sums in
+// another.  A plan that covers no token or fewer than the tensors (possible
+// only where validation is off) takes the separate passes.
+template <typename T>
+void absorb_bwd_full(AbsorbArgs a, const void *q_raw, const void *W_Q, const void *q_proj,
+                     void *dq_raw, void *dW_Q, void *dW_K, int64_t T_qp, int DQ,
+                     const ProjectWs &w, hipStream_t st) {
+  ChunkSums sums;
+  const bool one = a.T_q > 0 && a.T_q == T_qp;
+  if (one) {
+    a.sums = &sums;
+    launch_absorb_prep<T>(a, q_proj, dq_raw != nullptr || dW_Q != nullptr ? w.wt : nullptr, st);
+    mfma_absorb_du_dx<T>(a, st);
+    launch_absorb_dwv<T>(a, st);
+  } else {
+    project_u<T>(q_proj, a.wk, a.u_out, T_qp, a.H, a.F, a.DH, st);
+    absorb_bwd_all<T>(a, st);
+  }
+  if (dq_raw != nullptr || dW_Q != nullptr || dW_K != nullptr)
+    project_bwd<T>(q_raw, W_Q, a.wk, q_proj, a.du, dq_raw, dW_Q, dW_K, T_qp, a.H, DQ, a.F, a.DH,
+                   w, one ? &sums : nullptr, st);
+  if (one) launch_chunk_sums<T>(sums, st);
 }
 
 // The same products on fp32 operands (weights read in place).
@@ -973,11 +1005,11 @@ int vafa_absorb_project_bwd(const void *q_raw, const void *W_Q, const void *W_K,
   switch (dtype) {
     case VAFA_BF16:
       project_bwd<bf16>(q_raw, W_Q, W_K, q_proj, du, dq_raw, dW_Q, dW_K, T_q, (int)H, (int)D_Q,
-                        (int)D_KV, (int)D_H, w, st);
+                        (int)D_KV, (int)D_H, w, nullptr, st);
       break;
     case VAFA_F16:
       project_bwd<f16>(q_raw, W_Q, W_K, q_proj, du, dq_raw, dW_Q, dW_K, T_q, (int)H, (int)D_Q,
-                       (int)D_KV, (int)D_H, w, st);
+                       (int)D_KV, (int)D_H, w, nullptr, st);
       break;
     default:
       return fail(VAFA_ERR_VALUE, "project_bwd: 16-bit dtypes only (got %d)", (int)dtype);
@@ -1019,6 +1051,32 @@ int vafa_absorb_project_f32_bwd(const float *q_raw, const float *W_Q, const floa
   return check_launch("vafa_absorb_project_f32_bwd");
 }
 
+static AbsorbArgs bwd_args(const void *u, const void *X, const void *W_V, const void *O,
+                           const void *dO, const float *lse, void *du, void *dX, void *dW_V,
+                           const int32_t *plan_dev, const vafa_plan_info *info, int64_t D_KV,
+                           int64_t D_H, float scale, const AbsorbWs &w) {
+  AbsorbArgs a{};
+  a.u = u; a.X = X; a.wv = W_V; a.O_in = O; a.dO = dO; a.lse_in = lse;
+  a.du = du; a.dX = dX; a.dwv = dW_V;
+  a.delta = w.delta; a.dax = w.dax; a.ax = w.ax; a.dwv_part = w.dwv_part;
+  a.n_tchunks = w.n_tchunks; a.tchunk = w.tchunk;
+  a.part_du = w.part_du; a.part_ax = w.part_ax;
+  a.qtc_items = plan_dev + info->off_dqc; a.n_qtc = info->n_dqc;
+  a.qtc_rows = (int)info->max_dqc_rows;
+  a.items = plan_dev + info->off_fwd; a.n_items = info->n_fwd;
+  a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
+  a.comb_rows = (int)info->max_comb_rows;
+  a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
+  a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
+  if (info->n_dq > 0) {  // the du pass's own items (split key ranges, merged tiles first)
+    a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
+    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv;
+  }
+  a.T_q = info->T_q; a.T_k = info->T_k;
+  a.H = (int)info->H; a.F = (int)D_KV; a.DH = (int)D_H; a.scale = scale;
+  return a;
+}
+
 int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O,
                     const void *dO, const float *lse, void *du, void *dX, void *dW_V,
                     const int32_t *plan_dev, const vafa_plan_info *info, int64_t D_KV,
@@ -1036,9 +1094,7 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
     return fail(VAFA_ERR_WORKSPACE, "workspace of %lld bytes, %lld needed",
                 (long long)workspace_bytes, (long long)w.bytes);
   const hipStream_t st = (hipStream_t)stream;
-  AbsorbArgs a{};
-  a.u = u; a.X = X; a.wv = W_V; a.O_in = O; a.dO = dO; a.lse_in = lse;
-  a.du = du; a.dX = dX; a.dwv = dW_V;
+  AbsorbArgs a = bwd_args(u, X, W_V, O, dO, lse, du, dX, dW_V, plan_dev, info, D_KV, D_H, scale, w);
   const bool pad = absorb_pad(info->H, D_KV, D_H, dtype, true);
   const int64_t F = pad ? absorb_fpad(D_KV) : D_KV;
   const int eb = elem_bytes(dtype);
@@ -1048,23 +1104,8 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
     launch_pad_cols(W_V, w.pW, 1, D_KV * info->H * D_H, F * info->H * D_H, eb, st);
     a.u = w.pu; a.X = w.pX; a.wv = w.pW;
     a.du = w.pdu; a.dX = w.pdX; a.dwv = w.pdW;
+    a.F = (int)F;
   }
-  a.delta = w.delta; a.dax = w.dax; a.ax = w.ax; a.dwv_part = w.dwv_part;
-  a.n_tchunks = w.n_tchunks; a.tchunk = w.tchunk;
-  a.part_du = w.part_du; a.part_ax = w.part_ax;
-  a.qtc_items = plan_dev + info->off_dqc; a.n_qtc = info->n_dqc;
-  a.qtc_rows = (int)info->max_dqc_rows;
-  a.items = plan_dev + info->off_fwd; a.n_items = info->n_fwd;
-  a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
-  a.comb_rows = (int)info->max_comb_rows;
-  a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
-  a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
-  if (info->n_dq > 0) {  // the du pass's own items (split key ranges, merged tiles first)
-    a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
-    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv;
-  }
-  a.T_q = info->T_q; a.T_k = info->T_k;
-  a.H = (int)info->H; a.F = (int)F; a.DH = (int)D_H; a.scale = scale;
   if (int rc = by_dtype<ABwd>(dtype, a, st)) return rc;
   if (pad) {
     launch_unpad_cols(w.pdu, du, info->T_q * info->H, D_KV, F, eb, st);
@@ -1072,6 +1113,71 @@ int vafa_absorb_bwd(const void *u, const void *X, const void *W_V, const void *O
     launch_unpad_cols(w.pdW, dW_V, 1, D_KV * info->H * D_H, F * info->H * D_H, eb, st);
   }
   return check_launch("vafa_absorb_bwd");
+}
+
+// Workspace of the whole backward: u, du, then the two parts'.
+struct FullBwdWs {
+  void *u = nullptr, *du = nullptr;
+  AbsorbWs a;
+  ProjectWs p;
+  int64_t bytes = 0;
+};
+static FullBwdWs carve_full_bwd(void *ws, const vafa_plan_info *info, int64_t T_q, int64_t D_Q,
+                                int64_t D_KV, int64_t D_H) {
+  Carver c(ws);
+  FullBwdWs w;
+  const int64_t rows = (T_q > info->T_q ? T_q : info->T_q) * info->H * D_KV * 2;
+  w.u = c.take<void>(rows);
+  w.du = c.take<void>(rows);
+  auto rest = [&]() { return ws ? static_cast<char *>(ws) + c.used : nullptr; };
+  w.a = carve_absorb(rest(), info, D_KV, D_H, true);
+  c.used += w.a.bytes;
+  w.p = carve_project(rest(), T_q, info->H, D_Q, D_KV, D_H, true, false, true);
+  w.bytes = c.used + w.p.bytes;
+  return w;
+}
+
+int64_t vafa_absorb_bwd_full_workspace(const vafa_plan_info *info, int64_t T_q, int64_t D_Q,
+                                       int64_t D_KV, int64_t D_H) {
+  if (check_info(info, 2)) return -1;
+  if (check_project_dims("bwd_full_workspace", T_q, info->H, D_Q, D_KV, D_H)) return -1;
+  return carve_full_bwd(nullptr, info, T_q, D_Q, D_KV, D_H).bytes;
+}
+
+int vafa_absorb_bwd_full(const void *q_raw, const void *X, const void *W_Q, const void *W_K,
+                         const void *W_V, const void *q_proj, const void *O, const void *dO,
+                         const float *lse, void *dq_raw, void *dX, void *dW_Q, void *dW_K,
+                         void *dW_V, int64_t T_q, const int32_t *plan_dev,
+                         const vafa_plan_info *info, int64_t D_Q, int64_t D_KV, int64_t D_H,
+                         int32_t dtype, float scale, void *workspace, int64_t workspace_bytes,
+                         void *stream) {
+  if (int rc = check_info(info, 2)) return rc;
+  if (int rc = check_absorb_dims(D_KV, D_H)) return rc;
+  if (int rc = check_project_dims("absorb_bwd_full", T_q, info->H, D_Q, D_KV, D_H)) return rc;
+  if (info->T_q > T_q || info->n_fkv < 0 || info->n_fkv > info->n_dq)
+    return fail(VAFA_ERR_VALUE, "absorb_bwd_full: plan of %lld query tokens for %lld",
+                (long long)info->T_q, (long long)T_q);
+  if (!fold_supported(info->H, D_KV, D_H, dtype))
+    return fail(VAFA_ERR_VALUE,
+                "absorb_bwd_full: H=%lld, D_KV=%lld, D_H=%lld, dtype %d is not a shape of the "
+                "folded kernel (vafa_absorb_fold_supported)",
+                (long long)info->H, (long long)D_KV, (long long)D_H, (int)dtype);
+  if (int rc = check_aligned("absorb_bwd_full", {q_raw, X, W_Q, W_K, W_V, q_proj, O, dO, dq_raw,
+                                                 dX, dW_Q, dW_K, dW_V, workspace}))
+    return rc;
+  const FullBwdWs w = carve_full_bwd(workspace, info, T_q, D_Q, D_KV, D_H);
+  if (workspace == nullptr || workspace_bytes < w.bytes)
+    return fail(VAFA_ERR_WORKSPACE, "workspace of %lld bytes, %lld needed",
+                (long long)workspace_bytes, (long long)w.bytes);
+  AbsorbArgs a = bwd_args(w.u, X, W_V, O, dO, lse, w.du, dX, dW_V, plan_dev, info, D_KV, D_H,
+                          scale, w.a);
+  a.u_out = w.u; a.wk = W_K;
+  const hipStream_t st = (hipStream_t)stream;
+  if (dtype == VAFA_BF16)
+    absorb_bwd_full<bf16>(a, q_raw, W_Q, q_proj, dq_raw, dW_Q, dW_K, T_q, (int)D_Q, w.p, st);
+  else
+    absorb_bwd_full<f16>(a, q_raw, W_Q, q_proj, dq_raw, dW_Q, dW_K, T_q, (int)D_Q, w.p, st);
+  return check_launch("vafa_absorb_bwd_full");
 }
 
 }  // extern "C"

@@ -43,6 +43,19 @@ struct VarlenArgs {
   float *part_fq;  // fused dQ partial rows [n_fpart_rows, H, D] fp32
 };
 
+// Chunk partials of a weight gradient, out[o] = sum_c part[c * n_out + o]; a
+// caller that runs several collects them for one launch.
+struct ChunkSum {
+  const float *part;
+  void *out;
+  int64_t n_out, n_chunks;
+};
+struct ChunkSums {
+  ChunkSum v[3];
+  int n = 0;
+  void add(const ChunkSum &s) { v[n++] = s; }
+};
+
 struct AbsorbArgs {
   const void *u, *X, *wv, *O_in, *dO;
   void *O, *du, *dX, *dwv;
@@ -52,6 +65,8 @@ struct AbsorbArgs {
   float *part_o, *part_lse;   // split partial rows [rows, H, D_H] / [rows, H]
   void *dax;                  // dO W_V^T [T_q, H, F] in the input dtype (backward)
   float *ax;                  // aX [T_q, H, F] fp32 (backward, for dW_V)
+  void *u_out;                // whole op's backward: u, formed from q_proj
+  ChunkSums *sums;            // where to leave dW_V's chunk sum, or null: summed at once
   float *dwv_part;            // [n_tchunks, F, H, D_H] fp32 (backward)
   float *part_du, *part_ax;   // du / aX partials of split token tiles [rows, H, F] fp32
   void *wvt;                  // W_V re-laid out as [H, D_H, F padded to 32] (forward)
@@ -139,6 +154,8 @@ void launch_unpad_cols(const void *src, void *dst, int64_t rows, int64_t n, int6
 // out[o] = sum_c part[c * n_out + o] in chunk order, rounded to T
 template <typename T>
 void launch_chunk_sum(const float *part, void *out, int64_t n_out, int64_t n_chunks, hipStream_t);
+template <typename T>
+void launch_chunk_sums(const ChunkSums &, hipStream_t);  // all of them in one launch
 // du (rounded to T) and aX of the du pass's split token tiles: ordered sums of
 // their key chunks' fp32 partials (F % 4 == 0)
 template <typename T>
@@ -187,9 +204,13 @@ struct Wgrad {
   float *part;
   int64_t T_q, tchunk, n_chunks;
   int G, F, DH;
+  ChunkSums *sums;  // where to leave the chunk sum, or null: summed at once
 };
 bool wgrad16_supported(int F, bool dq);
 int wgrad16_slices(int F);  // column slices of A, each a workgroup of its own
+// u, dAX, delta and W_K^T (wkt, unless null) of the whole op's backward, one launch
+template <typename T>
+void launch_absorb_prep(const AbsorbArgs &, const void *q_proj, void *wkt, hipStream_t);
 template <typename T> void launch_wgrad16(const Wgrad &, hipStream_t);
 template <typename T> void launch_rowgemm(const RowGemm &, hipStream_t);
 // RowGemm on fp32 operands and fp32 matrix cores, any widths; kj: W is

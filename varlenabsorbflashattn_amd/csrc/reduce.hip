@@ -452,13 +452,12 @@ __global__ __launch_bounds__(256) void absorb_dwv_lds_kernel(
     }
 }
 
+// One output of a chunk sum: chunk order kept, eight independent loads in
+// flight per batch.
 template <typename T>
-__global__ __launch_bounds__(256) void absorb_dwv_sum_kernel(const float *__restrict__ part,
-                                                             T *__restrict__ dwv, int64_t n_out,
-                                                             int64_t n_chunks) {
-  const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void chunk_sum(const float *__restrict__ part, T *__restrict__ out,
+                                          int64_t n_out, int64_t n_chunks, int64_t o) {
   if (o >= n_out) return;
-  // chunk order kept; eight independent loads in flight per batch
   constexpr int kB = 8;
   float s = 0.f;
   for (int64_t c0 = 0; c0 < n_chunks; c0 += kB) {
@@ -468,7 +467,22 @@ __global__ __launch_bounds__(256) void absorb_dwv_sum_kernel(const float *__rest
 #pragma unroll
     for (int i = 0; i < kB; ++i) s += v[i];
   }
-  dwv[o] = from_f<T>(s);
+  out[o] = from_f<T>(s);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void absorb_dwv_sum_kernel(const float *__restrict__ part,
+                                                             T *__restrict__ dwv, int64_t n_out,
+                                                             int64_t n_chunks) {
+  chunk_sum<T>(part, dwv, n_out, n_chunks, (int64_t)blockIdx.x * 256 + threadIdx.x);
+}
+
+// Up to three weight gradients' sums (blockIdx.y) in one launch: three of 16 MB
+// of partials each take 8.9 us so, 17 one after the other.
+template <typename T>
+__global__ __launch_bounds__(256) void chunk_sums_kernel(ChunkSums s) {
+  const ChunkSum &c = blockIdx.y == 0 ? s.v[0] : (blockIdx.y == 1 ? s.v[1] : s.v[2]);
+  chunk_sum<T>(c.part, (T *)c.out, c.n_out, c.n_chunks, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 // [rows, 16] -> [rows, 32] with zero columns 16..31, and back: D=16 runs on
@@ -596,6 +610,14 @@ void launch_chunk_sum(const float *part, void *out, int64_t n_out, int64_t n_chu
                      (T *)out, n_out, n_chunks);
 }
 
+template <typename T>
+void launch_chunk_sums(const ChunkSums &s, hipStream_t st) {
+  int64_t n = 0;
+  for (int i = 0; i < s.n; ++i) n = n > s.v[i].n_out ? n : s.v[i].n_out;
+  if (n == 0) return;
+  hipLaunchKernelGGL(chunk_sums_kernel<T>, dim3(blocks_for(n), (unsigned)s.n), dim3(256), 0, st, s);
+}
+
 template <typename T, int FP>
 void dwv_lds(const AbsorbArgs &a, hipStream_t st) {
   const int n_db = (a.DH + 31) / 32;
@@ -606,7 +628,11 @@ void dwv_lds(const AbsorbArgs &a, hipStream_t st) {
     hipLaunchKernelGGL((absorb_dwv_lds_kernel<T, FP>), dim3((unsigned)wgs), dim3(256), smem, st,
                        a.ax, (const T *)a.dO, a.dwv_part, a.T_q, a.tchunk, a.H, a.F, a.DH, n_db);
   }
-  launch_chunk_sum<T>(a.dwv_part, a.dwv, (int64_t)a.F * a.H * a.DH, a.n_tchunks, st);
+  const ChunkSum sum{a.dwv_part, a.dwv, (int64_t)a.F * a.H * a.DH, a.n_tchunks};
+  if (a.sums != nullptr)
+    a.sums->add(sum);
+  else
+    launch_chunk_sum<T>(sum.part, sum.out, sum.n_out, sum.n_chunks, st);
 }
 
 // dW_V: the LDS-tiled kernel for 16-bit dO and D_KV <= 256 (a multiple of
@@ -673,6 +699,7 @@ void launch_unpad16(const void *src, void *dst, int64_t rows, int elem_bytes, hi
   template void launch_absorb_dwv<T>(const AbsorbArgs &, hipStream_t);                      \
   template void launch_wgrad<T, T>(const void *, const void *, float *, void *, int64_t,    \
                                    int64_t, int64_t, int, int, int, hipStream_t);           \
+  template void launch_chunk_sums<T>(const ChunkSums &, hipStream_t);                       \
   template void launch_chunk_sum<T>(const float *, void *, int64_t, int64_t, hipStream_t);
 VAFA_INST(float)
 VAFA_INST(f16)

@@ -27,7 +27,8 @@ struct Api {
 #define VAFA_FNS(X)                                                                       \
   X(last_error) X(varlen_fwd_workspace) X(varlen_fwd) X(varlen_bwd_workspace)             \
   X(varlen_bwd) X(absorb_fwd_workspace) X(absorb_fwd) X(absorb_bwd_workspace)             \
-  X(absorb_bwd) X(absorb_fwd_full_workspace) X(absorb_fwd_full) X(absorb_project_u)       \
+  X(absorb_bwd) X(absorb_fwd_full_workspace) X(absorb_fwd_full) X(absorb_bwd_full)        \
+  X(absorb_bwd_full_workspace)                                                            \
   X(absorb_project_workspace) X(absorb_project_fwd) X(absorb_project_bwd)                 \
   X(absorb_project_f32_workspace) X(absorb_project_f32_fwd) X(absorb_project_f32_bwd)
   VAFA_FNS(VAFA_FN)
@@ -221,22 +222,26 @@ Grads3 project_bwd(const Tensor &q_raw, const Tensor &W_Q, const Tensor &W_K, co
   return {opt(dq), opt(dwq), opt(dwk)};
 }
 
-// Backward of the whole 16-bit op: u from the saved q_proj, the inner
-// backward, the projection backward: (dq_raw, dX, dW_Q, dW_K, dW_V).
+// Backward of the whole 16-bit op: (dq_raw, dX, dW_Q, dW_K, dW_V).
 std::tuple<std::optional<Tensor>, Tensor, std::optional<Tensor>, std::optional<Tensor>, Tensor>
 absorb_full_bwd(const Tensor &q_raw, const Tensor &W_Q, const Tensor &W_K, const Tensor &q_proj,
                 const Tensor &X, const Tensor &W_V, const Tensor &O, const Tensor &lse,
                 const Tensor &g, const Plan &p, double scale, bool need_q, bool need_wq,
                 bool need_wk) {
-  const int64_t T_q = q_raw.size(0), H = W_Q.size(1), DH = W_Q.size(2), F = X.size(1);
   Call c(q_raw);
-  Tensor u = c.empty({T_q, H, F});
-  check(api.absorb_project_u(ptr(q_proj), ptr(W_K), ptr(u), T_q, H, F, DH, dtype_of(u), c.stream));
-  auto [du, dX, dW_V] = absorb_bwd(u, X, W_V, O, lse, g, p, scale);
-  Grads3 pr;
-  if (need_q || need_wq || need_wk)
-    pr = project_bwd(q_raw, W_Q, W_K, q_proj, du, need_q, need_wq, need_wk);
-  return {std::get<0>(pr), dX, std::get<1>(pr), std::get<2>(pr), dW_V};
+  const int64_t T_q = q_raw.size(0), DQ = q_raw.size(1), F = X.size(1), DH = W_Q.size(2);
+  const Tensor dO = grad_in(g, q_raw);
+  Tensor dX = c.like(X), dW_V = c.like(W_V), dq, dwq, dwk;
+  if (need_q) dq = c.like(q_raw);
+  if (need_wq) dwq = c.like(W_Q);
+  if (need_wk) dwk = c.like(W_K);
+  void *ws = c.workspace(api.absorb_bwd_full_workspace(&p.info, T_q, DQ, F, DH));
+  check(api.absorb_bwd_full(ptr(q_raw), ptr(X), ptr(W_Q), ptr(W_K), ptr(W_V), ptr(q_proj), ptr(O),
+                            ptr(dO), f32(lse), ptr(dq), ptr(dX), ptr(dwq), ptr(dwk), ptr(dW_V),
+                            T_q, p.dev(), &p.info, DQ, F, DH, dtype_of(q_raw), (float)scale, ws,
+                            c.ws_bytes(), c.stream));
+  auto opt = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
+  return {opt(dq), dX, opt(dwq), opt(dwk), dW_V};
 }
 
 }  // namespace
