@@ -270,7 +270,7 @@ def _fold_shape(H: int, d_kv: int, D_H: int, dtype: torch.dtype) -> bool:
 
 def _fold_native(q_raw, X, W_Q, W_K, W_V) -> bool:
     """Whether packed_target_attn can run with u folded into the attention
-    kernel (vafa_absorb_fwd_fold): the native projection's operands, X and
+    kernel (vafa_absorb_fwd_full): the native projection's operands, X and
     W_V of the same dtype on the same device, and a shape of the folded
     matrix-core kernel."""
     if q_raw.dtype == torch.float32 or not _project_native(q_raw, W_Q, W_K):
@@ -291,9 +291,9 @@ class _FoldedTargetAttn(torch.autograd.Function):
     rounded to the input dtype), then the attention, whose workgroups form
     u = q_proj_h W_K,h^T for their own rows on the matrix cores -- u is never
     written to memory.
-    Backward: u is formed once from the saved q_proj (vafa_absorb_project_u,
-    the same products), then the inner backward gives du / dX / dW_V and the
-    projection backward dq_raw / dW_Q / dW_K, as the unfused path."""
+    Backward (vafa_absorb_bwd_full): u is formed once from the saved q_proj,
+    in one launch with dAX and delta, then the inner backward gives du / dX /
+    dW_V and the projection backward dq_raw / dW_Q / dW_K, as the unfused path."""
 
     @staticmethod
     def forward(ctx, q_raw, X, W_Q, W_K, W_V, cu_seqlens_q, cu_seqlens_k, scale,
