@@ -183,6 +183,20 @@ def test_absorb_merged_backward(device, H, d_kv, dtype):
         assert_close(n, a, r)
 
 
+# fp32 du pass: tiles of at most 32 rows, whose key tiles two waves share (rows at
+# the 16-row groups' edges and at the line, key counts at the 16-key tiles' and tile
+# pairs' edges), and tiles above it; whole and split key ranges, every width class.
+@pytest.mark.parametrize("H,d_kv", [(1, 40), (1, 128), (2, 192), (4, 216), (8, 256), (4, 384)])
+def test_absorb_f32_shared_key_tiles(device, H, d_kv):
+    rows = [1, 15, 16, 17, 31, 32, 33, 64, 32, 16, 32, 0, 32, 8, 80]
+    k_lens = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 65, 9, 700, 300, 129]
+    q_lens = [-(-r // H) for r in rows]
+    print(f"[absorb f32 shared tiles] H={H} d_kv={d_kv}", flush=True)
+    got, ref = run_case(q_lens, k_lens, torch.float32, device, d_q=64, d_kv=d_kv, H=H, D_H=32)
+    for n, a, r in zip(NAMES, got, ref):
+        assert_close(n, a, r)
+
+
 def test_absorb_merged_beside_streamed(device):
     """A launch of more than 384k keys whose segments lie on both sides of 64
     rows: merged items, and the du and dX kernels for the rest.  The keys of
