@@ -312,7 +312,8 @@ __global__ __launch_bounds__(256, FP > 256 ? 1 : 2) void absorb_fwd_f32_kernel(
 // second key tile of the same rows, their sums added through LDS at the end.
 // 512 samples of 1 to 8 tokens of 8 heads (157k keys, D_KV = 256), forward +
 // backward: 783 -> 710 us; before, head-major rows left every wave half empty on
-// those tiles and this kernel took 251 us.
+// those tiles and this kernel took 251 us.  2048 samples at D_KV = 512 6.91 -> 5.41
+// ms (57 spilled registers less), 16 heads of 16 3.27 -> 2.84 ms.
 // ---------------------------------------------------------------------------
 template <int FP>
 __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
