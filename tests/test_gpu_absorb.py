@@ -197,6 +197,48 @@ def test_absorb_f32_shared_key_tiles(device, H, d_kv):
         assert_close(n, a, r)
 
 
+# fp16 gradients of small magnitude through the one-kernel backward.  It rounds
+# dS = P (dP - delta) to fp16 without the scale, so an element's rounding error is
+# that of dS itself, uniform within an ulp (2^-24 in the subnormal range that small
+# upstream gradients reach); du sums them times scale * X.  Bound: twice the rms
+# that these errors, du's own rounding and 2^-10 for the rounded P and dAX predict.
+# Rounded after the scale (1/8 to 1/16), du would be 2 to 9 times past it.
+@pytest.mark.parametrize("m", [1.0, 1e-2, 1e-3])
+@pytest.mark.parametrize("H,D_H,d_kv,k_lens", [(8, 64, 256, [2000, 300]), (4, 256, 128, [4000])])
+def test_absorb_merged_small_fp16_gradients(device, H, D_H, d_kv, k_lens, m):
+    q_lens = [64 // H] * len(k_lens)
+    print(f"[absorb merged fp16] H={H} D_H={D_H} d_kv={d_kv} m={m}", flush=True)
+    g = torch.Generator().manual_seed(11)
+    T_q, T_k, scale = sum(q_lens), sum(k_lens), 1.0 / math.sqrt(D_H)
+    mk = lambda std, *s: (torch.randn(*s, generator=g) * std).half()
+    u, X = mk(1.0, T_q, H, d_kv), mk(1.0, T_k, d_kv)
+    W_V, dO = mk(math.sqrt(2.0 / (d_kv + H * D_H)), d_kv, H, D_H), mk(m, T_q, H, D_H)
+    cq, ck = cu_from_lens(q_lens), cu_from_lens(k_lens)
+    dev = [t.to(device).requires_grad_(True) for t in (u, X, W_V)]
+    O = target_attn_inner(*dev, cq.to(device), ck.to(device))
+    du = torch.autograd.grad(O, dev[0], dO.to(device))[0].cpu().double().numpy()
+
+    def ulp(x):
+        return np.exp2(np.maximum(np.floor(np.log2(np.abs(x) + 1e-30)), -14) - 10)
+
+    u, X, W_V, dO = (t.double().numpy() for t in (u, X, W_V, dO))
+    for s in range(len(q_lens)):
+        uu = u[cq[s]:cq[s + 1]].reshape(-1, d_kv)
+        x = X[ck[s]:ck[s + 1]]
+        dax = np.einsum("thd,fhd->thf", dO[cq[s]:cq[s + 1]], W_V).reshape(-1, d_kv)
+        P = np.exp(scale * (uu @ x.T))
+        P /= P.sum(1, keepdims=True)
+        dP = dax @ x.T
+        dS = P * (dP - (P * dP).sum(1, keepdims=True))
+        ref = scale * dS @ x
+        var = (scale ** 2 * (ulp(dS) ** 2 / 12) @ x ** 2 + ulp(ref) ** 2 / 12).mean()
+        bound = 2 * (math.sqrt(var) + 2.0 ** -10 * math.sqrt((ref ** 2).mean()))
+        err = math.sqrt(((du[cq[s]:cq[s + 1]].reshape(-1, d_kv) - ref) ** 2).mean())
+        print(f"  rms error {err:.3e}, bound {bound:.3e}, rms {math.sqrt((ref ** 2).mean()):.3e}",
+              flush=True)
+        assert err <= bound
+
+
 def test_absorb_merged_beside_streamed(device):
     """A launch of more than 384k keys whose segments lie on both sides of 64
     rows: merged items, and the du and dX kernels for the rest.  The keys of

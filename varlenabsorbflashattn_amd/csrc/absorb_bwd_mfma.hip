@@ -586,12 +586,15 @@ __global__ __launch_bounds__(64 * kDxWaves, FP > kMaxF ? 1 : 2) void absorb_dx_k
 // bytes at 4.3-4.6 TB/s, near a device copy's rate, so only a pass less makes
 // them faster.  One workgroup of 8 waves per CU (two per SIMD) holds a sample's
 // u and dAX rows in LDS, a 4-deep LDS-DMA ring of 32-key X tiles and two slots
-// of P and scale*dS, which the waves exchange so that each phase splits the way
-// it reads least:
+// of P and dS, which the waves exchange so that each phase splits the way it
+// reads least:
 //   A  wave (16 rows, 16 keys): S^T = X U^T, dP^T = X dAX^T (U^T / dAX^T
-//      fragments in registers), P and scale*dS rounded to T into the slot;
+//      fragments in registers), P and dS rounded to T into the slot;
 //   B  wave (32 features): du^T += X^T dS^T, aX^T += X^T P^T over all rows;
-//   C  wave (32 features): dX^T = dAX^T P + U^T (scale dS) over all rows, stored.
+//   C  wave (32 features): dX^T = dAX^T P + scale U^T dS over all rows, stored.
+// dS is rounded without the scale, which multiplies the fp32 sums, as in
+// absorb_du_kernel: scale * dS would lie 2 to 4 bits (D_H 16 to 256) nearer
+// fp16's subnormal range, where small upstream gradients lose bits.
 // Between two barriers a wave runs A of tile j+1, then B and C of tile j, so one
 // barrier per tile suffices.  Per 32-key tile and 64 rows 1536 cycles of
 // products per SIMD and 270 KB of LDS reads.  C4 (2048 samples, 648k keys, 853
@@ -734,7 +737,7 @@ __global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
       float p = fast_exp2(__builtin_fmaf(s[r], c, -L));
       if (kb + r >= k1) p = 0.f;
       pv[r] = static_cast<T>(p);
-      sv[r] = static_cast<T>(p * (dp[r] - dl) * scale);
+      sv[r] = static_cast<T>(p * (dp[r] - dl));
     }
     T *slot = ps + (j & 1) * 2 * S::kP + row * PS + lq * 8 + kh * 4;
     *reinterpret_cast<T4 *>(slot) = pv;
@@ -771,9 +774,9 @@ __global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
     load_c1(0);
     load_b(0);
     load_c2(0);
-    f32x16 acc;
+    f32x16 acc, accu;  // dAX^T P and U^T dS
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    for (int r = 0; r < 16; ++r) acc[r] = accu[r] = 0.f;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -787,10 +790,12 @@ __global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
       }
       if (g + 1 < NG) load_b(g + 1);
       __builtin_amdgcn_sched_barrier(0);
-      acc = M::mma(ou, od, acc);
+      accu = M::mma(ou, od, accu);
       if (g + 1 < NG) load_c2(g + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(accu[r], scale, acc[r]);
     // dX^T: element 4 g + e is feature 8 g + 4 lh + e of this lane's key; the
     // halves of a pair of g are swapped between lanes l and l + 32, so a lane
     // stores 8 features (16 bytes) of g = 2 i + lh and a row leaves as 2 x 32 bytes
@@ -865,12 +870,12 @@ __global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
         const int64_t o = ((int64_t)t0 * H + r) * F + f;
         T4 w;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(adu[i][g][e]);
+        for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(adu[i][g][e] * scale);
         *reinterpret_cast<T4 *>(du + o) = w;
         *reinterpret_cast<f32x4 *>(ax + o) = aax[i][g];
       } else {
         const int64_t o = ((int64_t)pbase * H + r) * F + f;
-        *reinterpret_cast<f32x4 *>(part_du + o) = adu[i][g];
+        *reinterpret_cast<f32x4 *>(part_du + o) = adu[i][g] * scale;
         *reinterpret_cast<f32x4 *>(part_ax + o) = aax[i][g];
       }
     }
