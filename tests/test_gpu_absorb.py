@@ -197,6 +197,28 @@ def test_absorb_f32_shared_key_tiles(device, H, d_kv):
         assert_close(n, a, r)
 
 
+# Segments without queries in the one-kernel backward: their keys, in ranges of up to
+# 1024, are cleared (every width class of the clearing store, ranges at its edges).
+@pytest.mark.parametrize("d_kv", [72, 216, 256])
+def test_absorb_clears_query_less_segments(device, d_kv):
+    q_lens, k_lens = [0, 8, 0, 0, 3, 0], [1025, 60, 1, 1024, 40, 5000]
+    print(f"[absorb clear] d_kv={d_kv}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    T_q, T_k = sum(q_lens), sum(k_lens)
+    X = torch.randn(T_k, d_kv, generator=g).to(torch.bfloat16).to(device).requires_grad_(True)
+    u = torch.randn(T_q, 8, d_kv, generator=g).to(torch.bfloat16).to(device)
+    W = (torch.randn(d_kv, 8, 32, generator=g) * 0.1).to(torch.bfloat16).to(device)
+    cq, ck = cu_from_lens(q_lens).to(device), cu_from_lens(k_lens).to(device)
+    dirty = torch.full((T_k, d_kv), float("nan"), dtype=torch.bfloat16, device=device)
+    O = target_attn_inner(u, X, W, cq, ck)
+    del dirty  # freed: dX takes its block
+    dX = torch.autograd.grad(O, X, torch.ones_like(O))[0]
+    assert torch.isfinite(dX).all()
+    ck = ck.tolist()
+    for s, q in enumerate(q_lens):
+        assert bool((dX[ck[s]:ck[s + 1]] != 0).any()) == (q > 0)
+
+
 # fp16 gradients of small magnitude through the one-kernel backward.  It rounds
 # dS = P (dP - delta) to fp16 without the scale, so an element's rounding error is
 # that of dS itself, uniform within an ulp (2^-24 in the subnormal range that small

@@ -611,3 +611,23 @@ def test_varlen_balanced_plan():
     for n, tile in ((127, 128), (128, 256)):
         p = _lib.plan_varlen(_cu([256] * n), _cu([256] * n), 2, 128, True)
         assert (p.info.q_tile, p.info.k_tile) == (tile, tile)
+
+
+@pytest.mark.parametrize("q_lens,k_lens", [([3, 0, 2], [50, 200001, 700]), ([0], [1025]),
+                                           ([0, 0, 8], [1024, 4096, 9])])
+def test_absorb_clear_items(q_lens, k_lens):
+    """A segment without queries is cleared by items of at most 1024 keys that
+    cover its range once, ahead of the items of fewer (key, row) products."""
+    cq, ck = _cu(q_lens), _cu(k_lens)
+    p = _lib.plan_absorb(cq, ck, 8, 256, 32)
+    dq = p.section("dq").tolist()
+    for s, (q, k) in enumerate(zip(q_lens, k_lens)):
+        if q == 0:
+            its = sorted((r[2], r[3]) for r in dq if r[5] == s)
+            assert its[0][0] == ck[s] and its[-1][1] == ck[s + 1]
+            assert all(a[1] == b[0] for a, b in zip(its, its[1:]))
+            assert all(0 < b - a <= 1024 for a, b in its)
+    # 1024 cleared keys are ordered before a tile of 9 keys and 32 rows
+    last = [i for i, r in enumerate(dq) if r[0] == r[1] and r[3] - r[2] == 1024]
+    tiny = [i for i, r in enumerate(dq) if r[0] < r[1] and r[3] - r[2] < 64]
+    assert not last or not tiny or max(last) < min(tiny)

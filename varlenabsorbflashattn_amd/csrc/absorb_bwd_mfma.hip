@@ -643,10 +643,12 @@ __global__ __launch_bounds__(64 * kMgWaves, 2) void absorb_bwd_kernel(
   const int tid = threadIdx.x;
   if (nrows == 0) {  // a sample without queries: its keys get zero gradient
     const u32x4 z = {0u, 0u, 0u, 0u};
+    T *rows = dX + (int64_t)k0 * F;
+    const int64_t n = (int64_t)(k1 - k0) * (F / 8);  // 16-byte chunks
     // (a uniform trip count: a divergent loop exit on the way to the return
     // would make the compiler pass every scalar of the kernel through VGPRs)
-    for (int k = k0; k < k1; ++k)
-      if (tid < F / 8) *reinterpret_cast<u32x4 *>(dX + (int64_t)k * F + tid * 8) = z;
+    for (int64_t i = 0; i < n; i += 64 * kMgWaves)
+      if (i + tid < n) *reinterpret_cast<u32x4 *>(rows + (i + tid) * 8) = z;
     return;
   }
   const int lane = tid & 63;

@@ -567,13 +567,15 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
       key_split(std::min<int64_t>(lq, TT) * H, lk, p, &ns, &chunk);
     }
     max_split = std::max(max_split, ns);
-    // the du pass's own split; a segment without queries is one item of the
-    // merged kernel, which clears its dX
+    // the du pass's own split; a segment without queries is items of the merged
+    // kernel, which clears its dX
     int64_t du_ns = 1, du_chunk = lk;
     if (du_items && lq > 0) key_split(kAbsorbRows, lk, du_pol, &du_ns, &du_chunk);
-    if (du_items && lq == 0 && lk > 0)
-      qs.push_back(Item{{(int32_t)q0, (int32_t)q0, (int32_t)k0, (int32_t)k1, -1, (int32_t)s, 0, 1},
-                        0});
+    for (int64_t k = k0; du_items && lq == 0 && k < k1; k += kAbsorbClearKeys) {
+      const int64_t ke = std::min(k + kAbsorbClearKeys, k1);
+      qs.push_back(Item{{(int32_t)q0, (int32_t)q0, (int32_t)k, (int32_t)ke, -1, (int32_t)s, 0, 1},
+                        (ke - k) * kAbsorbClearCost});
+    }
     const int64_t seg_prow = prow;
     for (int64_t t = q0; t < q1; t += TT) {
       const int64_t te = std::min(t + TT, q1), ntok = te - t;

@@ -82,6 +82,14 @@ constexpr int64_t kAbsorbSlack2 = 5;
 constexpr SplitPolicy kAbsorbDuPolicy{0, 1 << 30, 256, 1, 16, 256, 256, 64, 32};
 constexpr int64_t kAbsorbDuSlots = 512;
 constexpr int64_t kAbsorbDuSlack = 2;
+// A segment without queries is cleared by items of at most kAbsorbClearKeys keys.
+// In the longest-first order a key counts as kAbsorbClearCost rows: it is stored
+// and not read, about half of what a tile of 32 rows moves.  One item for the whole
+// range, 16 to 32 threads storing a key at a time, ended the launch alone: 256 samples
+// (D_KV = 256) beside one of 20k / 200k keys without queries, forward + backward
+// 603 / 5114 us -> 155 / 157.
+constexpr int64_t kAbsorbClearKeys = 1024;
+constexpr int64_t kAbsorbClearCost = 16;
 
 // Varlen backward, fused K-major path (dQ, dK, dV in one kernel, fp32 dQ
 // partials per key chunk summed in order): segments with at most kFusedMaxQ
