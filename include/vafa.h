@@ -125,7 +125,8 @@ typedef struct vafa_plan_info {
    * (most of the work lies in segments of at most 128 queries, whose items
    * share no key range: the heads then read whole token rows together);
    * 0 = item-major with heads innermost (the query tiles of a segment share
-   * its K/V in one XCD's L2) */
+   * its K/V in one XCD's L2).  Absorb: 1 = the 16-bit backward runs the n_fkv
+   * items on the kernel that forms dU and dX in one pass */
   int64_t xcd_heads;
 } vafa_plan_info;
 

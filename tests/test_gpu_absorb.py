@@ -262,18 +262,21 @@ def test_absorb_merged_small_fp16_gradients(device, H, D_H, d_kv, k_lens, m):
 
 
 def test_absorb_merged_beside_streamed(device):
-    """A launch of more than 384k keys whose segments lie on both sides of 64
-    rows: merged items, and the du and dX kernels for the rest.  The keys of
-    two long segments carry the launch over the line; the others' gradients
-    are compared with a launch without them."""
-    H, d_kv = 8, 128
+    """A launch whose segments lie on both sides of 64 rows, those of at most 64
+    with enough keys: merged items, and the du and dX kernels for the rest.  The
+    keys of two long segments carry the launch over the line; the others'
+    gradients are compared with a launch without them."""
+    H, d_kv = 8, 256
     q_lens, k_lens = [3, 9, 8, 20, 0, 1], [70, 300, 33, 129, 20, 5]
     g = torch.Generator().manual_seed(3)
     mk = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(torch.bfloat16)
 
     def grads(big):
-        ql, kl = q_lens + ([1, 9] if big else []), k_lens + ([200000] * 2 if big else [])
+        ql, kl = q_lens + ([1, 9] if big else []), k_lens + ([380000, 20000] if big else [])
         Tq, Tk = sum(ql), sum(kl)
+        info = _lib.plan_absorb(cu_from_lens(ql).numpy(), cu_from_lens(kl).numpy(), H, d_kv,
+                                32).info
+        assert info.xcd_heads == big and 0 < info.n_fkv < info.n_dq
         u, X, W, dO = ins
         dev = [t.to(device).requires_grad_(True) for t in (u[:Tq], X[:Tk], W)]
         O = target_attn_inner(*dev, cu_from_lens(ql).to(device), cu_from_lens(kl).to(device))

@@ -631,3 +631,19 @@ def test_absorb_clear_items(q_lens, k_lens):
     last = [i for i, r in enumerate(dq) if r[0] == r[1] and r[3] - r[2] == 1024]
     tiny = [i for i, r in enumerate(dq) if r[0] < r[1] and r[3] - r[2] < 64]
     assert not last or not tiny or max(last) < min(tiny)
+
+
+@pytest.mark.parametrize("d_kv", [128, 216, 256])
+def test_absorb_merged_rule(d_kv):
+    """The one-pass backward kernel is chosen by the keys of its own segments: for
+    all of a launch, and beside segments of more than 64 rows from 88M X elements
+    on, however many keys those, or segments without queries, hold."""
+    line = -(-(88 << 20) // d_kv)
+    for q_lens, k_lens, merge in [([8, 3], [50, 7], 1), ([8, 0], [50, 10**6], 1),
+                                  ([9, 3], [10**6, 7], 0), ([9, 3, 0], [50, 7, 10**6], 0),
+                                  ([9, 8], [5, line - 1], 0), ([9, 8], [5, line], 1),
+                                  ([9], [10**6], 0)]:
+        p = _lib.plan_absorb(_cu(q_lens), _cu(k_lens), 8, d_kv, 32)
+        assert p.info.xcd_heads == merge, (q_lens, k_lens)
+        assert p.info.n_fkv == sum(1 for r in p.section("dq").tolist()
+                                   if q_lens[r[5]] * 8 <= 64)

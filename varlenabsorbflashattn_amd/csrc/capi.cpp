@@ -361,8 +361,7 @@ void absorb_fwd_all(const AbsorbArgs &a, hipStream_t st) {
 template <typename T>
 void mfma_absorb_du_dx(const AbsorbArgs &a, hipStream_t st) {
   AbsorbArgs r = a;  // what the merged kernel leaves to the du and dX kernels
-  const bool all = a.n_merged == a.n_qseg;
-  if (a.n_merged > 0 && mfma_absorb_merged(a.F) && (all || a.T_k > kAbsorbMergedKeys)) {
+  if (a.merge && a.n_merged > 0 && mfma_absorb_merged(a.F)) {
     launch_mfma_absorb_bwd_merged<T>(a, st);
     r.qseg_items = a.qseg_items + a.n_merged * VAFA_ITEM_INTS;
     r.n_qseg = a.n_qseg - a.n_merged;
@@ -1070,7 +1069,7 @@ static AbsorbArgs bwd_args(const void *u, const void *X, const void *W_V, const 
   a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
   if (info->n_dq > 0) {  // the du pass's own items (split key ranges, merged tiles first)
     a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
-    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv;
+    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv; a.merge = info->xcd_heads != 0;
   }
   a.T_q = info->T_q; a.T_k = info->T_k;
   a.H = (int)info->H; a.F = (int)D_KV; a.DH = (int)D_H; a.scale = scale;

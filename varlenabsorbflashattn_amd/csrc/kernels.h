@@ -92,6 +92,7 @@ struct AbsorbArgs {
   int comb_rows;              // most tokens of one combine item
   const int32_t *merged_items;  // token tiles whose du, aX and dX one kernel forms
   int64_t n_merged;
+  bool merge;                   // whether that kernel pays off in this launch
   const int32_t *qtc_items;   // split token tiles of the du pass
   int64_t n_qtc;
   int qtc_rows;               // most tokens of one of them

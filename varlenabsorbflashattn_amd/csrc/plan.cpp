@@ -515,7 +515,6 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   int rc = check_pair(cu_q, cu_k, n1);
   if (rc) return rc;
   if (H < 1) return fail(VAFA_ERR_ASSERT, "H must be >= 1");
-  (void)D_KV;
   (void)D_H;
   const int64_t TT = std::max<int64_t>(1, kAbsorbRows / H);
   const int64_t BK = cu_k[n1 - 1] <= kAbsorbSmallKeys ? kAbsorbSmallKTile : kAbsorbKTile;
@@ -552,9 +551,11 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   qt.items.reserve(n_tiles);
   kv.items.reserve(cu_k[n1 - 1] / BK + n1);
   int64_t prow = 0, qprow = 0, max_split = 1;
+  int64_t merged_keys = 0;  // of the merged kernel's segments with queries
   for (int64_t s = 0; s + 1 < n1; ++s) {
     const int64_t q0 = cu_q[s], q1 = cu_q[s + 1], k0 = cu_k[s], k1 = cu_k[s + 1];
     const int64_t lq = q1 - q0, lk = k1 - k0;
+    if (lq > 0 && lq * H <= kDxResidentRows) merged_keys += lk;
     // one split decision per segment (its tiles share the key ranges)
     int64_t ns = 1, chunk = lk;
     if (lq > 0) {
@@ -641,6 +642,7 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   });
   comb.keep_order();
   qsc.keep_order();
+  info->xcd_heads = mg_end == qs.order.end() || merged_keys * D_KV >= kAbsorbMergedElems ? 1 : 0;
   info->n_part_rows = prow;
   info->n_fpart_rows = qprow;
   info->max_split = max_split;

@@ -123,10 +123,15 @@ constexpr int kXcds = 8;
 // streamed in 32-row blocks (absorb_dx_kernel).
 constexpr int kDxResidentRows = 64;
 // 16-bit backward: the segments of at most kDxResidentRows rows run on the
-// merged kernel when they are all of the launch or it holds more keys than this;
-// in a smaller mixed launch a third kernel costs more than the pass saved (100
-// samples of <= 2048 keys, a quarter above 64 rows, forward + backward: 187 us
-// merged, 179 not; 500 samples 437 and 470).
-constexpr int64_t kAbsorbMergedKeys = 384 * 1024;
+// merged kernel when they are all of the launch or hold at least this many X
+// elements (keys x D_KV).  In a mixed launch the merged kernel runs ahead of the
+// other two, whose CUs it leaves idle at its end, so the pass over X that it saves
+// has to be worth a kernel's tail, however long the other segments are.  Forward +
+// backward, us, not merged / merged at M elements (samples of <= 2048 keys, 8 heads):
+// D_KV 256  M = 40M 480 / 508, 58M 598 / 622, 82M 556 / 558, 96M 383 / 381, 106M
+// 362 / 343, 119M 1077 / 1045, 191M 956 / 888; D_KV 192  62M 424 / 434, 72M 301 /
+// 315, 89M 385 / 366, 103M 368 / 358; D_KV 128  29M 365 / 403, 60M 287 / 301, 74M
+// 270 / 289, 67M (of 307M) 1235 / 1219, 96M 555 / 538, 129M 497 / 476.
+constexpr int64_t kAbsorbMergedElems = int64_t{88} << 20;
 
 }  // namespace vafa
