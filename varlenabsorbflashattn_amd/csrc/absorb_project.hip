@@ -332,8 +332,12 @@ struct WgSmem {
   static constexpr int kBytes = 2 * kStage * 2;
 };
 
+// At 512 columns with dq the accumulators leave just room for two workgroups per
+// CU (256 registers): slices are compiled in only where launch_wgrad16 takes them,
+// at 256 columns without dq, and the bound holds the rest to that.  9276 tokens of 8
+// heads of 128, D_KV 512: 67 us; 106 at 258 registers and one workgroup.
 template <typename T, int FP, bool DQ>
-__global__ __launch_bounds__(256) void wgrad_kernel(
+__global__ __launch_bounds__(256, FP > 256 ? 2 : 1) void wgrad_kernel(
     const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ Wt, T *__restrict__ dq,
     float *__restrict__ part, int64_t T_q, int64_t tchunk, int G, int lda, int DH, int n_db,
     int n_fb) {
@@ -348,15 +352,16 @@ __global__ __launch_bounds__(256) void wgrad_kernel(
   int64_t b = blockIdx.x;
   const int db = (int)(b % n_db);
   b /= n_db;
-  const int fb = (int)(b % n_fb);  // FP-wide slice of A's columns
-  b /= n_fb;
+  constexpr bool kSlices = FP == 256 && !DQ;
+  const int fb = kSlices ? (int)(b % n_fb) : 0;  // FP-wide slice of A's columns
+  if constexpr (kSlices) b /= n_fb;
   const int g = (int)(b % G);
   const int64_t c = b / G;
   const int64_t ta = c * tchunk, tb = ta + tchunk < T_q ? ta + tchunk : T_q;
   const int d0 = db * kWgDB;
   const int dn = DH - d0 < kWgDB ? DH - d0 : kWgDB;
   A += fb * FP;
-  const int F = lda - fb * FP < FP ? lda - fb * FP : FP;  // columns of this slice
+  const int F = !kSlices || lda - fb * FP < FP ? lda - fb * FP : FP;  // columns of this slice
 
   constexpr int kACh = FP / 8;                    // 16-byte chunks per A row
   constexpr int kAPer = kWgTok * kACh / 256;      // A chunks per thread
