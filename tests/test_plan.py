@@ -647,3 +647,20 @@ def test_absorb_merged_rule(d_kv):
         assert p.info.xcd_heads == merge, (q_lens, k_lens)
         assert p.info.n_fkv == sum(1 for r in p.section("dq").tolist()
                                    if q_lens[r[5]] * 8 <= 64)
+
+
+def test_absorb_wide_feature_splits():
+    """D_KV > 256 (one workgroup per CU): dX tiles of 128, 256 or 512 keys, the
+    widest of which there are 256; forward chunks of at most 1024 keys, or 1/256 of
+    the launch's, and no finer than the launch needs to fill 256 CUs."""
+    for n, bk in ((63, 128), (64, 256), (127, 256), (128, 512), (500, 512)):
+        p = _lib.plan_absorb(_cu([1] * n), _cu([1024] * n), 8, 264, 32)
+        assert p.info.k_tile == bk, n
+    for n, longest in ((600, 2000), (128, 1024), (64, 704), (16, 192), (4, 128)):
+        p = _lib.plan_absorb(_cu([1] * n), _cu([2000] * n), 8, 512, 32)
+        f = p.section("fwd")
+        assert int((f[:, 3] - f[:, 2]).max()) == longest, n
+    # at 256 features and below the rules are unchanged
+    for F in (250, 256):
+        p = _lib.plan_absorb(_cu([1] * 128), _cu([1024] * 128), 8, F, 32)
+        assert p.info.k_tile == 128

@@ -515,9 +515,13 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
   int rc = check_pair(cu_q, cu_k, n1);
   if (rc) return rc;
   if (H < 1) return fail(VAFA_ERR_ASSERT, "H must be >= 1");
-  (void)D_H;
   const int64_t TT = std::max<int64_t>(1, kAbsorbRows / H);
-  const int64_t BK = cu_k[n1 - 1] <= kAbsorbSmallKeys ? kAbsorbSmallKTile : kAbsorbKTile;
+  const bool wide = D_KV > kAbsorbWideF;
+  int64_t BK = cu_k[n1 - 1] <= kAbsorbSmallKeys ? kAbsorbSmallKTile : kAbsorbKTile;
+  if (wide) {  // the widest dX tile of which there is one per CU
+    BK = 4 * kAbsorbSmallKTile;
+    while (BK > kAbsorbSmallKTile && cu_k[n1 - 1] < BK * kAbsorbWideSlots) BK /= 2;
+  }
   // Key chunks of split segments, from the launch's total work: a chunk holds
   // a multiple of the average keys per resident workgroup (never below the
   // policy's long_chunk), and only longer key ranges split.  Longest-first
@@ -530,12 +534,22 @@ int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64
     n_tiles += tiles;
     work += tiles * (cu_k[s + 1] - cu_k[s]);
   }
-  auto raise_chunk = [work](SplitPolicy &p, int64_t slack, int64_t slots) {
-    p.long_chunk = std::max<int64_t>(p.long_chunk, round_up(cdiv(slack * work, slots), p.align));
+  auto raise_chunk = [](SplitPolicy &p, int64_t w, int64_t slack, int64_t slots) {
+    p.long_chunk = std::max<int64_t>(p.long_chunk, round_up(cdiv(slack * w, slots), p.align));
     p.long_threshold = p.long_chunk;
   };
-  raise_chunk(pol, kAbsorbSlack2, 2 * kAbsorbSlots);
-  raise_chunk(du_pol, kAbsorbDuSlack, kAbsorbDuSlots);
+  if (wide) {  // (kAbsorbWideF)
+    const int64_t w = work + n_tiles * (kAbsorbWideItem + D_H);
+    SplitPolicy whole = pol;
+    whole.long_chunk = kAbsorbWideChunk;
+    raise_chunk(whole, work, 3, kAbsorbSlots);
+    raise_chunk(pol, w, kAbsorbSlack2, 4 * kAbsorbWideSlots);
+    if (whole.long_chunk < pol.long_chunk) pol = whole;
+    raise_chunk(du_pol, w, kAbsorbDuSlack, kAbsorbWideSlots);
+  } else {
+    raise_chunk(pol, work, kAbsorbSlack2, 2 * kAbsorbSlots);
+    raise_chunk(du_pol, work, kAbsorbDuSlack, kAbsorbDuSlots);
+  }
   const bool du_items = H <= kAbsorbRows;  // the wave-per-row kernels run qt and kv
   std::memset(info, 0, sizeof(*info));
   info->magic = VAFA_PLAN_MAGIC;

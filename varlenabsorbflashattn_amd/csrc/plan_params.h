@@ -82,6 +82,21 @@ constexpr int64_t kAbsorbSlack2 = 5;
 constexpr SplitPolicy kAbsorbDuPolicy{0, 1 << 30, 256, 1, 16, 256, 256, 64, 32};
 constexpr int64_t kAbsorbDuSlots = 512;
 constexpr int64_t kAbsorbDuSlack = 2;
+// D_KV > kAbsorbWideF: one workgroup per CU in every pass, and an item costs a
+// prologue and an epilogue worth kAbsorbWideItem + D_H keys, which count towards
+// the average.  Forward chunks hold 5/4 of the average keys per CU, but no more
+// than 1024 or 1/256 of the keys (chunks of that size keep the tail of a large launch
+// short); dU chunks twice the average; dX tiles of 128, 256 or 512 keys leave one
+// per CU.  Forward / forward + backward, us, at whole ranges and 512-key dX tiles -> the
+// rules of narrower features -> these, D_KV 512: 512 samples of 8 heads of 32 72 / 415 ->
+// 79 / 455 -> 72 / 414; 512 of 8 heads of 128 145 / 604 -> 172 / 677 -> 145 / 598; 64
+// and 256 of 16 heads of 128 121 / 610 -> 153 / 506 -> 116 / 451 and 182 / 764 -> 231 /
+// 818 -> 182 / 730; 64 and 256 of 8 heads of 32 in fp32, whose products outweigh an
+// item's cost, 379 / 2066 -> 97 / 426 -> 115 / 444 and 410 / 2171 -> 225 / 945 -> 241 /
+// 1106 (the planner does not see the data type).
+constexpr int64_t kAbsorbWideF = 256;
+constexpr int64_t kAbsorbWideSlots = 256;
+constexpr int64_t kAbsorbWideItem = 64;
 // A segment without queries is cleared by items of at most kAbsorbClearKeys keys.
 // In the longest-first order a key counts as kAbsorbClearCost rows: it is stored
 // and not read, about half of what a tile of 32 rows moves.  One item for the whole
