@@ -197,6 +197,18 @@ def test_absorb_f32_shared_key_tiles(device, H, d_kv):
         assert_close(n, a, r)
 
 
+# More than 64 heads: a wave per (token, head) row, whole and split key ranges, a
+# width that is not padded.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("H,D_H,d_kv", [(65, 16, 32), (96, 32, 50)])
+def test_absorb_above_64_heads(device, H, D_H, d_kv, dtype):
+    q_lens, k_lens = [2, 0, 5], [70, 9, 1300]
+    print(f"[absorb above 64 heads {dtype}] H={H} D_H={D_H} d_kv={d_kv}", flush=True)
+    got, ref = run_case(q_lens, k_lens, dtype, device, d_q=64, d_kv=d_kv, H=H, D_H=D_H)
+    for n, a, r in zip(NAMES, got, ref):
+        assert_close(n, a, r)
+
+
 # Segments without queries in the one-kernel backward: their keys, in ranges of up to
 # 1024, are cleared (every width class of the clearing store, ranges at its edges).
 @pytest.mark.parametrize("d_kv", [72, 216, 256])

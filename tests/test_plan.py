@@ -664,3 +664,16 @@ def test_absorb_wide_feature_splits():
     for F in (250, 256):
         p = _lib.plan_absorb(_cu([1] * 128), _cu([1024] * 128), 8, F, 32)
         assert p.info.k_tile == 128
+
+
+@pytest.mark.parametrize("H", [64, 65, 96, 1000])
+def test_absorb_workspace_any_head_count(H):
+    """Workspace queries answer for any head count, those above the matrix-core
+    kernels' 64 (at most one token per item) among them."""
+    p = _lib.plan_absorb(_cu([3, 0, 2]), _cu([5000, 7, 1]), H, 64, 16)
+    L = _lib.lib()
+    for F, D_H in ((64, 16), (50, 128), (512, 256)):
+        fwd = L.vafa_absorb_fwd_workspace(p.info, F, D_H)
+        assert fwd >= p.info.n_part_rows * H * (D_H + 1) * 4
+        assert L.vafa_absorb_bwd_workspace(p.info, F, D_H) >= 5 * H * F * 4
+        assert L.vafa_absorb_fwd_fold_workspace(p.info, F, D_H) > 0

@@ -489,8 +489,9 @@ bool mfma_absorb_fwd_supported(int H, int F, int DH) {
 }
 
 // Most heads among the 16 rows of one forward wave (rows head-major,
-// floor(64/H) tokens per head).
+// floor(64/H) tokens per head); 0 above 64 heads, which no wave here runs.
 int absorb_heads_per_wave(int H) {
+  if (H > kAbsorbRows) return 0;
   const int TT = kAbsorbRows / H;
   int m = 0;
   for (int w = 0; w < kFwdWaves; ++w) {
