@@ -624,6 +624,29 @@ def test_project_f32(device, T, d_q, d_kv, H, D_H):
         assert got.shape == r.shape and (err <= (n + 2) * 2.0 ** -24 * m).all()
 
 
+@pytest.mark.parametrize("T", [9000, 20001])
+def test_project_f32_both_routes(device, T):
+    """On both sides of the token line (H D_H = 256, training from about 11k) u and
+    its gradients agree with the library's kernels within the bound of
+    test_project_f32, twice, as each side has its own sums."""
+    from varlenabsorbflashattn_amd.absorb import _Project, _project_native, _project_u
+    g = torch.Generator().manual_seed(T)
+    ins = [torch.randn(*s, generator=g).to(device).requires_grad_(True)
+           for s in ((T, 256), (256, 1, 256), (256, 1, 256))]
+    du = torch.randn(T, 1, 256, generator=g).to(device)
+    print(f"[project f32 routes] T={T}", flush=True)
+    assert _project_native(*ins) == (T < 10000)
+    u, own = _project_u(*ins), _Project.apply(*ins)
+    a = torch.autograd.grad(u, ins, du)
+    b = torch.autograd.grad(own, ins, du)
+    q, wq, wk, d = (t.detach().abs() for t in (*ins, du))
+    wq, wk, d = wq[:, 0], wk[:, 0], d[:, 0]
+    qp, dqp = q @ wq, d @ wk
+    mags = (qp @ wk.t(), dqp @ wq.t(), q.t() @ dqp, d.t() @ qp)
+    for x, y, m, n in zip((u, *a), (own, *b), mags, (512, 512, 256 + T, 256 + T)):
+        assert ((x - y).abs() <= 2 * (n + 2) * 2.0 ** -24 * m.view_as(x)).all()
+
+
 def test_project_rejects_bad_shapes(device):
     """Unsupported widths and dtypes return an error, and nothing runs."""
     from varlenabsorbflashattn_amd import _lib

@@ -49,3 +49,21 @@ def test_projection_heads_do_not_mix():
     (dW_K,) = torch.autograd.grad(u, (W_K,), du)
     assert torch.count_nonzero(dW_K[:, [0, 2, 3], :]) == 0
     assert torch.count_nonzero(dW_K[:, 1, :]) == dW_K[:, 1, :].numel()
+
+
+def test_f32_projection_rule():
+    """fp32 projections take torch's GEMMs only where those were measured faster:
+    many tokens of few heads, and for inference earlier than for training."""
+    from varlenabsorbflashattn_amd.absorb import _project_f32_pays as pays
+    for T in (1, 256, 2400, 50000, 200000):
+        assert pays(T, 8, 256, 256, 32, False) and pays(T, 8, 256, 256, 32, True)
+        assert pays(T, 12, 128, 96, 64, False) and pays(T, 12, 128, 96, 64, True)
+    lines = {(8, 968, 216, 32): (10000, 20000, 50000, 200000),
+             (1, 256, 256, 256): (5000, 10000, 10000, 20000),
+             (1, 256, 256, 32): (20000, 50000, 50000, 200000),
+             (4, 250, 256, 64): (10000, 20000, 50000, None),
+             (2, 968, 250, 128): (2400, 5000, 2400, 5000)}
+    for (H, d_q, d_kv, D_H), (f0, f1, t0, t1) in lines.items():
+        assert pays(f0, H, d_q, d_kv, D_H, False) and not pays(f1, H, d_q, d_kv, D_H, False)
+        assert pays(t0, H, d_q, d_kv, D_H, True)
+        assert t1 is None or not pays(t1, H, d_q, d_kv, D_H, True)

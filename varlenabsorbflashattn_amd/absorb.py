@@ -235,10 +235,40 @@ def _project_native(q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -
         return False
     if q_raw.dtype == torch.float32:
         # (autocast applies to the torch formulation only)
-        return (0 < d_q <= 65536 and 0 < d_kv <= 65536 and W_Q.shape[1] * D_H <= 65536
-                and W_Q.shape[1] <= 1024 and not torch.is_autocast_enabled())
+        H = W_Q.shape[1]
+        return (0 < d_q <= 65536 and 0 < d_kv <= 65536 and H * D_H <= 65536
+                and H <= 1024 and not torch.is_autocast_enabled()
+                and _project_f32_pays(q_raw.shape[0], H, d_q, d_kv, D_H,
+                                      torch.is_grad_enabled() and
+                                      any(t.requires_grad for t in (q_raw, W_Q, W_K))))
     return (q_raw.dtype in (torch.bfloat16, torch.float16)
             and d_q % 8 == 0 and d_kv % 8 == 0)
+
+
+def _project_f32_pays(T_q: int, H: int, d_q: int, d_kv: int, D_H: int, grad: bool) -> bool:
+    """Whether the fp32 projections run on this library's kernels rather than on
+    torch's GEMMs: what either takes on large launches, from the rates measured
+    there, and what torch's calls cost at least.
+
+    The row GEMM streams its operands from L2 at 47 TFLOP/s over D_Q and 50 over
+    D_KV; 25 where u's sums are shorter than 64 (D_H = 32), about half over widths
+    that are not whole 16-byte chunks and where H D_H leaves half of its 64 columns
+    empty.  Its backward runs at 44 (28 over such a D_KV).  Torch's reach 110, and 95
+    backward, but multiply H blocks per D_KV, of which one is not zero, and take
+    25 us, with a backward 100, longer to call.  us, torch / own, forward and forward
+    + backward, H x D_H, D_Q, D_KV, tokens: 8 x 32, 256, 256, 2400 101 / 35 and 415 /
+    101, 200k 1941 / 1658 and 6466 / 4210; 8 x 32, 968, 216, 10k 190 / 147, 20k 274 /
+    280, 50k 2361 / 2086, 200k 7586 / 8303; 1 x 256, 256, 256, 5k 52 / 40, 10k 52 / 56 and
+    208 / 184, 20k 307 / 367, 200k 552 / 996 and 2199 / 3299."""
+    x = 2e-6 * T_q * H * D_H  # us x TFLOP/s per feature
+    aligned = d_kv % 4 == 0
+    own = d_q / (47 if d_q % 4 == 0 and H * D_H >= 64 else 23) + \
+        d_kv / ((50 if D_H >= 64 else 25) * (1 if aligned else 0.63))
+    blocks = d_q + H * d_kv
+    if not grad:
+        return x * (own - blocks / 110) < 25
+    own += 2 * d_q / 44 + 2 * d_kv / (44 if aligned else 28)
+    return x * (own - blocks * (1 / 110 + 2 / 95)) < 100
 
 
 class _Project(torch.autograd.Function):
@@ -324,7 +354,8 @@ def _project_u(q_raw: torch.Tensor, W_Q: torch.Tensor, W_K: torch.Tensor) -> tor
     contiguous ``[T_q, H, d_kv]``.
 
     CUDA operands run on ``_Project`` (both directions in this library's
-    kernels) in fp32 and, with D_Q, D_KV, D_H multiples of 8, in 16 bits.
+    kernels) in fp32 up to the token counts of ``_project_f32_pays`` and, with
+    D_Q, D_KV, D_H multiples of 8, in 16 bits.
     Other operands (odd 16-bit widths, the CPU) take the reference's own
     formulation on torch's GEMMs: q_proj =
     q_raw @ W_Q, then u = q_proj @ blockdiag(W_K[:,h,:]^T), ONE GEMM that

@@ -13,6 +13,8 @@
 // reference's 16-bit GEMMs.  The weight gradients dW_K = sum_t du^T q_proj
 // per head and dW_Q = sum_t q_raw^T dq_proj are token reductions and run on
 // the chunked, ordered (deterministic) reduction of dW_V.
+#include <type_traits>
+
 #include "absorb_tiles.h"
 
 namespace vafa {
@@ -486,11 +488,12 @@ __global__ __launch_bounds__(256, FP > 256 ? 2 : 1) void wgrad_kernel(
 // 256: 0.3 GFLOP) and latency-bound, so operands go straight from L2 to
 // registers, 64 k per batch.  In product i of a 16-wide k block lane group lq
 // holds k = 4*lq + i, so a lane's operand is 16 contiguous bytes along k.  Any
-// width runs: VEC = 16-byte accesses where every stride is a multiple of 4.
+// width runs: VEC = 16-byte loads where every input row starts on 16 bytes, SVEC =
+// 16-byte stores where every output row does.
 // 2397 tokens, D_Q = D_KV = 256 forward and backward: torch's GEMMs, block
 // diagonal and copies took 285 us of GPU time, these kernels and the weight
 // gradients 108.
-template <bool KJ, bool VEC>
+template <bool KJ, bool VEC, bool SVEC>
 __global__ __launch_bounds__(256) void rowgemm_f32_kernel(
     const float *__restrict__ X, const float *__restrict__ W, float *__restrict__ Y, int64_t T_q,
     int G, int J, int K, int64_t ldx, int64_t xs, int64_t ws, int64_t ldw, int64_t ldy,
@@ -561,7 +564,7 @@ __global__ __launch_bounds__(256) void rowgemm_f32_kernel(
     const int64_t t = tb + 16 * hf + l16;
     if (t >= T_q || jo >= J) continue;
     float *y = Y + t * ldy + g * ys + jo;
-    if constexpr (VEC) {
+    if constexpr (SVEC) {
       *reinterpret_cast<f32x4 *>(y) = acc[hf];
     } else {
 #pragma unroll
@@ -659,17 +662,22 @@ void launch_rowgemm_f32(const RowGemm &p, bool kj, hipStream_t st) {
   const int n_jb = (p.J + 63) / 64;
   const int64_t wgs = (p.T_q + kRgTok - 1) / kRgTok * p.G * n_jb;
   if (wgs == 0) return;
-  const bool vec = p.J % 4 == 0 && p.K % 4 == 0 && p.ldx % 4 == 0 && p.xs % 4 == 0 &&
-                   p.ws % 4 == 0 && p.ldw % 4 == 0 && p.ldy % 4 == 0 && p.ys % 4 == 0;
+  const bool vec = p.K % 4 == 0 && p.ldx % 4 == 0 && p.xs % 4 == 0 &&
+                   (kj || (p.ws % 4 == 0 && p.ldw % 4 == 0));
+  const bool svec = p.J % 4 == 0 && p.ldy % 4 == 0 && p.ys % 4 == 0;
   auto run = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, st, (const float *)p.X,
                        (const float *)p.W, (float *)p.Y, p.T_q, p.G, p.J, p.K, p.ldx, p.xs, p.ws,
                        p.ldw, p.ldy, p.ys, n_jb);
   };
-  if (kj)
-    vec ? run(rowgemm_f32_kernel<true, true>) : run(rowgemm_f32_kernel<true, false>);
-  else
-    vec ? run(rowgemm_f32_kernel<false, true>) : run(rowgemm_f32_kernel<false, false>);
+  auto pick = [&](auto k) {
+    constexpr bool KJ = decltype(k)::value;
+    if (vec)
+      svec ? run(rowgemm_f32_kernel<KJ, true, true>) : run(rowgemm_f32_kernel<KJ, true, false>);
+    else
+      svec ? run(rowgemm_f32_kernel<KJ, false, true>) : run(rowgemm_f32_kernel<KJ, false, false>);
+  };
+  kj ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 bool rowgemm_supported(const RowGemm &p) {
