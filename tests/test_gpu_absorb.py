@@ -197,6 +197,17 @@ def test_absorb_f32_shared_key_tiles(device, H, d_kv):
         assert_close(n, a, r)
 
 
+def test_absorb_host_array_cu_seqlens(device):
+    """Calls without validation take cu_seqlens as arrays too."""
+    cq, ck = cu_from_lens([3, 2]), cu_from_lens([40, 7])
+    g = torch.Generator().manual_seed(0)
+    args = [torch.randn(*s, generator=g).to(torch.bfloat16).to(device)
+            for s in ((5, 8, 64), (47, 64), (64, 8, 32))]
+    want = target_attn_inner(*args, cq.to(device), ck.to(device))
+    got = target_attn_inner(*args, cq.numpy(), ck.numpy(), validate=False)
+    assert torch.equal(got, want)
+
+
 # More than 64 heads: a wave per (token, head) row, whole and split key ranges, a
 # width that is not padded.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])

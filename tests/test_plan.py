@@ -677,3 +677,17 @@ def test_absorb_workspace_any_head_count(H):
         assert fwd >= p.info.n_part_rows * H * (D_H + 1) * 4
         assert L.vafa_absorb_bwd_workspace(p.info, F, D_H) >= 5 * H * F * 4
         assert L.vafa_absorb_fwd_fold_workspace(p.info, F, D_H) > 0
+
+
+def test_host_cu_pair_inputs():
+    """cu_seqlens as tensors of any dtype, arrays or lists give the same plan key
+    contents (int64) or keep their own integer dtype; the pair may mix them."""
+    import torch
+    want = [0, 3, 9]
+    forms = [np.array(want), want, tuple(want), torch.tensor(want), torch.tensor(want).float(),
+             torch.tensor(want, dtype=torch.int32), torch.tensor(want, dtype=torch.uint8)]
+    for a in forms:
+        for b in forms:
+            x, y = _lib.host_cu_pair(a, b)
+            assert x.tolist() == y.tolist() == want
+            _lib.plan_key("absorb", x, y, (8, 64, 32), "cuda:0")

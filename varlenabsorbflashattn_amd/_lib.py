@@ -327,10 +327,12 @@ _CACHE_MAX = 64
 
 
 def host_cu_pair(a, b) -> Tuple[np.ndarray, np.ndarray]:
-    """Host copies of two cu_seqlens tensors in their own dtype, with one device
-    sync where as_host_i64_pair takes one."""
+    """Host copies of two cu_seqlens in their own integer dtype, with one device
+    sync where as_host_i64_pair takes one; int64 copies of other tensors, and of
+    arrays and lists (which calls without validation take)."""
     import torch
-    if (a.is_floating_point() or a.is_complex() or b.is_floating_point() or b.is_complex()):
+    if not all(isinstance(t, torch.Tensor) and not t.is_floating_point() and not t.is_complex()
+               for t in (a, b)):
         return as_host_i64_pair(a, b)
     if a is b:
         h = a.detach().cpu().numpy()
