@@ -559,3 +559,49 @@ def test_host_module_maps_errors(device):
         _lib.ops().varlen_fwd(*(x[:, :, :48].contiguous() for _ in range(3)), wide.native, 1.0)
     with pytest.raises(AssertionError, match="dtype"):
         _lib.ops().varlen_fwd(*(x.double() for _ in range(3)), wide.native, 1.0)
+
+
+def test_host_module_releases_the_gil(device, tmp_path):
+    """Other Python threads run while the host module allocates and launches: bound
+    to a stand-in for the library, every call reaches it without the GIL."""
+    import ctypes
+    import re
+    import shutil
+    import subprocess
+    from varlenabsorbflashattn_amd import _lib
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no C++ compiler for the stand-in library")
+    _lib.lib()
+    with open(_lib.LIB_PATH, "rb") as f:
+        names = sorted(set(re.findall(rb"vafa_[a-z0-9_]+", f.read())) & {
+            n.encode() for n in _lib.EXPORTED})
+    src = 'extern "C" int PyGILState_Check();\nstatic int held = 0, calls = 0;\n'
+    src += 'extern "C" const char *vafa_last_error() { return "stand-in"; }\n'
+    for n in (n.decode() for n in names):
+        if n != "vafa_last_error":
+            src += (f'extern "C" long {n}() {{ held += PyGILState_Check(); ++calls; '
+                    f'return {16 if n.endswith("workspace") else 0}; }}\n')
+    src += 'extern "C" int gil_held() { return held; }\nextern "C" int n_calls() { return calls; }\n'
+    (tmp_path / "s.cpp").write_text(src)
+    so = str(tmp_path / "libstandin.so")
+    subprocess.run([cxx, "-shared", "-fPIC", str(tmp_path / "s.cpp"), "-o", so], check=True)
+    ops = _lib.ops()
+    mk = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=device)
+    q, X, w = mk(4, 2, 64), mk(4, 64), mk(64, 2, 64)
+    plan = ops.Plan(torch.zeros(8, dtype=torch.int32, device=device), bytes(_lib.PlanInfo()))
+    lse, qr = torch.zeros(4, 2, device=device), mk(4, 64)
+    try:
+        ops.bind(so)
+        ops.varlen_fwd(q, q, q, plan, 1.0)
+        ops.varlen_bwd(q, q, q, q, lse, q, plan, 1.0)
+        ops.absorb_fwd(q, X, w, plan, 1.0)
+        ops.absorb_bwd(q, X, w, q, lse, q, plan, 1.0)
+        ops.absorb_full_fwd(qr, X, w, w, w, plan, 1.0)
+        ops.absorb_full_bwd(qr, w, w, mk(4, 128), X, w, q, lse, q, plan, 1.0, True, True, True)
+        ops.project_fwd(qr, w, w)
+        ops.project_bwd(qr, w, w, mk(4, 128), q, True, True, True)
+    finally:
+        ops.bind(_lib.LIB_PATH)
+    standin = ctypes.CDLL(so)
+    assert standin.n_calls() == 16 and standin.gil_held() == 0

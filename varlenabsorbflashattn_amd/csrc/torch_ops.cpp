@@ -257,13 +257,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<Plan>(m, "Plan").def(py::init([](Tensor items, const py::bytes &info) {
     return Plan(std::move(items), std::string(info));
   }));
+  // allocation and launch may wait (a full queue, an allocator retry): other
+  // Python threads run meanwhile, as they do under a ctypes call
+  py::call_guard<py::gil_scoped_release> no_gil;
   m.def("bind", &bind_library);
-  m.def("varlen_fwd", &varlen_fwd);
-  m.def("varlen_bwd", &varlen_bwd);
-  m.def("absorb_fwd", &absorb_fwd);
-  m.def("absorb_bwd", &absorb_bwd);
-  m.def("absorb_full_fwd", &absorb_full_fwd);
-  m.def("absorb_full_bwd", &absorb_full_bwd);
-  m.def("project_fwd", &project_fwd);
-  m.def("project_bwd", &project_bwd);
+  m.def("varlen_fwd", &varlen_fwd, no_gil);
+  m.def("varlen_bwd", &varlen_bwd, no_gil);
+  m.def("absorb_fwd", &absorb_fwd, no_gil);
+  m.def("absorb_bwd", &absorb_bwd, no_gil);
+  m.def("absorb_full_fwd", &absorb_full_fwd, no_gil);
+  m.def("absorb_full_bwd", &absorb_full_bwd, no_gil);
+  m.def("project_fwd", &project_fwd, no_gil);
+  m.def("project_bwd", &project_bwd, no_gil);
 }
