@@ -833,7 +833,6 @@ int vafa_absorb_fwd(const void *u, const void *X, const void *W_V, void *O, floa
   a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
   a.comb_rows = (int)info->max_comb_rows;
   a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
-  a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
   a.T_q = info->T_q; a.T_k = info->T_k;
   a.H = (int)info->H; a.F = (int)F; a.DH = (int)D_H; a.scale = scale;
   if (int rc = by_dtype<AFwd>(dtype, a, st)) return rc;
@@ -1066,11 +1065,9 @@ static AbsorbArgs bwd_args(const void *u, const void *X, const void *W_V, const 
   a.comb_items = plan_dev + info->off_comb; a.n_comb = info->n_comb;
   a.comb_rows = (int)info->max_comb_rows;
   a.kv_items = plan_dev + info->off_kv; a.n_kv = info->n_kv; a.n_kv_res = info->n_kv_res;
-  a.qseg_items = plan_dev + info->off_qt; a.n_qseg = info->n_qt;
-  if (info->n_dq > 0) {  // the du pass's own items (split key ranges, merged tiles first)
-    a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
-    a.merged_items = a.qseg_items; a.n_merged = info->n_fkv; a.merge = info->xcd_heads != 0;
-  }
+  a.qt_items = plan_dev + info->off_qt; a.n_qt = info->n_qt;
+  a.qseg_items = plan_dev + info->off_dq; a.n_qseg = info->n_dq;
+  a.merged_items = a.qseg_items; a.n_merged = info->n_fkv; a.merge = info->xcd_heads != 0;
   a.T_q = info->T_q; a.T_k = info->T_k;
   a.H = (int)info->H; a.F = (int)D_KV; a.DH = (int)D_H; a.scale = scale;
   return a;

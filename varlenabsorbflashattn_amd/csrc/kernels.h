@@ -86,8 +86,11 @@ struct AbsorbArgs {
   void *wqt;
   int64_t T_qp;
   int DQ;
-  const int32_t *items, *comb_items, *kv_items, *qseg_items;
-  int64_t n_items, n_comb, n_kv, n_qseg;
+  const int32_t *items, *comb_items, *kv_items;
+  int64_t n_items, n_comb, n_kv;
+  const int32_t *qt_items;    // whole token tiles, for the wave-per-row du kernel
+  const int32_t *qseg_items;  // the matrix-core du kernels' items, key ranges split
+  int64_t n_qt, n_qseg;
   int64_t n_kv_res;           // leading kv items for absorb_dx_res_kernel
   int comb_rows;              // most tokens of one combine item
   const int32_t *merged_items;  // token tiles whose du, aX and dX one kernel forms

@@ -400,10 +400,10 @@ void launch_simt_absorb_fwd(const AbsorbArgs &a, hipStream_t st) {
 
 template <typename T>
 void launch_simt_absorb_du(const AbsorbArgs &a, hipStream_t st) {
-  if (a.n_qseg == 0) return;
-  hipLaunchKernelGGL(simt_absorb_du<T>, dim3(a.n_qseg), dim3(256), 0, st, (const T *)a.u,
+  if (a.n_qt == 0) return;
+  hipLaunchKernelGGL(simt_absorb_du<T>, dim3(a.n_qt), dim3(256), 0, st, (const T *)a.u,
                      (const T *)a.X, a.lse_in, a.delta, (T *)a.du, (const T *)a.dax, a.ax,
-                     a.qseg_items, a.H, a.F, a.scale * kLog2e, a.scale);
+                     a.qt_items, a.H, a.F, a.scale * kLog2e, a.scale);
 }
 
 template <typename T>
