@@ -117,3 +117,26 @@ def assert_within_reference_numerics(name: str, out: torch.Tensor, exact: np.nda
     assert e["mean_abs"] <= slack * em["mean_abs"] + tol_mean * s, \
         f"{name}: mean error {e['mean_abs']:.3e} beyond {slack} x the reference numerics' " \
         f"{em['mean_abs']:.3e} + {tol_mean * s:.3e}"
+
+
+# Relative bounds, for gradients whose own scale lies below the absolute ones (an
+# all-zero tensor fails them): unit roundoffs u of the dtype.  A 16-bit gradient
+# passes through a handful of roundings (q_proj, u, dAX, P and dS, du, itself),
+# independent from element to element, so its 2-norm error is a few u / sqrt(3) and
+# one element's a few u of the largest; fp32 sums of up to a few thousand products
+# in another order stay within sqrt(n) u of their magnitudes.
+REL = {torch.bfloat16: 4 * 2.0 ** -8, torch.float16: 4 * 2.0 ** -11, torch.float32: 64 * 2.0 ** -24}
+
+
+def assert_rel(name: str, out: torch.Tensor, ref: np.ndarray) -> None:
+    """2-norm error over the norm, and largest error over the largest value (twice
+    the bound), of a tensor that is not zero."""
+    a = out.detach().float().cpu().numpy().astype(np.float64)
+    r = np.asarray(ref, dtype=np.float64)
+    assert a.shape == r.shape and np.isfinite(a).all(), name
+    norm, top = float(np.linalg.norm(r)), float(np.abs(r).max())
+    assert norm > 0.0, f"{name}: the case must have a gradient"
+    rel, far = float(np.linalg.norm(a - r)) / norm, float(np.abs(a - r).max()) / top
+    print(f"  {name:8s} rel={rel:.3e} max/max={far:.3e} norm={norm:.3e}", flush=True)
+    tol = REL[out.dtype]
+    assert rel <= tol and far <= 2 * tol, f"{name}: {rel:.3e}, {far:.3e} > {tol:.1e}"
