@@ -50,38 +50,80 @@ static void check_ranges(const std::vector<int32_t> &plan, int64_t off, int64_t 
   }
 }
 
-static void one_plan(bool absorb, const std::vector<int64_t> &cq, const std::vector<int64_t> &ck,
-                     int64_t H, int64_t D) {
-  vafa_plan_info info;
+// Partial rows: split items of [first, first + n) write rows pbase .. pbase +
+// tokens (fields 4 and 0, 1), the combine items read nsplit times as many from
+// pbase (fields 2, 3) on; all inside [0, rows).
+static void check_partials(const std::vector<int32_t> &plan, int64_t off, int64_t n, int64_t coff,
+                           int64_t nc, int64_t rows, int64_t most) {
+  for (int64_t i = 0; i < n; ++i) {
+    const int32_t *it = plan.data() + off + i * VAFA_ITEM_INTS;
+    if (it[4] >= 0) CHECK(it[4] + (int64_t)it[1] - it[0] <= rows);
+  }
+  for (int64_t i = 0; i < nc; ++i) {
+    const int32_t *it = plan.data() + coff + i * VAFA_ITEM_INTS;
+    CHECK(it[2] >= 0 && it[3] > 1 && it[1] - it[0] <= most);
+    CHECK(it[2] + (int64_t)it[3] * (it[1] - it[0]) <= rows);
+  }
+}
+
+enum Planner { kVarlen, kBalanced, kAbsorb };
+
+static int run_planner(Planner which, const std::vector<int64_t> &cq,
+                       const std::vector<int64_t> &ck, int64_t H, int64_t D, int64_t F,
+                       int32_t *plan, int64_t cap, vafa_plan_info *info) {
   const int64_t n1 = (int64_t)cq.size();
-  int rc = absorb ? vafa_plan_absorb(cq.data(), ck.data(), n1, H, 256, D, nullptr, 0, &info)
-                  : vafa_plan_varlen(cq.data(), ck.data(), n1, H, D, nullptr, 0, &info);
+  switch (which) {
+    case kAbsorb: return vafa_plan_absorb(cq.data(), ck.data(), n1, H, F, D, plan, cap, info);
+    case kBalanced:
+      return vafa_plan_varlen_balanced(cq.data(), ck.data(), n1, H, D, plan, cap, info);
+    default: return vafa_plan_varlen(cq.data(), ck.data(), n1, H, D, plan, cap, info);
+  }
+}
+
+static void one_plan(Planner which, const std::vector<int64_t> &cq, const std::vector<int64_t> &ck,
+                     int64_t H, int64_t D, int64_t F = 0) {
+  vafa_plan_info info;
+  int rc = run_planner(which, cq, ck, H, D, F, nullptr, 0, &info);
   CHECK(rc == VAFA_OK);
   if (rc != VAFA_OK) return;
   CHECK(info.plan_ints % VAFA_ITEM_INTS == 0 && info.T_q == cq.back() && info.T_k == ck.back());
   std::vector<int32_t> plan((size_t)info.plan_ints + 1, -7);
   if (info.plan_ints >= VAFA_ITEM_INTS) {
     vafa_plan_info small;
-    rc = absorb ? vafa_plan_absorb(cq.data(), ck.data(), n1, H, 256, D, plan.data(),
-                                   info.plan_ints - VAFA_ITEM_INTS, &small)
-                : vafa_plan_varlen(cq.data(), ck.data(), n1, H, D, plan.data(),
-                                   info.plan_ints - VAFA_ITEM_INTS, &small);
+    rc = run_planner(which, cq, ck, H, D, F, plan.data(), info.plan_ints - VAFA_ITEM_INTS, &small);
     CHECK(rc == VAFA_ERR_CAPACITY);
   }
-  rc = absorb ? vafa_plan_absorb(cq.data(), ck.data(), n1, H, 256, D, plan.data(),
-                                 info.plan_ints, &info)
-              : vafa_plan_varlen(cq.data(), ck.data(), n1, H, D, plan.data(), info.plan_ints,
-                                 &info);
+  rc = run_planner(which, cq, ck, H, D, F, plan.data(), info.plan_ints, &info);
   CHECK(rc == VAFA_OK);
   CHECK(plan.back() == -7);  // nothing written past plan_ints
   const int64_t Tq = cq.back(), Tk = ck.back();
   check_ranges(plan, info.off_fwd, info.n_fwd, 0, 2, Tq, Tk);  // {q0,q1,k0,k1}
   check_ranges(plan, info.off_kv, info.n_kv, 0, 2, Tk, Tq);    // {k0,k1,q0,q1}
-  if (!absorb) {
-    check_ranges(plan, info.off_dq, info.n_dq, 0, 2, Tq, Tk);
+  check_ranges(plan, info.off_dq, info.n_dq, 0, 2, Tq, Tk);
+  check_partials(plan, info.off_fwd, info.n_fwd, info.off_comb, info.n_comb, info.n_part_rows,
+                 info.max_comb_rows);
+  if (which != kAbsorb) {
     check_ranges(plan, info.off_fkv, info.n_fkv, 0, 2, Tk, Tq);
+    check_partials(plan, info.off_dq, info.n_dq, info.off_dqc, info.n_dqc, info.n_part_rows,
+                   info.max_dqc_rows);
   } else {
     check_ranges(plan, info.off_qt, info.n_qt, 0, 2, Tq, Tk);
+    check_partials(plan, info.off_dq, info.n_dq, info.off_dqc, info.n_dqc, info.n_fpart_rows,
+                   info.max_dqc_rows);
+    // the leading items are the one-pass kernel's: at most 64 rows, or none and at
+    // most 1024 keys; the kv items beyond n_kv_res belong to the other segments
+    CHECK(info.off_fkv == info.off_dq && 0 <= info.n_fkv && info.n_fkv <= info.n_dq);
+    CHECK(0 <= info.n_kv_res && info.n_kv_res <= info.n_kv);
+    std::vector<char> merged(cq.size(), 0);
+    for (int64_t i = 0; i < info.n_dq; ++i) {
+      const int32_t *it = plan.data() + info.off_dq + i * VAFA_ITEM_INTS;
+      const int64_t s = it[5], rows = (cq[s + 1] - cq[s]) * H;
+      CHECK((i < info.n_fkv) == (rows <= 64));
+      if (it[0] == it[1]) CHECK(rows == 0 && it[3] - it[2] <= 1024);
+      merged[s] = i < info.n_fkv;
+    }
+    for (int64_t i = 0; H <= 64 && i < info.n_kv; ++i)
+      CHECK((i < info.n_kv_res) == (bool)merged[plan[info.off_kv + i * VAFA_ITEM_INTS + 4]]);
   }
 }
 
@@ -115,8 +157,10 @@ int main(int argc, char **argv) {
     CHECK(vafa_chunk_indices(cq.data(), n1, BT, tab.data(), rows, &rows) == VAFA_OK);
     CHECK(tab.back() == -7);
     // plans
-    one_plan(false, cq, ck, Hs[g() % 6], Ds[g() % 5]);
-    one_plan(true, cq, ck, Hs[g() % 4], Ds[g() % 4]);
+    const int64_t Fs[] = {32, 256, 264, 512};
+    one_plan(kVarlen, cq, ck, Hs[g() % 6], Ds[g() % 5]);
+    one_plan(kBalanced, cq, ck, Hs[g() % 6], Ds[g() % 5]);
+    one_plan(kAbsorb, cq, ck, g() % 8 ? Hs[g() % 4] : 1 + g() % 80, Ds[g() % 4], Fs[g() % 4]);
     // corrupted cu_seqlens: rejected with an error code
     if (n > 0) {
       std::vector<int64_t> bad = cq;

@@ -85,7 +85,7 @@ def test_c3_subset_split_forward(device):
           f"Lq in [{min(q_lens)},{max(q_lens)}]", flush=True)
     assert max(k_lens) >= 30000 and 1 in q_lens and 16 in q_lens
     # the config's 4-16 key chunks per (sequence, head)
-    plan = _lib.plan_varlen(_cu_np(q_lens), _cu_np(k_lens), case.H, case.D)
+    plan = _lib.plan_varlen(_cu_np(q_lens), _cu_np(k_lens), case.H, case.D, balanced=True)
     fwd = plan.section("fwd")
     assert len(fwd) and np.all(fwd[:, 4] >= 0), "every C3 tile runs split"
     assert fwd[:, 7].min() >= 4 and fwd[:, 7].max() <= 16
@@ -108,7 +108,8 @@ def test_c3_full_size_split_forward(device):
     lq, lk = np.asarray(case.q_lens), np.asarray(case.k_lens)
     print(f"[C3 full] H={case.H} D={case.D} n={len(lq)} sum_Lq={int(lq.sum())} "
           f"sum_Lk={int(lk.sum())} max_Lk={int(lk.max())}", flush=True)
-    plan = _lib.plan_varlen(_cu_np(case.q_lens), _cu_np(case.k_lens), case.H, case.D)
+    plan = _lib.plan_varlen(_cu_np(case.q_lens), _cu_np(case.k_lens), case.H, case.D,
+                            balanced=True)
     fwd = plan.section("fwd")
     assert np.all(fwd[:, 4] >= 0) and fwd[:, 7].min() >= 4 and fwd[:, 7].max() <= 16
     q, k, v = W.varlen_tensors(case, device)

@@ -176,23 +176,40 @@ WIDE_CASES = [
 ]
 
 
+@pytest.fixture
+def run_plans(monkeypatch):
+    """The plans a test's calls run, in a cache of their own; with ``rules[0]``
+    "fixed" the fixed-rule ones, whose tiles are those of large launches."""
+    from collections import OrderedDict
+    from varlenabsorbflashattn_amd import _lib
+    plan_varlen, used, rules = _lib.plan_varlen, [], ["balanced"]
+
+    def plan(*a, balanced=False):
+        used.append(plan_varlen(*a, balanced=balanced and rules[0] == "balanced"))
+        return used[-1]
+
+    monkeypatch.setattr(_lib, "plan_varlen", plan)
+    monkeypatch.setattr(_lib, "_CACHE", OrderedDict())
+    return rules, used
+
+
 @pytest.mark.parametrize("dist", [1.0, 8.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("case", range(len(WIDE_CASES)))
-def test_varlen_wide_tiles(device, case, D, dtype, dist):
+def test_varlen_wide_tiles(device, run_plans, case, D, dtype, dist):
     """256-row query tiles (8-wave forward and dQ workgroups) at D = 64 / 128,
     bf16 and fp16: split-K items, one-key and tail-only items, partial waves.
     At dist = 8 (scores scaled 64x, fa-tools/benchmark_packed_varlen_flash_attn.py:226-233)
     later key tiles raise the running max far above the first tile's, so the
     lazy rescale runs on most tiles."""
-    from varlenabsorbflashattn_amd import _lib
+    rules, used = run_plans
+    rules[0] = "fixed"
     q_lens, k_lens = WIDE_CASES[case]
-    plan = _lib.plan_varlen(cu_from_lens(q_lens).numpy(), cu_from_lens(k_lens).numpy(), 4, D)
-    assert plan.info.q_tile == 256
     print(f"[varlen wide] q={q_lens} k={k_lens} D={D} {dtype} dist={dist}", flush=True)
     got, ref, emul = run_case(q_lens, k_lens, 4, D, dtype, device, dist_scale=dist,
                               reference_numerics=True)
+    assert used and used[0].info.q_tile == 256
     rel = dist > 1.0  # near one-hot rows: see test_varlen_input_scales
     assert_close("o", got[0], ref[0], rel=rel)
     for name, a, r, m in zip(("dq", "dk", "dv"), got[1:], ref[1:], emul):
@@ -203,28 +220,21 @@ def test_varlen_wide_tiles(device, case, D, dtype, dist):
 
 
 # Small launches run the balanced plan (128-row and 128-key tiles, finer key
-# chunks); these run the fixed-rule plan of the same cases, whose tiles are the
-# ones large launches take (256 rows, at D = 128 256 keys), and a balanced plan
-# of many splits.
+# chunks); these run both plans of the same cases, the fixed-rule one with the tiles
+# of large launches (256 rows, at D = 128 256 keys), and a balanced plan of many
+# splits.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32],
                          ids=["bf16", "f16", "f32"])
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("case", range(len(WIDE_CASES)))
-def test_varlen_fixed_rule_plan(device, monkeypatch, case, D, dtype):
-    from collections import OrderedDict
-    from varlenabsorbflashattn_amd import _lib
-    plan_varlen, used = _lib.plan_varlen, []
-
-    def fixed(*a, balanced=False):
-        used.append(plan_varlen(*a))
-        return used[-1]
-
-    monkeypatch.setattr(_lib, "plan_varlen", fixed)
-    monkeypatch.setattr(_lib, "_CACHE", OrderedDict())
+@pytest.mark.parametrize("rule,tile", [("fixed", 256), ("balanced", 128)])
+def test_varlen_both_plans(device, run_plans, rule, tile, case, D, dtype):
+    rules, used = run_plans
+    rules[0] = rule
     q_lens, k_lens = WIDE_CASES[case]
-    print(f"[varlen fixed-rule plan] q={q_lens} k={k_lens} D={D} {dtype}", flush=True)
+    print(f"[varlen {rule} plan] q={q_lens} k={k_lens} D={D} {dtype}", flush=True)
     got, ref = run_case(q_lens, k_lens, 4, D, dtype, device)
-    assert used and used[0].info.q_tile == 256
+    assert used and used[0].info.q_tile == tile
     for name, a, r in zip(("o", "dq", "dk", "dv"), got, ref):
         assert_close(name, a, r)
 
@@ -249,16 +259,19 @@ def test_varlen_balanced_splits(device, q_lens, k_lens, D):
     (5, [3, 16, 1, 9], [3000, 1500, 1024, 40], 128),  # decode-shaped: an item's heads on one XCD
     (7, [130, 20], [5000, 9000], 32),             # split-K items and their combine
 ])
-def test_varlen_odd_head_counts(device, H, q_lens, k_lens, D):
+def test_varlen_odd_head_counts(device, run_plans, H, q_lens, k_lens, D):
     """Head counts that are not multiples of the 8 XCDs, on both forward grid
-    layouts (the plan's xcd_heads flag), forward and backward."""
-    from varlenabsorbflashattn_amd import _lib
-    plan = _lib.plan_varlen(cu_from_lens(q_lens).numpy(), cu_from_lens(k_lens).numpy(), H, D)
-    print(f"[varlen odd H] H={H} q={q_lens} k={k_lens} D={D} xcd_heads={plan.info.xcd_heads}",
-          flush=True)
-    got, ref = run_case(q_lens, k_lens, H, D, torch.bfloat16, device)
-    for name, a, r in zip(("o", "dq", "dk", "dv"), got, ref):
-        assert_close(name, a, r)
+    layouts (the plan's xcd_heads flag) and both plans, forward and backward."""
+    rules, used = run_plans
+    for rules[0] in ("balanced", "fixed"):
+        from varlenabsorbflashattn_amd import _lib
+        _lib._CACHE.clear()
+        print(f"[varlen odd H] H={H} q={q_lens} k={k_lens} D={D} {rules[0]}", flush=True)
+        got, ref = run_case(q_lens, k_lens, H, D, torch.bfloat16, device)
+        print(f"  xcd_heads={used[-1].info.xcd_heads} q_tile={used[-1].info.q_tile}", flush=True)
+        for name, a, r in zip(("o", "dq", "dk", "dv"), got, ref):
+            assert_close(name, a, r)
+    assert len(used) == 2
 
 
 def test_single_key_returns_v(device):
