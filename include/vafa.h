@@ -98,7 +98,8 @@ typedef struct vafa_plan_info {
   int64_t off_fwd, n_fwd;         /* forward / dq items (query tiles)      */
   int64_t off_comb, n_comb;       /* combine items                         */
   int64_t off_kv, n_kv;           /* key-tile items (dK/dV, absorb dX)     */
-  int64_t off_qt, n_qt;           /* unsplit query tiles (absorb dU pass)  */
+  int64_t off_qt, n_qt;           /* absorb: unsplit query tiles (dU on the
+                                     wave-per-row kernels)                  */
   int64_t n_part_rows;            /* partial rows written by split items   */
   int64_t plan_ints;              /* total plan length in int32            */
   int64_t q_tile, k_tile;         /* tile sizes the plan was built for:
@@ -113,13 +114,17 @@ typedef struct vafa_plan_info {
   /* varlen backward: the dQ pass runs over the forward items of the
    * segments that are not fused (dq, dqc: filtered copies of fwd, comb);
    * fused segments (at most 16 queries, D <= 64) run dQ/dK/dV in one
-   * K-major pass over fkv items whose fp32 dQ partials fcomb sums. */
-  int64_t off_dq, n_dq;           /* dQ-pass items                          */
-  int64_t off_dqc, n_dqc;         /* dQ-pass combine items                  */
+   * K-major pass over fkv items whose fp32 dQ partials fcomb sums.
+   * Absorb backward (H <= 64): dq and dqc are the dU pass's own items, key
+   * ranges split, and the sums of its fp32 dU / aX partials (n_fpart_rows);
+   * the first n_fkv of them (off_fkv == off_dq) belong to segments of at most
+   * 64 (token, head) rows, which one kernel can take with their dX. */
+  int64_t off_dq, n_dq;           /* dQ (absorb dU) pass items              */
+  int64_t off_dqc, n_dqc;         /* its combine items                      */
   int64_t max_dqc_rows;
-  int64_t off_fkv, n_fkv;         /* fused key-chunk items                  */
-  int64_t off_fcomb, n_fcomb;     /* fused dQ-partial sums                  */
-  int64_t n_fpart_rows;           /* fused dQ partial rows                  */
+  int64_t off_fkv, n_fkv;         /* fused key-chunk (absorb: one-pass) items */
+  int64_t off_fcomb, n_fcomb;     /* fused dQ-partial sums (varlen)         */
+  int64_t n_fpart_rows;           /* fused dQ (absorb dU / aX) partial rows */
   int64_t max_fcomb_rows;
   /* varlen forward grid: 1 = the H heads of a forward item run on one XCD
    * (most of the work lies in segments of at most 128 queries, whose items

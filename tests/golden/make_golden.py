@@ -1,5 +1,5 @@
 """Writes config1_oracle_summary.json: a regression pin of the CPU oracle on
-configs[0] (packed varlen self-attention, fp32, lens {17,64,128,200}, H=4,
+C1 (packed varlen self-attention, fp32, lens {17,64,128,200}, H=4,
 D=64, scale 1/8, q/k/v/dO ~ N(0,1) from numpy default_rng(2024)).
 
 The summary holds, per output (o, lse, dq, dk, dv, computed in float64),

@@ -1,6 +1,6 @@
 """Shared error metrics for the GPU parity tests.
 
-Tolerance (north-star spec): max-abs <= 2e-2 and mean-abs <= 2e-3 for 16-bit
+Tolerance: max-abs <= 2e-2 and mean-abs <= 2e-3 for 16-bit
 outputs and gradients against an fp32 (here float64) reference, 1e-4 / 1e-5
 for fp32 I/O.  Both are ABSOLUTE bounds on the raw difference:
   * max |ref| <= RAW_LIMIT (= 2): the raw max-abs and the raw mean-abs are
@@ -101,7 +101,7 @@ def assert_within_reference_numerics(name: str, out: torch.Tensor, exact: np.nda
     algorithm meets the raw bound there.  ``emulated`` is the oracle with
     exactly those roundings (oracle.varlen.backward(round_ps=...)); ``out``
     must stay within ``slack`` times the emulation's own error against the
-    exact gradient, plus the north-star bound relative to max(1, rms(ref)),
+    exact gradient, plus the stated bound relative to max(1, rms(ref)),
     for the max and for the mean."""
     tol_max, tol_mean = TOL[out.dtype]
     e = errors(out, exact)

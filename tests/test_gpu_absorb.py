@@ -154,8 +154,8 @@ def test_absorb_wide_dh_split(device, H, D_H, d_kv, dtype):
         assert_close(n, a, r)
 
 
-# The dU pass over key chunks of at least 256 keys (fp32 partials summed in
-# order): ranges at the chunk's edges, tiles of one token and of several per
+# The dU pass over key chunks, of ranges above 256 keys (fp32 partials summed in
+# order): ranges at that line's and the chunks' edges, tiles of one token and of several per
 # sample, whole and split tiles in one launch, D_KV = 512 (two workgroups per
 # tile), a padded D_KV.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32],

@@ -1,14 +1,14 @@
-"""GPU parity on the benchmark workloads themselves.
+"""GPU parity on the benchmark workloads themselves (C2 to C5).
 
 Every configuration that bench.py times is checked here on its own shape and
-plan, against the numpy oracle in float32 on the host (the north-star
+plan, against the numpy oracle in float32 on the host (the stated
 reference precision) with the tolerances of tests/parity.py:
-  * configs[1] (C2): the whole 64-sequence H=16 D=128 batch, O and all grads;
-  * configs[2] (C3): the full 256-sequence launch that bench.py times (its
+  * C2: the whole 64-sequence H=16 D=128 batch, O and all grads;
+  * C3: the full 256-sequence launch that bench.py times (its
     own plan, 4-16 key chunks per (sequence, head)), every head compared in
     groups of four; plus a seeded 24-sequence subset with its plan asserted;
-  * configs[3] (C4): all 2048 samples, inner forward and backward;
-  * configs[4] (C5): the full 8192-sample forward (its own plan), every
+  * C4: all 2048 samples, inner forward and backward;
+  * C5: the full 8192-sample forward (its own plan), every
     sample's output rows compared against the oracle in batches.
 Inputs follow varlenabsorbflashattn_amd.workloads (the generator bench.py uses).
 Bounds: tests/parity.py (raw max-abs <= 2e-2 on tensors with max |ref| <= 2,
@@ -167,7 +167,7 @@ def test_c4_full_fwd_bwd(device, dtype):
 
 
 def test_c4_whole_op_folded(device):
-    """configs[3] through packed_target_attn as bench.py times it: 16-bit
+    """C4 through packed_target_attn as bench.py times it: 16-bit
     inputs take the folded projection (u formed inside the attention kernel),
     forward and the five gradients against the fp32 oracle."""
     from varlenabsorbflashattn_amd import packed_target_attn

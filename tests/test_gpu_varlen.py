@@ -137,7 +137,7 @@ def test_varlen_fp32_matrix_cores(device, name, q_lens, k_lens, D):
 
 
 def test_varlen_config1_fp32(device):
-    """configs[0]: fp32, lens {17,64,128,200}, H=4, D=64 (N(0,1) inputs)."""
+    """C1: fp32, lens {17,64,128,200}, H=4, D=64 (N(0,1) inputs)."""
     got, ref = run_case([17, 64, 128, 200], [17, 64, 128, 200], 4, 64, torch.float32, device,
                         seed=1)
     assert_close("o", got[0], ref[0])

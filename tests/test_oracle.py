@@ -346,7 +346,7 @@ def test_absorb_inner_lse_and_uniform_case():
     np.testing.assert_allclose(lse[2:], math.log2(6), atol=1e-12)
 
 
-# ---- committed golden summary of configs[0] --------------------------------------
+# ---- committed golden summary of C1 --------------------------------------
 
 def test_config1_golden_summary():
     path = os.path.join(ROOT, "tests", "golden", "config1_oracle_summary.json")

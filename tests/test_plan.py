@@ -409,9 +409,9 @@ def test_host_cu_pair_matches_single_copies():
 
 def test_absorb_split_chunk_follows_total_work():
     """Key ranges split only beyond a chunk that grows with the launch's total
-    work: thousands of samples of <= 8192 keys (configs[3] / configs[4]
-    shapes) stay whole, while a handful of very long samples are split into
-    chunks of at least 1024 keys so that they fill the GPU."""
+    work: thousands of samples of <= 8192 keys (C4 and C5) stay whole,
+    while a handful of very long samples are split into chunks of at least 1024
+    keys so that they fill the GPU."""
     from varlenabsorbflashattn_amd import workloads as W
 
     def split_counts(ql, kl):

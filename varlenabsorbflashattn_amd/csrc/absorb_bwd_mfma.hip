@@ -598,8 +598,9 @@ __global__ __launch_bounds__(64 * kDxWaves, FP > kMaxF ? 1 : 2) void absorb_dx_k
 // Between two barriers a wave runs A of tile j+1, then B and C of tile j, so one
 // barrier per tile suffices.  Per 32-key tile and 64 rows 1536 cycles of
 // products per SIMD and 270 KB of LDS reads.  C4 (2048 samples, 648k keys, 853
-// MB): 273 us in the two kernels, 202 here (4.2 TB/s); 1127 samples of <= 2048
-// keys, D_KV 216 (those of at most 64 rows): 326 -> 245.  Measured on the way: dX
+// MB): 273 us in the two kernels, 201 here (861 MB by the counters, 4.3 TB/s;
+// matrix cores 17% busy, a third of the LDS cycles bank conflicts); 1127 samples of
+// <= 2048 keys, D_KV 216 (those of at most 64 rows): 326 -> 234.  Measured on the way: dX
 // stored as 2-byte elements (16 stores a wave and tile instead of 2) 280 -> 226;
 // waves of one SIMD in opposite phase order (twice the code, 10 spills) 226
 // against 202; B and C before A 207.

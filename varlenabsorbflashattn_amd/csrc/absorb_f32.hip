@@ -2,13 +2,16 @@
 // (v_mfma_f32_16x16x4_f32): the reference's documented call, which computes
 // with fp32 inputs and IEEE fp32 dots (ta/interface.py:371, 389-391;
 // ta/kernels.py:258-270).  Same work decomposition as the 16-bit kernels:
-//   * forward (ta/kernels.py:185-284) and du/aX (ta/kernels.py:354-498): a
-//     workgroup of 4 waves x 16 rows owns the H heads of floor(64/H) tokens
-//     of one sample (head-major; with H not dividing 64 the last rows idle)
-//     and streams the sample's X rows once through a 3-deep ring of 16-key
-//     LDS tiles filled by buffer_load ... lds;
-//   * dX (ta/kernels.py:528-900): a workgroup owns up to 256 keys of one
-//     sample, 16 per wave per pass, and streams the sample's (token, head)
+//   * forward (ta/kernels.py:185-284): a workgroup of 4 waves x 16 rows owns
+//     the H heads of floor(64/H) tokens of one sample (head-major; with H not
+//     dividing 64 the last rows idle) and streams the sample's X rows, or one
+//     chunk of them, once through a 3-deep ring of 16-key LDS tiles filled by
+//     buffer_load ... lds;
+//   * du/aX (ta/kernels.py:354-498): the same tokens' rows lie compactly,
+//     token by token, X comes through four such tiles, two a barrier, and
+//     tiles of at most 32 rows share their key tiles between wave pairs;
+//   * dX (ta/kernels.py:528-900): a workgroup owns the plan's key tile (128
+//     to 512 keys of one sample), 16 per wave per pass, and streams the sample's (token, head)
 //     rows of u and dAX through LDS in blocks of 32, summing over heads in
 //     registers (deterministic).
 //
@@ -36,11 +39,11 @@ __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) {
 }
 
 constexpr int kKT = 16;    // keys per LDS tile (forward, du)
-constexpr int kNBuf = 3;   // LDS ring depth
+constexpr int kNBuf = 3;   // LDS ring depth (forward)
 constexpr int kRBlk = 32;  // (token, head) rows per LDS block (dX)
 
 // padded feature width: a multiple of 64 (the aX^T / du^T / dX^T tiling) up
-// to 256; 512 above (the forward only)
+// to 256; 512 above
 inline int fp64_of(int F) { return F > 256 ? 512 : (F + 63) / 64 * 64; }
 
 // LDS row stride (floats): 16 consecutive rows read at one column by the
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(256) void transpose_wv_f32_kernel(const float *__re
   wvt[i] = f < F ? wv[((int64_t)f * H + h) * DH + d] : 0.f;
 }
 
-// Row geometry of a 64-row workgroup (forward and du): row = wave*16 + l16
+// Row geometry of a 64-row workgroup (forward): row = wave*16 + l16
 // is token row % TT of head row / TT, TT = floor(64 / H) tokens (rows past
 // H * TT idle).  A wave's rows span heads h_first..h_last.
 struct Rows64 {
@@ -471,7 +474,7 @@ __global__ __launch_bounds__(256, 1) void absorb_du_f32_kernel(
 
 // ---------------------------------------------------------------------------
 // Backward, key side (ta/kernels.py:528-900): item {k0, k1, t0, t1, ...}
-// covers up to 256 keys of one sample and all of its (token, head) rows
+// covers a key tile of one sample and all of its (token, head) rows
 // R = t*H + h in [t0*H, t1*H):
 //   dX_j = sum_R (scale * dS_Rj u_R + P_Rj dAX_R),
 // summed over rows and heads in registers in a fixed order.  Each pass gives

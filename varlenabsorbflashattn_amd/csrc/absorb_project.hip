@@ -492,7 +492,9 @@ __global__ __launch_bounds__(256, FP > 256 ? 2 : 1) void wgrad_kernel(
 // 16-byte stores where every output row does.
 // 2397 tokens, D_Q = D_KV = 256 forward and backward: torch's GEMMs, block
 // diagonal and copies took 285 us of GPU time, these kernels and the weight
-// gradients 108.
+// gradients 108.  With many tokens of few heads it is bound by those L2 reads (30 to
+// 55 TFLOP/s) and the caller takes torch's GEMMs instead (_project_f32_pays in
+// absorb.py).
 template <bool KJ, bool VEC, bool SVEC>
 __global__ __launch_bounds__(256) void rowgemm_f32_kernel(
     const float *__restrict__ X, const float *__restrict__ W, float *__restrict__ Y, int64_t T_q,

@@ -90,7 +90,7 @@ void key_split(int64_t rows, int64_t lk, const SplitPolicy &p, int64_t *ns_out,
 // 256-key dK/dV tiles pay off at D=128 (two waves per SIMD either way) when
 // most of the work lies in segments with more than 128 keys; at D <= 64 the
 // 4-wave kernel holds more waves per SIMD and stays.  Measured on the MI355X:
-// configs[1] forward -2%, dK/dV -2.5%; configs[2] forward +10% with 256-row
+// C2 forward -2%, dK/dV -2.5%; C3 forward +10% with 256-row
 // tiles; stage-1 replay (D=64) forward -6.6%, dK/dV +1.7% with 256-key tiles.
 void varlen_tiles(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t D, int64_t *bm,
                   int64_t *bk, int64_t *xcd_heads) {
@@ -108,8 +108,8 @@ void varlen_tiles(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t 
   // queries (one query tile per key range), the H workgroups of an item run
   // on one XCD and read whole token rows of K/V together; otherwise the query
   // tiles of a segment run on one XCD and share its K/V in L2.  Measured on
-  // the MI355X: configs[2] 5.58-5.70 -> 6.01-6.09 TB/s with grouped heads,
-  // configs[1] forward 0.529 -> 0.548 ms (so it keeps the item-major grid).
+  // the MI355X: C3 5.58-5.70 -> 6.01-6.09 TB/s with grouped heads, C2 forward
+  // 0.529 -> 0.548 ms (so it keeps the item-major grid).
   *xcd_heads = work > 0.0 && 2.0 * long_q < work ? 1 : 0;
 }
 
@@ -499,16 +499,17 @@ int vafa_plan_varlen_balanced(const int64_t *cu_q, const int64_t *cu_k, int64_t 
 //   kv section  : {k0, k1, t0, t1, seg, 0, 0, 0} key tiles for dX with the
 //                 segment's whole token range [t0, t1).
 //   qt section  : {t0, t1, k0, k1, -1, seg, 0, 1} unsplit token tiles with the
-//                 segment's whole key range (backward dU pass).
-//   dq, dqc     : (H <= kAbsorbRows) the items the backward runs instead of
-//                 qt, {t0, t1, k0, k1, pbase, seg, split, nsplit}, key ranges
+//                 segment's whole key range (dU on the wave-per-row kernels).
+//   dq, dqc     : (H <= kAbsorbRows) the items of the matrix-core kernels'
+//                 dU pass, {t0, t1, k0, k1, pbase, seg, split, nsplit}, key ranges
 //                 split by a policy of their own with fp32 du / aX partials in
 //                 rows pbase + r (n_fpart_rows in all), and one item per split
 //                 tile, laid out as the comb items.  The first n_fkv items (off_fkv
 //                 = off_dq) belong to segments of at most kDxResidentRows rows,
-//                 whose dX the merged kernel forms too (t0 == t1: a segment
-//                 without queries, whose dX is cleared); the kv items beyond
-//                 n_kv_res belong to the others.
+//                 whose dX the merged kernel forms too (t0 == t1: a key range
+//                 of a segment without queries, whose dX is cleared) where
+//                 xcd_heads is 1; the kv items beyond n_kv_res belong to the
+//                 others.
 int vafa_plan_absorb(const int64_t *cu_q, const int64_t *cu_k, int64_t n1, int64_t H,
                      int64_t D_KV, int64_t D_H, int32_t *plan, int64_t plan_cap,
                      vafa_plan_info *info) {

@@ -14,7 +14,8 @@ constexpr int kVarlenWideTile = 256;
 // Absorb: a forward workgroup covers up to kAbsorbRows (token, head) rows;
 // a dX workgroup covers up to kAbsorbKTile keys of one sample (two 128-key
 // sub-tiles on the matrix-core path), kAbsorbSmallKTile in launches of at most
-// kAbsorbSmallKeys keys, whose dX grid would leave CUs idle.  GPU time of
+// kAbsorbSmallKeys keys, whose dX grid would leave CUs idle (D_KV > 256:
+// kAbsorbWideF below).  GPU time of
 // forward + backward, us, at 512 / 256 / 128 keys: C4 (648k keys) 543 / 543 /
 // 547, 1127 samples of <= 2048 keys (1.37M) 969 / 949 / 994, 256 and 64 C4
 // samples (80k, 20k) 162 / 155 / 157 and 131 / 121 / 115, 512 C4 samples in
@@ -41,8 +42,9 @@ constexpr SplitPolicy kVarlenPolicy{16, 1024, 2048, 4, 16, 4096, 4096, 64, 64};
 // share of the work.  Below 3/5 item per resident 128-row workgroup (two per
 // CU; 4/5 at D = 256, one per CU) key ranges split beyond 3/2 of the average
 // keys per workgroup, below two items each decode tiles into chunks of half of
-// it (up to twice the splits); never below min_chunk keys, and only while the
-// fp32 partial rows stay within max_part_bytes.  GPU time, us, fixed rules ->
+// it (up to twice the splits), chunks of at least min_chunk keys before a range is
+// divided evenly (513 keys end as 320 + 193), and only while the fp32 partial rows
+// stay within max_part_bytes.  GPU time, us, fixed rules ->
 // balanced (self-attention lengths log-uniform in [1, 4096] unless stated, H =
 // heads): 16 sequences D = 128 H = 4 forward + backward 262 -> 215, 8 sequences
 // H = 16 227 -> 206, 16 sequences D = 256 H = 2 402 -> 341, fp32 D = 64 32
@@ -74,8 +76,9 @@ constexpr int64_t kAbsorbSlots = 768;
 constexpr int64_t kAbsorbSlack2 = 5;
 // Absorb backward, dU pass: two resident workgroups per CU; a chunk holds
 // kAbsorbDuSlack times the average keys per workgroup.  A split tile writes
-// and re-reads 8 bytes of fp32 partials per (row, feature), so chunks stay at
-// 256 keys and up.  GPU time of forward + backward, us, whole ranges -> split:
+// and re-reads 8 bytes of fp32 partials per (row, feature), so only ranges above
+// 256 keys split (evenly: 257 keys into 192 + 65).  GPU time of forward + backward,
+// us, whole ranges -> split:
 // 64 / 256 / 700 C4 samples 158 / 201 / 257 -> 131 / 162 / 234, 512 and 64 C4
 // samples in fp32 1318 -> 985 and 872 -> 548; all of C4 unchanged (544, whole
 // at this slack; 553 at half of it).

@@ -87,7 +87,7 @@ def config2(seed: int = 0, n_seq: int = 64) -> VarlenCase:
 
 
 def config2_tokens(seed: int = 0, total: int = 128 * 1024) -> VarlenCase:
-    """configs[1] read by its token count ("about 128k total tokens"): the same
+    """C2 read by its token count ("about 128k total tokens"): the same
     seeded log-uniform draw as config2 (whose 64 sequences are its prefix),
     extended until the packed length reaches ``total`` tokens."""
     rng = np.random.default_rng(seed)
