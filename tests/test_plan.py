@@ -636,9 +636,9 @@ def test_absorb_clear_items(q_lens, k_lens):
 @pytest.mark.parametrize("d_kv", [128, 216, 256])
 def test_absorb_merged_rule(d_kv):
     """The one-pass backward kernel is chosen by the keys of its own segments: for
-    all of a launch, and beside segments of more than 64 rows from 88M X elements
+    all of a launch, and beside segments of more than 64 rows from 75M X elements
     on, however many keys those, or segments without queries, hold."""
-    line = -(-(88 << 20) // d_kv)
+    line = -(-(72 << 20) // d_kv)
     for q_lens, k_lens, merge in [([8, 3], [50, 7], 1), ([8, 0], [50, 10**6], 1),
                                   ([9, 3], [10**6, 7], 0), ([9, 3, 0], [50, 7, 10**6], 0),
                                   ([9, 8], [5, line - 1], 0), ([9, 8], [5, line], 1),

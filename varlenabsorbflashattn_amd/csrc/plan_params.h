@@ -147,9 +147,10 @@ constexpr int kDxResidentRows = 64;
 // has to be worth a kernel's tail, however long the other segments are.  Forward +
 // backward, us, not merged / merged at M elements (samples of <= 2048 keys, 8 heads):
 // D_KV 256  M = 40M 480 / 508, 58M 598 / 622, 82M 556 / 558, 96M 383 / 381, 106M
-// 362 / 343, 119M 1077 / 1045, 191M 956 / 888; D_KV 192  62M 424 / 434, 72M 301 /
+// 362 / 343, 119M 1077 / 1045, 191M 956 / 888, 16 heads 45M 457 / 491, 80M 759 / 734,
+// 32 heads 85M 2224 / 2194; D_KV 192  62M 424 / 434, 72M 301 /
 // 315, 89M 385 / 366, 103M 368 / 358; D_KV 128  29M 365 / 403, 60M 287 / 301, 74M
 // 270 / 289, 67M (of 307M) 1235 / 1219, 96M 555 / 538, 129M 497 / 476.
-constexpr int64_t kAbsorbMergedElems = int64_t{88} << 20;
+constexpr int64_t kAbsorbMergedElems = int64_t{72} << 20;
 
 }  // namespace vafa
